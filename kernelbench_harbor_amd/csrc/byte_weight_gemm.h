@@ -14,12 +14,16 @@
 //    steps of 32 k for MB blocks of 16 rows (each dequantised weight fragment feeds MB MFMAs, so
 //    the weights are streamed once per 16 MB rows); all loads up front; 16x16x32 fp16/bf16
 //    MFMAs; split-K epilogue of splitk.h, once per row block.
-//  * larger M: tiled_f16_gemm (tiled_f16.h) with ByteSlabPolicy.
+//  * larger M: the warp-specialised wide tiles (tiled_ws.h, tiled_ws256.h) with ByteWidePolicy, or
+//    tiled_f16_gemm (tiled_f16.h) with ByteSlabPolicy for shapes they do not cover.
 #pragma once
 
 #include "kbh_common.h"
 #include "splitk.h"
 #include "tiled_f16.h"
+#include "tiled_ws.h"
+#include "tiled_ws256.h"
+#include "w4_dequant.h"
 
 namespace kbh {
 namespace {
@@ -196,7 +200,123 @@ struct ByteSlabPolicy {
   }
 };
 
+// Rows (k, k+1) of column J of a 4-column dword pair (a: row k, b: row k+1), times scale bits s:
+// one dword of two dtype values, each rounded once (the arithmetic of byte4_dequant).
+template <bool BF16, int DEC, int J>
+__device__ inline uint32_t byte_pair_dequant(uint32_t a, uint32_t b, uint16_t s) {
+  if constexpr (DEC == kDecInt8) {
+    if constexpr (BF16) {
+      const float sf = bf16_bits_to_f32(s);
+      const float qa = (float)(int8_t)((a >> (8 * J)) & 0xffu), qb = (float)(int8_t)((b >> (8 * J)) & 0xffu);
+      return f32x2_to_bf16x2_bits(qa * sf, qb * sf);
+    } else {
+      // byte ^ 0x6480 is the fp16 1024 + (q + 128); minus 1152 gives q exactly
+      const _Float16 sh = __builtin_bit_cast(_Float16, s);
+      const _Float16 bias = (_Float16)1152.0f;
+      const h2_t q = __builtin_bit_cast(h2_t, pair_bytes<J>(a, b) ^ 0x64806480u) - h2_t{bias, bias};
+      return __builtin_bit_cast(uint32_t, q * h2_t{sh, sh});
+    }
+  } else {
+    // columns 0, 1 (or 2, 3) of both rows as two 16-bit halves (k, k+1)
+    const uint32_t P = __builtin_amdgcn_perm(b, a, J < 2 ? 0x05010400u : 0x07030602u);
+    if constexpr (BF16) {
+      const float sf = f16_bits_to_f32(s);
+      const f2_t v = __builtin_amdgcn_cvt_pk_f32_fp8(P, (J & 1) != 0);
+      return f32x2_to_bf16x2_bits(v[0] * sf, v[1] * sf);
+    } else {
+      const _Float16 sh = __builtin_bit_cast(_Float16, s);
+      return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(P, 1.0f, (J & 1) != 0) * h2_t{sh, sh});
+    }
+  }
+}
+
+// Weight producer of the warp-specialised kernels (32 rows x 256 columns per slab). Thread t owns
+// rows 4rb .. 4rb+3 of columns 8cb .. 8cb+7 (the F16WidePolicy / W8WidePolicy thread map, whose
+// LDS writes are bank-conflict free): four 8-byte loads, and per column its 4 consecutive K values
+// as one 8-byte piece of the K-contiguous operand layout (wide_b_offset). The two-row pairs come
+// straight from v_perm_b32 on two rows (no 4x4 byte transpose): the e4m3 conversions take either
+// 16-bit half of a dword.
+template <bool BF16, int DEC>
+struct ByteWidePolicy {
+  static constexpr int kTN = 256;
+  static constexpr bool kHasFast = false;
+  const uint8_t* w;
+  const uint16_t* scales;
+  int N, block;
+  struct Raw {
+    kbh_u32x2 r[4];
+  };
+  struct RawHalf {
+    kbh_u32x2 r[2];
+  };
+  struct Grp {
+    kbh_u32x4 s;
+  };
+  struct ScanPre {};
+  __device__ ByteWidePolicy at_expert(int) const { return *this; }
+  __device__ static int cb_of(int t) { return (t & 7) | (((t >> 4) & 3) << 3); }
+  __device__ static int rb_of(int t) { return ((t >> 3) & 1) | ((t >> 6) << 1); }
+  __device__ void load(Raw& r, int k0, int n0, int t) const {
+    const uint8_t* p = w + (size_t)(k0 + 4 * rb_of(t)) * N + n0 + 8 * cb_of(t);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)  // cached: the row blocks of a K range share them in L2
+      r.r[i] = *reinterpret_cast<const kbh_u32x2*>(p + (size_t)i * N);
+  }
+  // Two producer sets: set `half` takes rows 4rb + 2 half, +1.
+  __device__ void load_half(RawHalf& r, int k0, int n0, int t, int half) const {
+    const uint8_t* p = w + (size_t)(k0 + 4 * rb_of(t) + 2 * half) * N + n0 + 8 * cb_of(t);
+    r.r[0] = *reinterpret_cast<const kbh_u32x2*>(p);
+    r.r[1] = *reinterpret_cast<const kbh_u32x2*>(p + N);
+  }
+  __device__ void load_group(Grp& g, int k0, int n0, int t) const {
+    g.s = *reinterpret_cast<const kbh_u32x4*>(scales + (size_t)(k0 / block) * N + n0 + 8 * cb_of(t));
+  }
+  template <bool FAST>
+  __device__ void prepare_group(Grp&) const {}
+  // Values of column c of rows (2i, 2i+1) for NI row pairs, all columns.
+  template <int NI, class R>
+  __device__ void dequant(const R& r, const Grp& g, uint32_t (&v)[8][NI]) const {
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t a = r.r[2 * i][h], b = r.r[2 * i + 1][h];
+        v[4 * h + 0][i] = byte_pair_dequant<BF16, DEC, 0>(a, b, half_of(g.s, 4 * h + 0));
+        v[4 * h + 1][i] = byte_pair_dequant<BF16, DEC, 1>(a, b, half_of(g.s, 4 * h + 1));
+        v[4 * h + 2][i] = byte_pair_dequant<BF16, DEC, 2>(a, b, half_of(g.s, 4 * h + 2));
+        v[4 * h + 3][i] = byte_pair_dequant<BF16, DEC, 3>(a, b, half_of(g.s, 4 * h + 3));
+      }
+  }
+  // wide_b_offset<256>(8 rb, 8 cb + c) = base + 16 (c ^ fw)
+  __device__ static uint8_t* base_of(uint8_t* Bs, int cb, int rb) {
+    return Bs + wide_b_offset<256>(8 * rb, 8 * cb) - wide_slot(8 * cb) * 16 + cb * 128;
+  }
+  template <bool FAST>
+  __device__ void store_all(const Raw& r, const Grp& g, uint8_t* Bs, int t) const {
+    const int cb = cb_of(t), rb = rb_of(t);
+    uint8_t* base = base_of(Bs, cb, rb);
+    const int fw = (cb ^ (cb >> 3)) & 7;
+    uint32_t v[8][2];
+    dequant<2>(r, g, v);
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      *reinterpret_cast<kbh_u32x2*>(base + ((c ^ fw) << 4)) = kbh_u32x2{v[c][0], v[c][1]};
+  }
+  template <bool FAST>
+  __device__ void store_half(const RawHalf& r, const Grp& g, uint8_t* Bs, int t, int half) const {
+    const int cb = cb_of(t), rb = rb_of(t);
+    uint8_t* base = base_of(Bs, cb, rb) + 4 * half;
+    const int fw = (cb ^ (cb >> 3)) & 7;
+    uint32_t v[8][1];
+    dequant<1>(r, g, v);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) *reinterpret_cast<uint32_t*>(base + ((c ^ fw) << 4)) = v[c][0];
+  }
+};
+
 constexpr int kByteTiledMinM = 128;
+constexpr int kByteWideMinM = 33;
+constexpr int kByteWidePD = 4;
 
 struct BytePlan {
   int spw, waves, ntiles, mb, mblocks, splits;
@@ -218,6 +338,53 @@ bool plan_byte_decode(int M, int N, int K, BytePlan* p) {
   return p->waves > 0;
 }
 
+struct ByteWide {
+  WidePlan plan;
+  int spg;
+};
+
+// Wide tiles from kByteWideMinM rows: the W4A16 geometry (64-row tiles up to 64 rows, 128-row
+// ones up to 256, 256-row ones above unless the estimate prefers 128 rows). They replace
+// tiled_f16_gemm's 256 x 128 tiles, which split no K (K=14336 N=4096: 32 workgroups and ~300 us
+// at every M from 128 to 1024; now 30.7 / 43.0 / 75.2 / 124 us at M=128 / 256 / 512 / 1024, and
+// 342 -> 226 at 2048), and the decode kernel's 64-row blocks (M=48 42.9 -> 21.8, M=96 73.2 ->
+// 28.4). Up to 64 rows the decode kernel stays where its grid is one workgroup per CU: every
+// weight is then in flight at once and it needs fewer split-K slices (K=N=4096 M=64 14.6 against
+// 19.8 us, K=2048 N=8192 15.5 / 19.6; with a second round of workgroups the wide tiles win:
+// K=4096 N=6144 25.6 / 18.6, K=N=3584 16.9 / 15.9).
+bool plan_byte_wide(int M, int N, int K, int block, ByteWide* w) {
+  if (M < kByteWideMinM || N % 256 != 0) return false;
+  // the kernels stage x with 32-bit offsets
+  if ((size_t)(M + 256) * K * 2 >= ((size_t)1 << 31)) return false;
+  BytePlan d;
+  if (M <= 64 && plan_byte_decode(M, N, K, &d) && d.ntiles * d.splits * d.mblocks <= 256) return false;
+  w->spg = block / 32;
+  return plan_wide(M, N, K, 256, 32, wide_k_unroll(K, w->spg, kByteWidePD), 256, &w->plan,
+                   M <= 64 ? 64 : 128, true, 256);
+}
+
+template <bool BF16, int DEC, int SPG>
+void launch_byte_wide(const ByteWide& w, const void* x, const void* wt, const void* scales, void* y,
+                      float* slices, int M, int N, int K, int block, hipStream_t st) {
+  using E = WideHalf<BF16>;
+  using BP = ByteWidePolicy<BF16, DEC>;
+  using EP = HalfOut<BF16>;
+  const BP bp{(const uint8_t*)wt, (const uint16_t*)scales, N, block};
+  const EP ep{(uint16_t*)y, N};
+  const WidePlan& p = w.plan;
+  if (p.tm == 256)
+    hipLaunchKernelGGL((tiled_ws256_gemm<E, SPG, BP, EP, kByteWidePD>), dim3(p.grid), dim3(768), 0,
+                       st, x, bp, ep, slices, M, N, K, p.splits, p.slabs_per_split);
+  else if (p.tm == 128)
+    hipLaunchKernelGGL((tiled_ws_gemm<E, 128, 2, SPG, BP, EP, DenseRows, kByteWidePD, 1, true>),
+                       dim3(p.grid), dim3(512), 0, st, x, bp, ep, slices, M, N, K, p.splits,
+                       p.slabs_per_split, DenseRows{M});
+  else
+    hipLaunchKernelGGL((tiled_ws_gemm<E, 64, 2, SPG, BP, EP, DenseRows, kByteWidePD, 2>),
+                       dim3(p.grid), dim3(768), 0, st, x, bp, ep, slices, M, N, K, p.splits,
+                       p.slabs_per_split, DenseRows{M});
+}
+
 // Runs the GEMM; with `defer_sum` and a split K the slices are left in the workspace
 // (acc[splits][M][N] fp32) for the caller to sum, and *splits_out tells how many (1: y written).
 template <bool BF16, int DEC>
@@ -225,6 +392,28 @@ int byte_gemm_run(const void* x, const void* w, const void* scales, void* y, voi
                   size_t workspace_bytes, int M, int N, int K, int block, hipStream_t st,
                   bool defer_sum = false, int* splits_out = nullptr) {
   if (splits_out) *splits_out = 1;
+  ByteWide wide;
+  if (plan_byte_wide(M, N, K, block, &wide)) {
+    const int splits = wide.plan.splits;
+    const size_t need = wide_workspace_bytes(M, N, splits);
+    if (need > 0 && (!workspace || workspace_bytes < need)) return KBH_ERR_WORKSPACE;
+    if (need > 0 && !aligned16(workspace)) return KBH_ERR_ALIGN;
+    float* slices = (float*)workspace;
+    switch (wide.spg) {
+      case 1: launch_byte_wide<BF16, DEC, 1>(wide, x, w, scales, y, slices, M, N, K, block, st); break;
+      case 2: launch_byte_wide<BF16, DEC, 2>(wide, x, w, scales, y, slices, M, N, K, block, st); break;
+      case 4: launch_byte_wide<BF16, DEC, 4>(wide, x, w, scales, y, slices, M, N, K, block, st); break;
+      default: launch_byte_wide<BF16, DEC, 8>(wide, x, w, scales, y, slices, M, N, K, block, st); break;
+    }
+    if (splits_out) *splits_out = splits;
+    if (splits > 1 && !defer_sum) {
+      using EP = HalfOut<BF16>;
+      const size_t n4 = (size_t)M * N / 4;
+      hipLaunchKernelGGL((wide_reduce_kernel<WideHalf<BF16>, EP>), dim3((unsigned)((n4 + 255) / 256)),
+                         dim3(256), 0, st, slices, EP{(uint16_t*)y, N}, N, n4, splits);
+    }
+    return launch_status();
+  }
   if (M >= kByteTiledMinM && K % (TBK * TDEPTH) == 0) {
     const ByteSlabPolicy<BF16, DEC> bp{(const uint8_t*)w, (const uint16_t*)scales, N, block};
     hipLaunchKernelGGL((tiled_f16_gemm<BF16, ByteSlabPolicy<BF16, DEC>>), tiled_f16_grid(M, N),
@@ -256,10 +445,12 @@ int byte_gemm_run(const void* x, const void* w, const void* scales, void* y, voi
 }
 
 // Workspace bytes of byte_gemm_run for this shape (0 when K is not split).
-size_t byte_gemm_workspace_bytes(int M, int N, int K) {
-  BytePlan p;
-  if (M < 1 || N < 128 || K < 32) return 0;
+size_t byte_gemm_workspace_bytes(int M, int N, int K, int block) {
+  if (M < 1 || N < 128 || K < 32 || block < 32 || K % block != 0) return 0;
+  ByteWide w;
+  if (plan_byte_wide(M, N, K, block, &w)) return wide_workspace_bytes(M, N, w.plan.splits);
   if (M >= kByteTiledMinM && K % (TBK * TDEPTH) == 0) return 0;  // tiled path: no split
+  BytePlan p;
   if (!plan_byte_decode(M, N, K, &p)) return 0;
   return splitk_workspace_bytes(M, N, p.splits);
 }

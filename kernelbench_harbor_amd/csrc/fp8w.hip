@@ -11,10 +11,7 @@
 #include "byte_weight_gemm.h"
 
 extern "C" size_t kbh_fp8w_workspace_bytes(int M, int N, int K, int block) {
-  (void)block;
-  kbh::BytePlan p;
-  if (M < 1 || N < 128 || K < 32 || !kbh::plan_byte_decode(M, N, K, &p)) return 0;
-  return kbh::splitk_workspace_bytes(M, N, p.splits);
+  return kbh::byte_gemm_workspace_bytes(M, N, K, block);
 }
 
 extern "C" int kbh_fp8w_gemm(const void* x, const uint8_t* w_fp8, const void* scales, void* y,

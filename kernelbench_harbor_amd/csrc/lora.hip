@@ -156,20 +156,20 @@ __global__ __launch_bounds__(kLoraThreads) void lora_expand_add_kernel(
 }
 
 struct LoraLayout {
-  size_t part, total;
+  size_t slices, total;  // the shrink partials lie at offset 0
   int ds, dchunk;
 };
 
 // DS ranges of D for the shrink: enough workgroups (T x DS >= 1024, DS <= 16) while each keeps
 // at least four steps of 1024 / r rows (one round of four loads in flight per lane).
-LoraLayout lora_layout(int T, int D, int N, int r) {
+LoraLayout lora_layout(int T, int D, int N, int r, int group) {
   LoraLayout L;
   const int step = 1024 / r;
   const int ds_max = max(1, min(kLoraMaxSplits, D / (4 * step)));
   L.ds = max(1, min((1024 + T - 1) / T, ds_max));
   L.dchunk = (D + L.ds - 1) / L.ds;
-  L.part = round_up(byte_gemm_workspace_bytes(T, N, D), 256);
-  L.total = L.part + round_up((size_t)L.ds * T * r * 4, 256);
+  L.slices = round_up((size_t)L.ds * T * r * 4, 256);
+  L.total = L.slices + round_up(byte_gemm_workspace_bytes(T, N, D, group), 256);
   return L;
 }
 
@@ -177,17 +177,19 @@ template <bool BF16>
 int lora_run(const void* x, const int8_t* qweight, const void* scales, const void* A,
              const void* B, const int64_t* ids, void* y, void* ws, size_t ws_bytes, int T, int D,
              int N, int r, int L, int group, hipStream_t st) {
-  const LoraLayout lay = lora_layout(T, D, N, r);
-  float* part = (float*)((char*)ws + lay.part);
+  const LoraLayout lay = lora_layout(T, D, N, r, group);
+  if (ws_bytes < lay.total) return KBH_ERR_WORKSPACE;
+  float* part = (float*)ws;
+  float* slices = (float*)((char*)ws + lay.slices);
   int splits = 1;
-  const int s = byte_gemm_run<BF16, kDecInt8>(x, qweight, scales, y, ws, lay.part, T, N, D, group,
-                                              st, true, &splits);
+  const int s = byte_gemm_run<BF16, kDecInt8>(x, qweight, scales, y, slices, ws_bytes - lay.slices,
+                                              T, N, D, group, st, true, &splits);
   if (s != KBH_OK) return s;
   hipLaunchKernelGGL(lora_shrink_kernel<BF16>, dim3(T, lay.ds), dim3(kLoraThreads), 0, st,
                      (const uint16_t*)x, (const uint16_t*)A, ids, part, T, D, r, L, lay.dchunk);
   const dim3 grid((N / 4 + kLoraThreads - 1) / kLoraThreads, T);
   hipLaunchKernelGGL(lora_expand_add_kernel<BF16>, grid, dim3(kLoraThreads), 0, st,
-                     (const float*)part, (const uint16_t*)B, ids, (const float*)ws, splits,
+                     (const float*)part, (const uint16_t*)B, ids, (const float*)slices, splits,
                      (uint16_t*)y, T, N, r, L, lay.ds);
   return launch_status();
 }
@@ -197,7 +199,15 @@ int lora_run(const void* x, const int8_t* qweight, const void* scales, const voi
 
 extern "C" size_t kbh_lora_qgemm_workspace_bytes(int T, int D, int N, int r) {
   if (T < 1 || D < 32 || N < 128 || r < 1) return 0;
-  return kbh::lora_layout(T, D, N, r).total;
+  // The group size is not an argument here: room for the largest plan over the allowed groups
+  // (the split count of the base GEMM, hence its slices, depends on it).
+  size_t best = 0;
+  for (int group : {32, 64, 128, 256}) {
+    if (D % group != 0) continue;
+    const size_t b = kbh::lora_layout(T, D, N, r, group).total;
+    best = b > best ? b : best;
+  }
+  return best;
 }
 
 extern "C" int kbh_lora_qgemm(const void* x, const int8_t* qweight, const void* scales,
@@ -215,7 +225,6 @@ extern "C" int kbh_lora_qgemm(const void* x, const int8_t* qweight, const void* 
       !aligned16(workspace))
     return KBH_ERR_ALIGN;
   if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 7u) return KBH_ERR_ALIGN;
-  if (workspace_bytes < lora_layout(T, D, N, r).total) return KBH_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == KBH_BF16)
     return lora_run<true>(x, qweight, scales, A, B, lora_ids, y, workspace, workspace_bytes, T, D,

@@ -66,6 +66,11 @@ struct WideFlag {
   static constexpr bool value = B;
 };
 
+template <int I>
+struct WideIdx {
+  static constexpr int value = I;
+};
+
 // Element traits: MFMA and accumulator types of the two operand families.
 template <bool BF16>
 struct WideHalf {
@@ -537,6 +542,15 @@ inline bool plan_wide(int M, int N, int K, int tn, int slab_k, int unroll, int s
     if (plan_tm(tm_small, &q) < c256) *p = q;
   }
   return true;
+}
+
+// Slabs per K range must be a multiple of this for the warp-specialised kernels: their loop
+// iteration of U slabs (two quantization groups of spg slabs, a multiple of the 4-buffer ring and
+// of the prefetch ring), or U / 2 when K holds an odd number of half iterations (the loop then
+// leaves in the middle of its last iteration).
+inline int wide_k_unroll(int K, int spg, int pd) {
+  const int u = 2 * spg > pd ? 2 * spg : pd;
+  return K % (u * 32) == 0 ? u : u / 2;
 }
 
 // Workspace: `splits` slices of M x N 4-byte partial sums (none without split-K).

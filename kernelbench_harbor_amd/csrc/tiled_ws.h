@@ -14,7 +14,9 @@
 // producers write (s + 2) % 4. Each SIMD holds one wave of each role, so the dequantizing VALU
 // work of one runs beside the MFMAs of the other, where the 4-wave kernel issued both from the
 // same wave in turn. Both roles run their own loop of exactly KT barriers (plus the two of the
-// set-up), so the barrier counts match by construction, and then meet again for the epilogue:
+// set-up), so the barrier counts match by construction, and then meet again for the epilogue
+// (KT is a multiple of half an iteration of U slabs: both roles leave the last iteration in its
+// middle when K ends there):
 // split-K partial tiles go through the LDS ring, so that all 8 waves store whole rows.
 // 64-row tiles run two producer sets (waves 4..7 and 8..11, PS below), each dequantizing one
 // row pair of every thread's four rows.
@@ -171,9 +173,10 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
       __syncthreads();  // slabs 0 and 1 are in LDS
       // Slab kt + u + 2 during consumer slab kt + u. Slabs past the end re-produce the last one
       // into a buffer nobody reads, so the loop has no branch.
-      for (int kt = 0; kt < KT; kt += U) {
+      auto half = [&](auto h, int kt) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
+        for (int i = 0; i < U / 2; ++i) {
+          const int u = decltype(h)::value * (U / 2) + i;
           const int pu = u + 2;
           const int set = (pu / SPG) & 1;
           if (pu % SPG == 0) {  // slab kt + pu starts a group: its set is ready, reload the other
@@ -187,7 +190,13 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
           if constexpr (XD) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
           __syncthreads();
         }
+      };
+      int kt = 0;
+      for (; kt + U <= KT; kt += U) {
+        half(WideIdx<0>{}, kt);
+        half(WideIdx<1>{}, kt);
       }
+      if (kt < KT) half(WideIdx<0>{}, kt);  // K ends in half an iteration
     };
     if constexpr (kFast) {
       if (fast) produce(WideFlag<true>{});
@@ -259,9 +268,10 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
     kbh_u32x4 b0[CB], b1[CB];
     read_b(b0, 0, 0);
     constexpr int NMF = RB * CB;  // MFMAs per k16 step
-    for (int kt = 0; kt < KT; kt += U) {
+    auto half = [&](auto h, int kt) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int uu = 0; uu < U / 2; ++uu) {
+        const int u = decltype(h)::value * (U / 2) + uu;
         const int cur = u % NBUF, nxt = (u + 1) % NBUF, ra = u % PDA;
         read_a(A[ra], cur);
         read_b(b1, cur, 1);
@@ -287,7 +297,13 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
       }
+    };
+    int kt = 0;
+    for (; kt + U <= KT; kt += U) {
+      half(WideIdx<0>{}, kt);
+      half(WideIdx<1>{}, kt);
     }
+    if (kt < KT) half(WideIdx<0>{}, kt);  // as the producers
   }
 
   if constexpr (!EP::kPaired) {

@@ -122,9 +122,10 @@ __global__ __launch_bounds__(768, 1) void tiled_ws256_gemm(
       // at most one group load pair)
       asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
       __syncthreads();  // slabs 0 and 1 are in LDS
-      for (int kt = 0; kt < KT; kt += U) {
+      auto half = [&](auto h, int kt) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
+        for (int i = 0; i < U / 2; ++i) {
+          const int u = decltype(h)::value * (U / 2) + i;
           const int pu = u + 2;
           const int set = (pu / SPG) & 1;
           if (pu % SPG == 0) {
@@ -141,7 +142,13 @@ __global__ __launch_bounds__(768, 1) void tiled_ws256_gemm(
           asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
           __syncthreads();
         }
+      };
+      int kt = 0;
+      for (; kt + U <= KT; kt += U) {
+        half(WideIdx<0>{}, kt);
+        half(WideIdx<1>{}, kt);
       }
+      if (kt < KT) half(WideIdx<0>{}, kt);  // K ends in half an iteration
     };
     if constexpr (kFast) {
       if (fast) produce(WideFlag<true>{});
@@ -175,9 +182,10 @@ __global__ __launch_bounds__(768, 1) void tiled_ws256_gemm(
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
     __syncthreads();  // slabs 0 and 1 are in LDS
-    for (int kt = 0; kt < KT; kt += U) {
+    auto half = [&](auto h, int) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int uu = 0; uu < U / 2; ++uu) {
+        const int u = decltype(h)::value * (U / 2) + uu;
         const uint8_t* bb = bbuf(u % NBUF);
         const uint8_t* ab = abuf(u % NBUF);
 #pragma unroll
@@ -197,7 +205,13 @@ __global__ __launch_bounds__(768, 1) void tiled_ws256_gemm(
         }
         __syncthreads();
       }
+    };
+    int kt = 0;
+    for (; kt + U <= KT; kt += U) {
+      half(WideIdx<0>{}, kt);
+      half(WideIdx<1>{}, kt);
     }
+    if (kt < KT) half(WideIdx<0>{}, kt);  // as the producers
   }
 
   // The tile leaves through the ring, RP rows at a time: the MFMA waves write their

@@ -316,7 +316,12 @@ bool plan_w4_wide(int M, int N, int K, int group, W4Wide* w) {
   w->tn = (N % 256 == 0) ? 256 : 128;
   if (!small && w->tn != 256) return false;
   const int pd = w4_wide_pd(w->tn);
-  const int unroll = 2 * w->spg > pd ? 2 * w->spg : pd;  // the kernel's slabs per iteration
+  // The kernel's slabs per iteration; the warp-specialised kernels (256-column tiles, x under
+  // 2 GiB) also end in half an iteration: K = 29568 holds an odd number of 128-row groups (on the
+  // LDS-staged and decode kernels, which took it before, N=8192 M=64 / 256 / 1024 ran 164 / 784 /
+  // 771 us; now 62 / 161 / 518).
+  const bool ws = w->tn == 256 && (size_t)(M + 256) * K * 2 < ((size_t)1 << 31);
+  const int unroll = ws ? wide_k_unroll(K, w->spg, pd) : (2 * w->spg > pd ? 2 * w->spg : pd);
   // Up to 64 rows with 256-column tiles: 64 x 256 tiles (2 x 2 waves of 32 x 128); a 128-row
   // tile would spend half its MFMAs and A loads on padding. The split count is planned for one
   // workgroup per CU: more splits (two per CU) measured slower, their fp32 slices outweighing
