@@ -30,6 +30,7 @@
 #include "tiled_wide.h"
 #include "tiled_ws.h"
 #include "w4_dequant.h"
+#include "w4_stream.h"
 
 namespace kbh {
 namespace {
@@ -744,6 +745,54 @@ __global__ __launch_bounds__(256) void moe_reduce_combine_kernel(
   *reinterpret_cast<kbh_u32x2*>(y + e) = o;
 }
 
+// h[s][n] = dtype(silu(g) * u) with g and u the sums, in split order, of columns n and F + n of the
+// slices [splits][S][2F] (the streaming kernel's gate/up partial sums; fp32 math, one rounding).
+// Four columns per thread.
+template <bool BF16>
+__global__ __launch_bounds__(256) void moe_silu_sum_kernel(const float* __restrict__ part, int splits,
+                                                           uint16_t* __restrict__ h, int S, int F) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (size_t)S * F / 4) return;
+  const size_t s = 4 * i / (size_t)F, n = 4 * i - s * F;
+  const size_t slice4 = (size_t)S * 2 * F / 4;
+  const kbh_f32x4* p = reinterpret_cast<const kbh_f32x4*>(part + s * 2 * F + n);
+  const kbh_f32x4 g = sum_slices(p, slice4, splits), u = sum_slices(p + F / 4, slice4, splits);
+  uint16_t r[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r[q] = f32_to_half_bits<BF16>(keep_f32(silu_fast(g[q])) * u[q]);
+  kbh_u32x2 o;
+  o[0] = (uint32_t)r[0] | ((uint32_t)r[1] << 16);
+  o[1] = (uint32_t)r[2] | ((uint32_t)r[3] << 16);
+  *reinterpret_cast<kbh_u32x2*>(h + s * F + n) = o;
+}
+
+// FFN on the streaming kernel (w4_stream.h), below 32 routed rows per expert on average: 16-row
+// expert tiles whose weights are converted in registers without the per-weight arithmetic of the
+// wide tiles (those dequantize 128-row slabs through LDS for a few rows: ~3.4 VALU instructions
+// per weight, as long as the HBM time by itself). Mixtral layer, fp16: T=1 / 8 / 32 / 64 / 127
+// 322 / 439 / 450 / 444 / 514 -> 60 / 157 / 172 / 246 / 378 us (T=8 is 757 MB at 4.8 TB/s, the
+// rate of a large copy). Each 16-row tile past an expert's first costs its conversion again; the
+// line at 32 rows is where the 128-row tiles' measured cost is met within the range tested (1.36x
+// at 127 tokens). Both GEMMs split K until the tiles the batch can reach are about two workgroups
+// per CU, and leave fp32 slices.
+struct FfnStream {
+  int s1, s2;  // K splits of gate/up and of down
+};
+bool plan_ffn_stream(int T, int E, int D, int F, int group, FfnStream* p) {
+  if ((size_t)2 * T >= (size_t)32 * E) return false;
+  if (!w4_stream_ok(F, D, group) || !w4_stream_ok(D, F, group)) return false;
+  const int unit = group > kStreamChunk ? group : kStreamChunk;
+  const int reach = 2 * T < E ? 2 * T : E;  // experts the batch can reach
+  auto splits = [&](int col_tiles, int K) {
+    const int want = (512 + col_tiles * reach - 1) / (col_tiles * reach);
+    const int most = K / unit / kStreamWaves;  // at least one unit per wave
+    return want < 1 ? 1 : (want > most ? (most > 1 ? most : 1) : want);
+  };
+  p->s1 = splits(2 * F / kStreamCols, D);
+  p->s2 = splits(D / kStreamCols, F);
+  return true;
+}
+
 // FFN plan: TM x 256 expert tiles (TM = 256 rows when experts average at least 192 routed rows,
 // else 128: at ~128 rows per expert, 256-row tiles measured 20% slower despite fewer tiles), one
 // workgroup per CU with a 4-slab prefetch ring; gate/up unsplit (about
@@ -950,9 +999,57 @@ void launch_ffn_wide(const FfnPlan& fp, const MoeLayout& L, const MoeBuffers& mb
 #undef KBH_FFN
 }
 
+template <bool BF16>
+void launch_ffn_stream(const FfnStream& fs, const MoeLayout& L, const MoeBuffers& mb, const void* x,
+                       const W4Mat& gate, const W4Mat& up, const W4Mat& down, void* h, float* part,
+                       void* y, int T, int D, int F, int group, size_t gq, size_t gs, size_t dq,
+                       size_t ds, hipStream_t st) {
+  const int S = 2 * T;
+  W4StreamArgs a;
+  a.x = (const uint16_t*)x;
+  a.mat[0] = gate;
+  a.mat[1] = up;
+  a.slices = part;
+  a.tiles = mb.tiles;
+  a.perm = mb.perm;
+  a.q_stride = gq;
+  a.s_stride = gs;
+  a.M = S;
+  a.ld = 2 * F;
+  a.N = F;
+  a.K = D;
+  a.group = group;
+  a.splits = fs.s1;
+  a.tiles0 = F / kStreamCols;
+  a.gather = 1;
+  launch_w4_stream<BF16, true>(a, 2 * F / kStreamCols, L.max_tiles, st);
+  hipLaunchKernelGGL((moe_silu_sum_kernel<BF16>), dim3((unsigned)(((size_t)S * F / 4 + 255) / 256)),
+                     dim3(256), 0, st, (const float*)part, fs.s1, (uint16_t*)h, S, F);
+  a.x = (const uint16_t*)h;
+  a.mat[0] = a.mat[1] = down;
+  a.q_stride = dq;
+  a.s_stride = ds;
+  a.ld = a.N = D;
+  a.K = F;
+  a.splits = fs.s2;
+  a.tiles0 = D / kStreamCols;
+  a.gather = 0;
+  launch_w4_stream<BF16, true>(a, D / kStreamCols, L.max_tiles, st);
+  hipLaunchKernelGGL((moe_reduce_combine_kernel<BF16>),
+                     dim3((unsigned)(((size_t)T * D / 4 + 255) / 256)), dim3(256), 0, st,
+                     (const float*)part, fs.s2, mb.topw, (uint16_t*)y, T, D);
+}
+
 // FFN layout: TM-row tiles (the plan's) and room for the down projection's split-K partials when the wide
 // path applies (plan_ffn); otherwise the 256 x 128 grouped kernels run.
-MoeLayout ffn_layout(int T, int E, int D, int F, int group, bool* wide, FfnPlan* fp) {
+MoeLayout ffn_layout(int T, int E, int D, int F, int group, bool* wide, FfnPlan* fp, bool* stream,
+                     FfnStream* fs) {
+  *wide = false;
+  *stream = plan_ffn_stream(T, E, D, F, group, fs);
+  if (*stream) {  // the down projection's slices reuse the gate/up ones' place
+    const size_t gu = (size_t)fs->s1 * 2 * T * 2 * F * 4, dn = (size_t)fs->s2 * 2 * T * D * 4;
+    return moe_layout(T, E, F, 0, 16, gu > dn ? gu : dn);
+  }
   // The wide path stages x (T x D) and h (2T x F) through LDS with 32-bit buffer offsets, so it
   // needs 2T rows of either under 2 GiB; beyond that the grouped kernels (64-bit addresses) run.
   const size_t act_bytes = (size_t)2 * T * (size_t)(D > F ? D : F) * 2;
@@ -1033,9 +1130,10 @@ extern "C" size_t kbh_qmoe_ffn_workspace_bytes(int T, int D, int F, int E) {
   // groups (the split count of the down projection, hence its partials, depends on it).
   size_t best = 0;
   for (int group : {32, 64, 128, 256}) {
-    bool wide;
+    bool wide, stream;
     kbh::FfnPlan fp;
-    const size_t b = kbh::ffn_layout(T, E, D, F, group, &wide, &fp).total;
+    kbh::FfnStream fs;
+    const size_t b = kbh::ffn_layout(T, E, D, F, group, &wide, &fp, &stream, &fs).total;
     best = b > best ? b : best;
   }
   return best;
@@ -1060,9 +1158,10 @@ extern "C" int kbh_qmoe_ffn(const void* x, const void* router_logits, int logits
                         down_qweight, down_scales, down_zeros, y};
   for (const void* p : ptrs)
     if (!aligned16(p)) return KBH_ERR_ALIGN;
-  bool wide;
+  bool wide, streamed;
   FfnPlan fp;
-  const MoeLayout L = ffn_layout(T, E, D, F, group, &wide, &fp);
+  FfnStream fs;
+  const MoeLayout L = ffn_layout(T, E, D, F, group, &wide, &fp, &streamed, &fs);
   if (workspace_bytes < L.total) return KBH_ERR_WORKSPACE;
   const MoeBuffers mb = moe_buffers(workspace, L);
   hipStream_t st = (hipStream_t)stream;
@@ -1073,8 +1172,16 @@ extern "C" int kbh_qmoe_ffn(const void* x, const void* router_logits, int logits
   // gate/up: [D -> F] packed along F; down: [F -> D] packed along D
   const size_t gq = (size_t)D * (F / 8), gs = (size_t)(D / group) * F;
   const size_t dq = (size_t)F * (D / 8), ds = (size_t)(F / group) * D;
+  float* part = (float*)((char*)workspace + L.part);
+  if (streamed) {
+    const W4Mat gm{(const uint32_t*)gate_qweight, (const uint16_t*)gate_scales, (const uint16_t*)gate_zeros};
+    const W4Mat um{(const uint32_t*)up_qweight, (const uint16_t*)up_scales, (const uint16_t*)up_zeros};
+    const W4Mat dm{(const uint32_t*)down_qweight, (const uint16_t*)down_scales, (const uint16_t*)down_zeros};
+    if (bf) launch_ffn_stream<true>(fs, L, mb, x, gm, um, dm, h, part, y, T, D, F, group, gq, gs, dq, ds, st);
+    else launch_ffn_stream<false>(fs, L, mb, x, gm, um, dm, h, part, y, T, D, F, group, gq, gs, dq, ds, st);
+    return launch_status();
+  }
   if (wide) {
-    float* part = (float*)((char*)workspace + L.part);
     if (bf)
       launch_ffn_wide<true>(fp, L, mb, x, gate_qweight, gate_scales, gate_zeros, up_qweight,
                             up_scales, up_zeros, down_qweight, down_scales, down_zeros, h, o, part,

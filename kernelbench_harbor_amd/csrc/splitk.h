@@ -21,18 +21,16 @@ namespace kbh {
 constexpr int kSplitKMaxWaves = 8;
 constexpr int kSplitKCsStride = 260;  // LDS elements per column set per wave (4*64 + pad)
 
-template <int NCS, typename T>
+template <int NCS, typename T, int WAVES = kSplitKMaxWaves>
 struct SplitKSmem {
-  __attribute__((aligned(16))) T red[kSplitKMaxWaves * NCS * kSplitKCsStride];
+  __attribute__((aligned(16))) T red[WAVES * NCS * kSplitKCsStride];
 };
 
 // V is the 4-element vector of T held per column set (kbh_f32x4 / kbh_i32x4).
-// emit(r, n, v): row r (< rows) of the tile, column n (< 16*NCS), reduced value v (splits == 1).
-// M: rows of one workspace slice; ld: its row stride (the output's N).
-template <int NCS, typename T, typename V, typename Emit>
-__device__ inline void splitk_reduce(const V (&tot)[NCS], SplitKSmem<NCS, T>& sm, T* acc,
-                                     int split, int splits, int rows, int M, int ld, int m0,
-                                     int n0, Emit emit) {
+// store(r, n, v): row r (< rows) of the tile, column n (< 16*NCS), value v summed over the waves.
+template <int NCS, typename T, typename V, int WAVES, typename Store>
+__device__ inline void splitk_wave_sum(const V (&tot)[NCS], SplitKSmem<NCS, T, WAVES>& sm, int rows,
+                                       Store store) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   if (4 * (lane >> 4) < rows) {
     T* slice = sm.red + wave * NCS * kSplitKCsStride;
@@ -54,13 +52,23 @@ __device__ inline void splitk_reduce(const V (&tot)[NCS], SplitKSmem<NCS, T>& sm
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 4 * (l >> 4) + i;
-      if (r >= rows) continue;
-      if (splits == 1)
-        emit(r, n, v[i]);
-      else
-        acc[((size_t)split * M + m0 + r) * ld + n0 + n] = v[i];
+      if (r < rows) store(r, n, v[i]);
     }
   }
+}
+
+// emit(r, n, v): row r (< rows) of the tile, column n (< 16*NCS), reduced value v (splits == 1).
+// M: rows of one workspace slice; ld: its row stride (the output's N).
+template <int NCS, typename T, typename V, typename Emit>
+__device__ inline void splitk_reduce(const V (&tot)[NCS], SplitKSmem<NCS, T>& sm, T* acc,
+                                     int split, int splits, int rows, int M, int ld, int m0,
+                                     int n0, Emit emit) {
+  splitk_wave_sum<NCS, T, V>(tot, sm, rows, [&](int r, int n, T v) {
+    if (splits == 1)
+      emit(r, n, v);
+    else
+      acc[((size_t)split * M + m0 + r) * ld + n0 + n] = v;
+  });
 }
 
 // Sums the fp32 split-K slices acc[splits][M*N] in split order and converts the sums to
