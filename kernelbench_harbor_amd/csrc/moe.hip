@@ -773,23 +773,16 @@ __global__ __launch_bounds__(256) void moe_silu_sum_kernel(const float* __restri
 // 322 / 439 / 450 / 444 / 514 -> 60 / 157 / 172 / 246 / 378 us (T=8 is 757 MB at 4.8 TB/s, the
 // rate of a large copy). Each 16-row tile past an expert's first costs its conversion again; the
 // line at 32 rows is where the 128-row tiles' measured cost is met within the range tested (1.36x
-// at 127 tokens). Both GEMMs split K until the tiles the batch can reach are about two workgroups
-// per CU, and leave fp32 slices.
+// at 127 tokens). Both GEMMs leave fp32 slices, K split for the tiles the batch can reach.
 struct FfnStream {
   int s1, s2;  // K splits of gate/up and of down
 };
 bool plan_ffn_stream(int T, int E, int D, int F, int group, FfnStream* p) {
   if ((size_t)2 * T >= (size_t)32 * E) return false;
   if (!w4_stream_ok(F, D, group) || !w4_stream_ok(D, F, group)) return false;
-  const int unit = group > kStreamChunk ? group : kStreamChunk;
   const int reach = 2 * T < E ? 2 * T : E;  // experts the batch can reach
-  auto splits = [&](int col_tiles, int K) {
-    const int want = (512 + col_tiles * reach - 1) / (col_tiles * reach);
-    const int most = K / unit / kStreamWaves;  // at least one unit per wave
-    return want < 1 ? 1 : (want > most ? (most > 1 ? most : 1) : want);
-  };
-  p->s1 = splits(2 * F / kStreamCols, D);
-  p->s2 = splits(D / kStreamCols, F);
+  p->s1 = w4_stream_splits(2 * T, F, D, group, reach, 2);
+  p->s2 = w4_stream_splits(2 * T, D, F, group, reach, 1);
   return true;
 }
 

@@ -223,6 +223,33 @@ inline bool w4_stream_ok(int N, int K, int group) {
   return N % kStreamCols == 0 && K % unit == 0 && (size_t)K * N / 2 < ((size_t)1 << 31);
 }
 
+// Estimated cost (decode_cost's units in w4a16.hip) of `row_tiles` row tiles of M rows in all on
+// `mats` K x N matrices split s ways: the weight KB a CU streams, one workgroup after another at
+// 22.5 KB per unit (a second round beside the first gains nothing: dense K=29568 N=8192 M=16 128 /
+// 256 / 448 workgroups 50.1 / 34.2 / 37.2 us; eight waves per workgroup measured the same) with a
+// fixed cost of its own, and the fp32 slices written and read.
+inline float w4_stream_cost(int M, int N, int K, int row_tiles, int mats, int s) {
+  const long wgs = (long)(N / kStreamCols) * row_tiles * mats * s;
+  const float kb = (float)K / s * (kStreamCols / 2048.0f);  // of one workgroup
+  return 3.7f + (float)((wgs + 255) / 256) * (1.0f + kb / 22.5f) + (float)s * M * N * mats * 8.0f / 1024.0f / 2540.0f;
+}
+
+// The K split of least estimated cost with at least one unit of K per wave.
+inline int w4_stream_splits(int M, int N, int K, int group, int row_tiles, int mats) {
+  const int unit = group > kStreamChunk ? group : kStreamChunk;
+  const int most = K / unit / kStreamWaves;
+  int best = 1;
+  float c = w4_stream_cost(M, N, K, row_tiles, mats, 1);
+  for (int s = 2; s <= most && s <= 64; ++s) {
+    const float cs = w4_stream_cost(M, N, K, row_tiles, mats, s);
+    if (cs < c) {
+      c = cs;
+      best = s;
+    }
+  }
+  return best;
+}
+
 template <bool BF16, bool GROUPED>
 void launch_w4_stream(const W4StreamArgs& a, int col_tiles, int row_tiles, hipStream_t st) {
   const dim3 grid((unsigned)(col_tiles * a.splits), (unsigned)row_tiles), block(64 * kStreamWaves);

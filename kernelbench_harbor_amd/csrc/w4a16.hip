@@ -38,6 +38,7 @@
 #include "tiled_ws.h"
 #include "tiled_ws256.h"
 #include "w4_dequant.h"
+#include "w4_stream.h"
 
 namespace kbh {
 namespace {
@@ -190,6 +191,8 @@ __global__ __launch_bounds__(kSplitKMaxWaves * 64) void w4a16_decode_kernel(
   });
 }
 
+constexpr int kWideMinM = 33;  // rows from which the wide tiles take over (below)
+
 struct DecodePlan {
   int nw, spw, spg, waves, ntiles, splits, mblocks;
 };
@@ -274,6 +277,52 @@ void launch_decode(const DecodePlan& p, const void* x, const int32_t* qw, const 
                       p.ntiles, 128 * NW, p.splits, stream);
 }
 
+// The streaming kernel (w4_stream.h) takes the calls that the decode kernel runs in several rounds
+// of workgroups, each of which fills and drains the memory pipeline: large layers, two row blocks,
+// and K x N that no wave split divides well (K = 11008, 18944, 29568). The two estimates
+// decide. Measured (decode -> stream, us, group 128 fp16) at M=16: 11008 x 4096 19.8 -> 13.7,
+// 18944 x 3584 23.9 -> 16.6, 28672 x 8192 38.9 -> 32.8, 29568 x 8192 51.3 -> 34.1, 8192 x 28672
+// 37.6 -> 35.8, 4096 x 128256 74.1 -> 56.9; M=32: 36.4 -> 16.0, 38.1 -> 23.5, 71.4 -> 49.3, 90.5 ->
+// 51.5, 70.2 -> 58.0, 140 -> 115. One-round grids stay with the decode kernel (14336 x 4096 M=16
+// 13.1 against 14.4, 4096 x 14336 13.1 / 14.7), as does an unsplit K (it writes y itself: K=512
+// N=66304 M=16 11.6 / 14.9). Returns the K splits, 0 for the decode kernel.
+int plan_stream(const DecodePlan& d, int M, int N, int K, int group) {
+  if (M >= kWideMinM || d.splits == 1 || !w4_stream_ok(N, K, group)) return 0;
+  const int mb = (M + 15) / 16;
+  const int s = w4_stream_splits(M, N, K, group, mb, 1);
+  // Where either plan's slices exceed the no-alloc entry point's array (they are written also when
+  // K is unsplit), the decode plan stays: that entry point accepts and refuses what it always has.
+  if ((size_t)s * M * N * 4 > KBH_W4A16_NOALLOC_SCRATCH_BYTES ||
+      splitk_workspace_bytes(M, N, d.splits) > KBH_W4A16_NOALLOC_SCRATCH_BYTES)
+    return 0;
+  const float dec = decode_cost(M, N, d.nw, d.spw, d.waves, d.splits, d.ntiles * d.splits * d.mblocks);
+  return w4_stream_cost(M, N, K, mb, 1, s) < dec ? s : 0;
+}
+
+// Workspace of a call on the decode or the streaming kernel.
+size_t decode_workspace_bytes(const DecodePlan& d, int M, int N, int K, int group) {
+  const int s = plan_stream(d, M, N, K, group);
+  return s > 0 ? round_up((size_t)s * M * N * 4, 256) : splitk_workspace_bytes(M, N, d.splits);
+}
+
+template <bool BF16>
+void launch_dense_stream(int splits, const void* x, const int32_t* qw, const void* s, const void* z,
+                         void* y, float* slices, int M, int N, int K, int group, hipStream_t st) {
+  W4StreamArgs a{};
+  a.x = (const uint16_t*)x;
+  a.mat[0] = a.mat[1] = W4Mat{(const uint32_t*)qw, (const uint16_t*)s, (const uint16_t*)z};
+  a.slices = slices;
+  a.M = M;
+  a.ld = a.N = N;
+  a.K = K;
+  a.group = group;
+  a.splits = splits;
+  a.tiles0 = N / kStreamCols;
+  launch_w4_stream<BF16, false>(a, a.tiles0, (M + 15) / 16, st);
+  launch_splitk_sum(reinterpret_cast<const kbh_f32x4*>(slices), HalfOut<BF16>{(uint16_t*)y, N}, M,
+                    N, a.tiles0, kStreamCols, splits, st);
+}
+
 template <bool BF16>
 void dispatch_decode(const DecodePlan& p, const void* x, const int32_t* qw, const void* s,
                      const void* z, void* y, float* acc, int M, int N, int K, int group,
@@ -297,7 +346,6 @@ void dispatch_decode(const DecodePlan& p, const void* x, const int32_t* qw, cons
 // form (tiled_ws256.h: 4 waves stage weights and x, 8 MFMA waves; K=14336 N=4096 M=1024
 // 153.0 -> 131.7 us, M=2048 282.7 -> 245.9 us against the 4-wave kernel). The older 256 x 128
 // LDS-staged kernel remains for shapes the wide kernel does not cover.
-constexpr int kWideMinM = 33;
 constexpr int kTiledMinM = 128;
 
 struct W4Wide {
@@ -427,7 +475,7 @@ size_t w4a16_path_bytes(int M, int N, int K, int group) {
   if (M >= kTiledMinM && K % (TBK * TDEPTH) == 0) return 0;
   DecodePlan p;
   if (!plan_decode(M, N, K, group / 32, &p)) return 0;
-  return splitk_workspace_bytes(M, N, p.splits);
+  return decode_workspace_bytes(p, M, N, K, group);
 }
 
 }  // namespace kbh
@@ -436,7 +484,7 @@ extern "C" size_t kbh_w4a16_workspace_bytes(int M, int N, int K, int group) {
   kbh::DecodePlan p;
   if (M < 1 || N < 128 || K < 32 || group < 32 || !kbh::plan_decode(M, N, K, group / 32, &p))
     return 0;
-  return kbh::splitk_workspace_bytes(M, N, p.splits);
+  return kbh::decode_workspace_bytes(p, M, N, K, group);
 }
 
 extern "C" size_t kbh_w4a16_scratch_bytes(int M, int N, int K, int group) {
@@ -488,10 +536,16 @@ extern "C" int kbh_w4a16_gemm(const void* x, const int32_t* qweight, const void*
 
   DecodePlan p;
   if (!plan_decode(M, N, K, group / 32, &p)) return KBH_ERR_SHAPE;
-  const size_t need = splitk_workspace_bytes(M, N, p.splits);
+  const int ss = plan_stream(p, M, N, K, group);  // its slices are written also when K is unsplit
+  const size_t need = decode_workspace_bytes(p, M, N, K, group);
   if (need > 0 && (!workspace || workspace_bytes < need)) return KBH_ERR_WORKSPACE;
   if (need > 0 && !aligned16(workspace)) return KBH_ERR_ALIGN;
   float* acc = (float*)workspace;
+  if (ss > 0) {
+    if (bf) launch_dense_stream<true>(ss, x, qweight, scales, zeros, y, acc, M, N, K, group, st);
+    else launch_dense_stream<false>(ss, x, qweight, scales, zeros, y, acc, M, N, K, group, st);
+    return launch_status();
+  }
   if (bf) dispatch_decode<true>(p, x, qweight, scales, zeros, y, acc, M, N, K, group, st);
   else dispatch_decode<false>(p, x, qweight, scales, zeros, y, acc, M, N, K, group, st);
   return launch_status();

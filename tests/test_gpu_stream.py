@@ -6,9 +6,10 @@ import numpy as np
 import pytest
 import torch
 
-from kernelbench_harbor_amd import inputs, ops
+from kernelbench_harbor_amd import _lib, inputs, ops
 from kernelbench_harbor_amd.harness import compare
 from oracle import qmoe as oq
+from oracle import w4a16 as ow
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +61,32 @@ def test_ffn_stream_full_width(dev):
     down = [a[8][:, :, -32:], a[9][:, :, -256:], a[10][:, :, -256:]]
     cmp = compare(y[:, -256:], oq.ffn_forward(*a[:8], *down))
     assert cmp.ok, cmp
+
+
+# K, N, group, K splits at M = 16: shapes whose decode grid is several workgroups per CU
+DENSE = [(18944, 2048, 128, 32), (18944, 2048, 64, 32), (9472, 4096, 32, 16), (4864, 8448, 256, 4),
+         (2048, 66304, 64, 2)]
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M", [1, 16, 17, 32])
+@pytest.mark.parametrize("K,N,group,splits", DENSE)
+def test_w4a16_stream(dev, K, N, group, splits, M, dtype):
+    """Dense rows: whole and partial 16-row tiles, uneven K ranges, unsplit K (M > 17 of the last shape); the first and last
+    256 columns against the oracle, and the no-alloc entry point's bits."""
+    if M == 16:  # the streaming plan (its slices)
+        assert _lib.load().kbh_w4a16_workspace_bytes(M, N, K, group) == splits * M * N * 4
+    x, q, s, z = inputs.w4a16(M, K, N, group, dtype, seed=M + K)
+    d = [t.to(dev) for t in (x, q, s, z)]
+    y = ops.w4a16_gemm(*d)
+    for c in (slice(0, 256), slice(N - 256, N)):
+        w = slice(c.start // 8, c.stop // 8)
+        gt = ow.forward(x.float().numpy(), q[:, w].numpy(), s[:, c].float().numpy(), z[:, c].float().numpy())
+        cmp = compare(y[:, c], gt)
+        assert cmp.ok, cmp
+    y2 = torch.empty_like(y)
+    code = 0 if dtype == F16 else 1
+    st = torch.cuda.current_stream().cuda_stream
+    assert _lib.load().kbh_w4a16_gemm_noalloc(*[t.data_ptr() for t in d], y2.data_ptr(), M, N, K,
+                                              group, code, st) == 0
+    assert torch.equal(y, y2)
