@@ -692,6 +692,16 @@ struct W4PairPolicy {
   __device__ void store_all(const Raw& r, const Grp& gr, uint8_t* Bs, int t) const {
     g.template store_all<FAST>(r, gr, Bs, t);
   }
+  // Two producer sets (W4WidePolicy::load_half / store_half).
+  using RawHalf = typename Half::RawHalf;
+  __device__ void load_half(RawHalf& r, int k0, int n0, int t, int half) const {
+    const int w = Half::word_of(t);
+    g.load_half_from(r, (w & 8) ? u.qw : g.qw, k0, n0 / 2 - shift(w), t, half);
+  }
+  template <bool FAST>
+  __device__ void store_half(const RawHalf& r, const Grp& gr, uint8_t* Bs, int t, int half) const {
+    g.template store_half<FAST>(r, gr, Bs, t, half);
+  }
 };
 
 // h[slot][n] = dtype(silu(gate) * up) from the paired accumulators (fp32 math, one rounding).
@@ -792,6 +802,10 @@ bool plan_ffn_stream(int T, int E, int D, int F, int group, FfnStream* p) {
 // 2T/TM x 2F/256 workgroups), down split over K until the estimated 2T/TM x D/256 tiles fill
 // the CUs.
 constexpr int kFfnPD = 4;
+// Producer sets of the 128-row tiles: bf16's fp32 dequantization needs two (Mixtral layer T=512
+// 1013 -> 954 us, T=128 691 -> 661); fp16 is 2-3% faster with one (785 against 802).
+template <bool BF16>
+constexpr int kFfnPS = BF16 ? 2 : 1;
 struct FfnPlan {
   int spg, tm;
   WidePlan down;
@@ -928,8 +942,8 @@ void launch_ffn_wide_spg(const FfnPlan& fp, const MoeLayout& L, const MoeBuffers
     // staged through LDS (XD: 32-bit offsets; ffn_layout takes this path only while 2T rows of
     // x and of h stay under 2 GiB).
     if constexpr (TM == 128)
-      hipLaunchKernelGGL((tiled_ws_gemm<E, TM, 2, SPG, BP, SiluPairOut<BF16>, RM, kFfnPD, 1, true>),
-                         dim3(grid), dim3(512), 0, st, x, bp, ep, (float*)nullptr, 2 * T, 2 * F,
+      hipLaunchKernelGGL((tiled_ws_gemm<E, TM, 2, SPG, BP, SiluPairOut<BF16>, RM, kFfnPD, kFfnPS<BF16>, true>),
+                         dim3(grid), dim3(256 * (1 + kFfnPS<BF16>)), 0, st, x, bp, ep, (float*)nullptr, 2 * T, 2 * F,
                          D, 1, D / 32, RM{mb.tiles, mb.perm});
     else
       hipLaunchKernelGGL((tiled_wide_gemm<E, TM, 4, SPG, BP, SiluPairOut<BF16>, RM, 1, kFfnPD>),
@@ -944,8 +958,8 @@ void launch_ffn_wide_spg(const FfnPlan& fp, const MoeLayout& L, const MoeBuffers
     const int splits = fp.down.splits;
     const int grid = L.max_tiles * (D / 256) * splits;
     if constexpr (TM == 128)
-      hipLaunchKernelGGL((tiled_ws_gemm<E, TM, 2, SPG, BP, HalfOut<BF16>, RM, kFfnPD, 1, true>),
-                         dim3(grid), dim3(512), 0, st, h, dp, ep, part, 2 * T, D, F, splits,
+      hipLaunchKernelGGL((tiled_ws_gemm<E, TM, 2, SPG, BP, HalfOut<BF16>, RM, kFfnPD, kFfnPS<BF16>, true>),
+                         dim3(grid), dim3(256 * (1 + kFfnPS<BF16>)), 0, st, h, dp, ep, part, 2 * T, D, F, splits,
                          fp.down.slabs_per_split, RM{mb.tiles, mb.perm});
     else
       hipLaunchKernelGGL((tiled_wide_gemm<E, TM, 4, SPG, BP, HalfOut<BF16>, RM, 1, kFfnPD>),

@@ -18,8 +18,8 @@
 // (KT is a multiple of half an iteration of U slabs: both roles leave the last iteration in its
 // middle when K ends there):
 // split-K partial tiles go through the LDS ring, so that all 8 waves store whole rows.
-// 64-row tiles run two producer sets (waves 4..7 and 8..11, PS below), each dequantizing one
-// row pair of every thread's four rows.
+// 64-row tiles, and 128-row tiles with bf16 weights to dequantize, run two producer sets (waves
+// 4..7 and 8..11, PS below), each dequantizing one row pair of every thread's four rows.
 // Measured against tiled_wide_gemm (same shapes, graph-replayed, bit-identical outputs): W4A16
 // K=14336 N=4096 M=64 29.1 -> 27.3 us, M=128 38.0 -> 35.3, M=256 55.3 -> 50.4, M=384 84.8 ->
 // 75.5, the Mixtral MoE SiLU FFN T=512 978 -> 864 us. Per-slab timestamps at M=256: the
@@ -45,8 +45,10 @@ struct WsRaw<BP, 2> {
 // PS: producer sets. 1: waves 4..7 dequantize whole slabs. 2: waves 4..7 and 8..11 run the same
 //   loop on the same thread ids and barriers, set p loading and dequantizing row pair p of each
 //   thread's rows (BP::load_half / store_half), so two producer waves share each SIMD's VALU
-//   with the MFMA wave (768 threads, at most 168 VGPRs per wave: 64-row tiles).
-// XD: x through the LDS ring too (128-row tiles, one producer set): the producers stage each
+//   with the MFMA wave (768 threads, at most 168 VGPRs per wave: 64-row tiles, or 128-row tiles
+//   whose MFMA waves read every fragment of a slab after its barrier, as tiled_ws256_gemm's do;
+//   W4A16 bf16 M=256 53.3 -> 50.4 us, the Mixtral FFN bf16 T=512 1047 -> 943).
+// XD: x through the LDS ring too (128-row tiles): the producers stage each
 //   slab's x rows with LDS-mode buffer loads three slabs ahead (as tiled_ws256_gemm does) and the
 //   MFMA waves read their A fragments from LDS instead of holding a register ring of them. The
 //   x offsets are 32-bit: the caller keeps M x K x 2 bytes under 2 GiB.
@@ -65,7 +67,11 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
   constexpr int U = 2 * SPG > PD ? 2 * SPG : PD;  // slabs per loop iteration
   static_assert(PD >= 2 && U % PD == 0 && U % (2 * SPG) == 0 && U % NBUF == 0, "unroll");
   static_assert(PS == 1 || PS == 2, "one or two producer sets");
-  static_assert(!XD || (TM == 128 && PS == 1 && !E::kStageX), "LDS x: 128-row fp16 tiles");
+  static_assert(!XD || (TM == 128 && !E::kStageX), "LDS x: 128-row fp16 tiles");
+  static_assert(PS == 1 || TM == 64 || XD, "two producer sets: 64-row tiles, or x in LDS");
+  // 12 waves leave 168 registers: beside 128 accumulators no fragments held over a barrier.
+  constexpr bool kLean = PS == 2 && TM == 128;
+  constexpr int XB = 2 / PS;  // XD: 16-row x blocks one producer wave stages per slab
   constexpr int NT = 256 * (1 + PS);  // threads
   __shared__ __attribute__((aligned(16))) uint8_t Bs[NBUF][SLAB];
   // XD: x of a slab, row r keeping its 16-byte chunk c at r * 64 + 16 (c ^ ((r >> 2) & 3)).
@@ -123,23 +129,23 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
     for (int i = 0; i < PD; ++i) load_b(R[i], i);
     load_g(G[0], 0);
     load_g(G[1], SPG);
-    // XD: producer wave p stages x blocks 2p and 2p + 1 (16 rows each) of every slab; lane l
-    // takes row l / 4 of a block and the chunk the swizzle puts at position l % 4.
+    // XD: producer wave p stages x blocks XB p .. XB p + XB - 1 (16 rows each) of every slab; lane
+    // l takes row l / 4 of a block and the chunk the swizzle puts at position l % 4.
     uint32_t vxh[2] = {0u, 0u};
     kbh_rsrc4 rx = {0u, 0u, 0u, 0u};
     auto stage_x = [&](int s, int buf) {
       if constexpr (XD) {
         const uint32_t k0b = (uint32_t)((kt0 + min(s, last)) * WSLAB_BYTES);
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-          lds_load16(lds_addr(&Xs[buf][1024 * (2 * (wave - 4) + h)]), vxh[h], rx, k0b);
+        for (int h = 0; h < XB; ++h)
+          lds_load16(lds_addr(&Xs[buf][1024 * (XB * (wave - 4) + h)]), vxh[h], rx, k0b);
       }
     };
     if constexpr (XD) {
       rx = raw_rsrc(x, (size_t)M * K * 2);
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = 16 * (2 * (wave - 4) + h) + (lane >> 2);
+      for (int h = 0; h < XB; ++h) {
+        const int r = 16 * (XB * (wave - 4) + h) + (lane >> 2);
         vxh[h] = (uint32_t)((size_t)rm.a_row(ti, r) * K * 2) +
                  (uint32_t)(16 * ((lane & 3) ^ ((lane >> 4) & 3)));
       }
@@ -167,9 +173,10 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
         put(R[1], G[0], Bs[1]);
       }
       load_b(R[1 % PD], PD + 1);
-      // XD: x of slabs 0 and 1 has landed (younger: slab 2's two x loads, the two raw-word
-      // loads and at most one group load pair)
-      if constexpr (XD) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+      // XD: x of slabs 0 and 1 has landed (younger: slab 2's x loads, the raw words of two slabs
+      // and at most one group load pair)
+      if constexpr (XD && PS == 1) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+      if constexpr (XD && PS == 2) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
       __syncthreads();  // slabs 0 and 1 are in LDS
       // Slab kt + u + 2 during consumer slab kt + u. Slabs past the end re-produce the last one
       // into a buffer nobody reads, so the loop has no branch.
@@ -186,8 +193,10 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
           put(R[pu % PD], G[set], Bs[pu % NBUF]);
           stage_x(kt + u + 3, (u + 3) % NBUF);  // into the x buffer idle during slab kt + u
           load_b(R[pu % PD], kt + pu + PD);
-          // XD: x of the next slab has landed (at least 16 loads are younger)
-          if constexpr (XD) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+          // XD: x of the next slab, staged two iterations ago, has landed (younger: that
+          // iteration's raw words, and x and raw words of the last two)
+          if constexpr (XD && PS == 1) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+          if constexpr (XD && PS == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
           __syncthreads();
         }
       };
@@ -265,8 +274,27 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
         for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
 
     __syncthreads();  // slabs 0 and 1 are in LDS
+    auto lean_half = [&](auto h, int) {
+#pragma unroll
+      for (int uu = 0; uu < U / 2; ++uu) {
+        const int cur = (decltype(h)::value * (U / 2) + uu) % NBUF;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {  // k16 steps
+          kbh_u32x4 af[RB], bf[CB];
+#pragma unroll
+          for (int i = 0; i < RB; ++i)
+            af[i] = *reinterpret_cast<const kbh_u32x4*>(&Xs[cur][xoff[st] + 2048 * i]);
+          read_b(bf, cur, st);
+#pragma unroll
+          for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < CB; ++j) acc[i][j] = E::mma(af[i], bf[j], acc[i][j]);
+        }
+        __syncthreads();
+      }
+    };
     kbh_u32x4 b0[CB], b1[CB];
-    read_b(b0, 0, 0);
+    if constexpr (!kLean) read_b(b0, 0, 0);
     constexpr int NMF = RB * CB;  // MFMAs per k16 step
     auto half = [&](auto h, int kt) {
 #pragma unroll
@@ -298,12 +326,16 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
         __syncthreads();
       }
     };
-    int kt = 0;
-    for (; kt + U <= KT; kt += U) {
-      half(WideIdx<0>{}, kt);
-      half(WideIdx<1>{}, kt);
-    }
-    if (kt < KT) half(WideIdx<0>{}, kt);  // as the producers
+    auto run = [&](auto& body) {
+      int kt = 0;
+      for (; kt + U <= KT; kt += U) {
+        body(WideIdx<0>{}, kt);
+        body(WideIdx<1>{}, kt);
+      }
+      if (kt < KT) body(WideIdx<0>{}, kt);  // as the producers
+    };
+    if constexpr (kLean) run(lean_half);
+    else run(half);
   }
 
   if constexpr (!EP::kPaired) {

@@ -357,10 +357,13 @@ struct W4WidePolicy {
     uint32_t w[2];
   };
   __device__ void load_half(RawHalf& r, int k0, int n0, int t, int half) const {
+    load_half_from(r, qw, k0, n0, t, half);
+  }
+  __device__ void load_half_from(RawHalf& r, const uint32_t* qw_, int k0, int n0, int t, int half) const {
     static_assert(kRows == 4, "row pairs of 4-row threads");
     const int w = word_of(t), h = rows_of(t);
     const int NP = N >> 3;
-    const uint32_t* q = qw + (size_t)(k0 + kRows * h + 2 * half) * NP + (n0 >> 3) + w;
+    const uint32_t* q = qw_ + (size_t)(k0 + kRows * h + 2 * half) * NP + (n0 >> 3) + w;
     r.w[0] = q[0];
     r.w[1] = q[NP];
   }

@@ -399,7 +399,10 @@ void launch_w4_wide(const W4Wide& w, const void* x, const int32_t* qw, const voi
   // Producer sets of the warp-specialised kernel: two for 64-row tiles, whose MFMA waves need
   // only 64 accumulator registers, so that 12 waves fit (K=14336 N=4096: M=33 24.2 -> 23.5 us,
   // M=48 25.4 -> 24.7, M=64 26.7 -> 26.4; an 8-slab raw ring on top measured no faster).
-  constexpr int PS = TM == 64 ? 2 : 1;
+  // bf16 takes two sets for 128-row tiles as well: its fp32 dequantization is about twice fp16's
+  // instructions (group 128, 4096 x 4096 M=128 27.6 -> 26.6 us; the Mixtral FFN T=512 1013 -> 954);
+  // fp16 is 1-3% faster with one (M=256 45.2 against 46.0).
+  constexpr int PS = TM == 64 || BF16 ? 2 : 1;
   if constexpr (TM <= 128 && TN == 256) {
     // 128-row tiles stage x through LDS too (XD) while x is under 2 GiB.
     if (TM == 128 && (size_t)M * K * 2 < ((size_t)1 << 31))
@@ -409,8 +412,8 @@ void launch_w4_wide(const W4Wide& w, const void* x, const int32_t* qw, const voi
                          x, bp, ep, scratch, M, N, K, w.plan.splits, w.plan.slabs_per_split,
                          DenseRows{M});
     else
-      hipLaunchKernelGGL((tiled_ws_gemm<E, TM, WM, SPG, BP, EP, DenseRows, w4_wide_pd(TN), PS>),
-                         dim3(w.plan.grid), dim3(256 * (1 + PS)), 0, st,
+      hipLaunchKernelGGL((tiled_ws_gemm<E, TM, WM, SPG, BP, EP, DenseRows, w4_wide_pd(TN), TM == 64 ? 2 : 1>),
+                         dim3(w.plan.grid), dim3(TM == 64 ? 768 : 512), 0, st,
                          x, bp, ep, scratch, M, N, K, w.plan.splits, w.plan.slabs_per_split,
                          DenseRows{M});
   } else {
