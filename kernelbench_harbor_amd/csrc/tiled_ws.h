@@ -180,7 +180,10 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
       __syncthreads();  // slabs 0 and 1 are in LDS
       // Slab kt + u + 2 during consumer slab kt + u. Slabs past the end re-produce the last one
       // into a buffer nobody reads, so the loop has no branch.
-      auto half = [&](auto h, int kt) {
+      // half<H>, TAIL: the half iteration that ends K, where the compiler drops the loads of raw
+      // words past the end (never used), so that only the x loads count for the wait.
+      auto half = [&](auto h, auto tail, int kt) {
+        constexpr bool TAIL = decltype(tail)::value;
 #pragma unroll
         for (int i = 0; i < U / 2; ++i) {
           const int u = decltype(h)::value * (U / 2) + i;
@@ -195,17 +198,19 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
           load_b(R[pu % PD], kt + pu + PD);
           // XD: x of the next slab, staged two iterations ago, has landed (younger: that
           // iteration's raw words, and x and raw words of the last two)
-          if constexpr (XD && PS == 1) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-          if constexpr (XD && PS == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+          if constexpr (XD && TAIL && PS == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+          if constexpr (XD && TAIL && PS == 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+          if constexpr (XD && !TAIL && PS == 1) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+          if constexpr (XD && !TAIL && PS == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
           __syncthreads();
         }
       };
       int kt = 0;
       for (; kt + U <= KT; kt += U) {
-        half(WideIdx<0>{}, kt);
-        half(WideIdx<1>{}, kt);
+        half(WideIdx<0>{}, WideFlag<false>{}, kt);
+        half(WideIdx<1>{}, WideFlag<false>{}, kt);
       }
-      if (kt < KT) half(WideIdx<0>{}, kt);  // K ends in half an iteration
+      if (kt < KT) half(WideIdx<0>{}, WideFlag<true>{}, kt);  // K ends in half an iteration
     };
     if constexpr (kFast) {
       if (fast) produce(WideFlag<true>{});

@@ -122,7 +122,10 @@ __global__ __launch_bounds__(768, 1) void tiled_ws256_gemm(
       // at most one group load pair)
       asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
       __syncthreads();  // slabs 0 and 1 are in LDS
-      auto half = [&](auto h, int kt) {
+      // TAIL: the half iteration that ends K (see tiled_ws.h: only the x loads are sure to be
+      // issued there)
+      auto half = [&](auto h, auto tail, int kt) {
+        constexpr bool TAIL = decltype(tail)::value;
 #pragma unroll
         for (int i = 0; i < U / 2; ++i) {
           const int u = decltype(h)::value * (U / 2) + i;
@@ -139,16 +142,17 @@ __global__ __launch_bounds__(768, 1) void tiled_ws256_gemm(
           load_b(R[pu % PD], kt + pu + PD);
           // x of the next slab (issued two iterations ago) has landed: at least 20 loads are
           // younger (4 raw words of that iteration, 8-10 loads of each of the last two).
-          asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
+          if constexpr (TAIL) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+          else asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
           __syncthreads();
         }
       };
       int kt = 0;
       for (; kt + U <= KT; kt += U) {
-        half(WideIdx<0>{}, kt);
-        half(WideIdx<1>{}, kt);
+        half(WideIdx<0>{}, WideFlag<false>{}, kt);
+        half(WideIdx<1>{}, WideFlag<false>{}, kt);
       }
-      if (kt < KT) half(WideIdx<0>{}, kt);  // K ends in half an iteration
+      if (kt < KT) half(WideIdx<0>{}, WideFlag<true>{}, kt);  // K ends in half an iteration
     };
     if constexpr (kFast) {
       if (fast) produce(WideFlag<true>{});

@@ -81,3 +81,22 @@ def test_w4a16_odd_number_of_groups(dev, M, K, N, group, dtype):
     y = ops.w4a16_gemm(*[t.to(dev) for t in (x, q, s, z)])
     cmp = compare(y, ow.forward(x.float().numpy(), q.numpy(), s.float().numpy(), z.float().numpy()))
     assert cmp.ok, cmp
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M,K,group", [(2100, 256, 256), (2100, 640, 128), (8200, 128, 128)])
+def test_w4a16_half_iteration_tails(dev, M, K, group, dtype):
+    """K ranges that end (or lie wholly) in half an iteration, on many workgroups at once: there
+    the compiler drops the raw-word loads past the end, so the wait for the staged x rows may count
+    the x loads alone. Every row against the oracle, and twice the same bits."""
+    N = 256
+    x, q, s, z = inputs.w4a16(M, K, N, group, dtype, seed=M)
+    d = [t.to(dev) for t in (x, q, s, z)]
+    y = ops.w4a16_gemm(*d)
+    gt = torch.from_numpy(np.asarray(ow.forward(x.float().numpy(), q.numpy(), s.float().numpy(),
+                                                z.float().numpy())))
+    err = (y.float().cpu() - gt).abs().amax(dim=1) / gt.abs().amax()
+    # one rounding of the output and one of each weight: 2^-8 (bf16) covers both in every row
+    assert err.max() <= 2.0 ** -8, (int(err.argmax()), float(err.max()))
+    for _ in range(3):
+        assert torch.equal(y, ops.w4a16_gemm(*d))
