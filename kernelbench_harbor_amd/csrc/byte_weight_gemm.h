@@ -344,7 +344,7 @@ struct ByteWide {
 };
 
 // Wide tiles from kByteWideMinM rows: the W4A16 geometry (64-row tiles up to 64 rows, 128-row
-// ones up to 256, 256-row ones above unless the estimate prefers 128 rows). They replace
+// ones up to 128, then 128 or 256 rows by the estimate). They replace
 // tiled_f16_gemm's 256 x 128 tiles, which split no K (K=14336 N=4096: 32 workgroups and ~300 us
 // at every M from 128 to 1024; now 30.7 / 43.0 / 75.2 / 124 us at M=128 / 256 / 512 / 1024, and
 // 342 -> 226 at 2048), and the decode kernel's 64-row blocks (M=48 42.9 -> 21.8, M=96 73.2 ->
@@ -353,14 +353,14 @@ struct ByteWide {
 // 19.8 us, K=2048 N=8192 15.5 / 19.6; with a second round of workgroups the wide tiles win:
 // K=4096 N=6144 25.6 / 18.6, K=N=3584 16.9 / 15.9).
 bool plan_byte_wide(int M, int N, int K, int block, ByteWide* w) {
-  if (M < kByteWideMinM || N % 256 != 0) return false;
+  if (M < kByteWideMinM || N < 256) return false;
   // the kernels stage x with 32-bit offsets
   if ((size_t)(M + 256) * K * 2 >= ((size_t)1 << 31)) return false;
   BytePlan d;
   if (M <= 64 && plan_byte_decode(M, N, K, &d) && d.ntiles * d.splits * d.mblocks <= 256) return false;
   w->spg = block / 32;
-  return plan_wide(M, N, K, 256, 32, wide_k_unroll(K, w->spg, kByteWidePD), 256, &w->plan,
-                   M <= 64 ? 64 : 128, true, 256);
+  const int unit = wide_iteration(w->spg, kByteWidePD) / 2;
+  return plan_wide(M, N, K, 256, 32, unit, unit, 256, kHalfCosts, &w->plan, M <= 64 ? 64 : 128);
 }
 
 template <bool BF16, int DEC, int SPG>
@@ -374,15 +374,13 @@ void launch_byte_wide(const ByteWide& w, const void* x, const void* wt, const vo
   const WidePlan& p = w.plan;
   if (p.tm == 256)
     hipLaunchKernelGGL((tiled_ws256_gemm<E, SPG, BP, EP, kByteWidePD>), dim3(p.grid), dim3(768), 0,
-                       st, x, bp, ep, slices, M, N, K, p.splits, p.slabs_per_split);
+                       st, x, bp, ep, slices, M, N, K, p.sp);
   else if (p.tm == 128)  // bf16's fp32 dequantization: two producer sets (M=256 44.4 -> 43.6 us)
     hipLaunchKernelGGL((tiled_ws_gemm<E, 128, 2, SPG, BP, EP, DenseRows, kByteWidePD, BF16 ? 2 : 1, true>),
-                       dim3(p.grid), dim3(BF16 ? 768 : 512), 0, st, x, bp, ep, slices, M, N, K, p.splits,
-                       p.slabs_per_split, DenseRows{M});
+                       dim3(p.grid), dim3(BF16 ? 768 : 512), 0, st, x, bp, ep, slices, M, N, K, p.sp, DenseRows{M});
   else
     hipLaunchKernelGGL((tiled_ws_gemm<E, 64, 2, SPG, BP, EP, DenseRows, kByteWidePD, 2>),
-                       dim3(p.grid), dim3(768), 0, st, x, bp, ep, slices, M, N, K, p.splits,
-                       p.slabs_per_split, DenseRows{M});
+                       dim3(p.grid), dim3(768), 0, st, x, bp, ep, slices, M, N, K, p.sp, DenseRows{M});
 }
 
 // Runs the GEMM; with `defer_sum` and a split K the slices are left in the workspace

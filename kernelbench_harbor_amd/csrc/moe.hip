@@ -799,8 +799,7 @@ bool plan_ffn_stream(int T, int E, int D, int F, int group, FfnStream* p) {
 // FFN plan: TM x 256 expert tiles (TM = 256 rows when experts average at least 192 routed rows,
 // else 128: at ~128 rows per expert, 256-row tiles measured 20% slower despite fewer tiles), one
 // workgroup per CU with a 4-slab prefetch ring; gate/up unsplit (about
-// 2T/TM x 2F/256 workgroups), down split over K until the estimated 2T/TM x D/256 tiles fill
-// the CUs.
+// 2T/TM x 2F/256 workgroups), down split over K by the wide tiles' cost estimate.
 constexpr int kFfnPD = 4;
 // Producer sets of the 128-row tiles: bf16's fp32 dequantization needs two (Mixtral layer T=512
 // 1013 -> 954 us, T=128 691 -> 661); fp16 is 2-3% faster with one (785 against 802).
@@ -813,9 +812,18 @@ struct FfnPlan {
 bool plan_ffn(int T, int E, int D, int F, int group, FfnPlan* p) {
   p->spg = group / 32;
   p->tm = (2 * T) / (E > 0 ? E : 1) >= 192 ? 256 : 128;
-  const int unroll = 2 * p->spg > kFfnPD ? 2 * p->spg : kFfnPD;  // the kernel's slabs per iteration
+  const int unroll = wide_iteration(p->spg, kFfnPD);
   if (F % 128 != 0 || D % 256 != 0 || D % (unroll * 32) != 0 || F % (unroll * 32) != 0) return false;
-  return plan_wide(2 * T, D, F, 256, 32, unroll, 256, &p->down, p->tm == 256 ? 256 : 128);
+  // down: the row tiles the batch makes (each expert's last one half full on average). Few tiles
+  // are split for four rounds of short workgroups (Mixtral T=256 595 us with 8 splits, 606 with 4,
+  // 631 with 2); many stay whole (T=512 778 us with 4 splits, 744 unsplit).
+  const int unit = p->tm == 256 ? unroll : unroll / 2;
+  const long rows = (2L * T + p->tm - 1) / p->tm + E / 2;
+  const long tiles = (rows > E ? rows : E) * (D / 256);
+  const int s = plan_splits(tiles, 2 * T, D, F / 32, unit, tiles < 160 ? 1024 : 256,
+                            p->tm == 256 ? kHalfCosts.h256 : kHalfCosts.h128, kHalfCosts);
+  p->down = WidePlan{p->tm, s, wide_split(F / 32, unit, s), 0};
+  return s > 0;
 }
 
 // ---- host side ------------------------------------------------------------------------------
@@ -944,11 +952,11 @@ void launch_ffn_wide_spg(const FfnPlan& fp, const MoeLayout& L, const MoeBuffers
     if constexpr (TM == 128)
       hipLaunchKernelGGL((tiled_ws_gemm<E, TM, 2, SPG, BP, SiluPairOut<BF16>, RM, kFfnPD, kFfnPS<BF16>, true>),
                          dim3(grid), dim3(256 * (1 + kFfnPS<BF16>)), 0, st, x, bp, ep, (float*)nullptr, 2 * T, 2 * F,
-                         D, 1, D / 32, RM{mb.tiles, mb.perm});
+                         D, WideSplit{1, D / 32, 0, D / 32}, RM{mb.tiles, mb.perm});
     else
       hipLaunchKernelGGL((tiled_wide_gemm<E, TM, 4, SPG, BP, SiluPairOut<BF16>, RM, 1, kFfnPD>),
                          dim3(grid), dim3(256), 0, st, x, bp, ep, (float*)nullptr, 2 * T, 2 * F,
-                         D, 1, D / 32, RM{mb.tiles, mb.perm});
+                         D, WideSplit{1, D / 32, 0, D / 32}, RM{mb.tiles, mb.perm});
   }
   // down: h rows in slot order, outputs (or split-K partials) in row 2t + k
   {
@@ -959,12 +967,10 @@ void launch_ffn_wide_spg(const FfnPlan& fp, const MoeLayout& L, const MoeBuffers
     const int grid = L.max_tiles * (D / 256) * splits;
     if constexpr (TM == 128)
       hipLaunchKernelGGL((tiled_ws_gemm<E, TM, 2, SPG, BP, HalfOut<BF16>, RM, kFfnPD, kFfnPS<BF16>, true>),
-                         dim3(grid), dim3(256 * (1 + kFfnPS<BF16>)), 0, st, h, dp, ep, part, 2 * T, D, F, splits,
-                         fp.down.slabs_per_split, RM{mb.tiles, mb.perm});
+                         dim3(grid), dim3(256 * (1 + kFfnPS<BF16>)), 0, st, h, dp, ep, part, 2 * T, D, F, fp.down.sp, RM{mb.tiles, mb.perm});
     else
       hipLaunchKernelGGL((tiled_wide_gemm<E, TM, 4, SPG, BP, HalfOut<BF16>, RM, 1, kFfnPD>),
-                         dim3(grid), dim3(256), 0, st, h, dp, ep, part, 2 * T, D, F, splits,
-                         fp.down.slabs_per_split, RM{mb.tiles, mb.perm});
+                         dim3(grid), dim3(256), 0, st, h, dp, ep, part, 2 * T, D, F, fp.down.sp, RM{mb.tiles, mb.perm});
     if (splits > 1) {
       const size_t n4 = (size_t)T * D / 4;
       hipLaunchKernelGGL((moe_reduce_combine_kernel<BF16>), dim3((unsigned)((n4 + 255) / 256)),
@@ -1276,12 +1282,12 @@ extern "C" int kbh_moe(const void* x, const void* w, const void* router_logits, 
       hipLaunchKernelGGL((tiled_ws_gemm<WideHalf<true>, 128, 2, 1, F16WidePolicy, HalfOut<true>, RM,
                                         4, 1, true>),
                          grid, dim3(512), 0, st, x, wp, HalfOut<true>{(uint16_t*)o, H},
-                         (float*)nullptr, (int)S, H, D, 1, D / 32, rm);
+                         (float*)nullptr, (int)S, H, D, WideSplit{1, D / 32, 0, D / 32}, rm);
     else
       hipLaunchKernelGGL((tiled_ws_gemm<WideHalf<false>, 128, 2, 1, F16WidePolicy, HalfOut<false>,
                                         RM, 4, 1, true>),
                          grid, dim3(512), 0, st, x, wp, HalfOut<false>{(uint16_t*)o, H},
-                         (float*)nullptr, (int)S, H, D, 1, D / 32, rm);
+                         (float*)nullptr, (int)S, H, D, WideSplit{1, D / 32, 0, D / 32}, rm);
     if (bf)
       hipLaunchKernelGGL(moe_combine_k_kernel<true>, cgrid, dim3(256), 0, st, (const uint16_t*)o,
                          mb.topw, (uint16_t*)y, T, H, topk);

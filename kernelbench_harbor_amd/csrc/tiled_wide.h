@@ -109,6 +109,19 @@ __device__ __host__ inline int wide_b_offset(int kb, int n) {
   return (kb >> 5) * (TN * 32) + ((kb >> 4) & 1) * (TN * 16) + wide_slot(n) * 16 + (kb & 15);
 }
 
+// The K ranges of a split-K launch, in slabs: whole units of `unit` slabs (the kernel's loop
+// granularity) spread evenly, the first `extra` splits one unit longer than the others' `base`
+// (set up on the host: the kernels divide nothing).
+struct WideSplit {
+  int splits, base, extra, unit;
+  __device__ int begin(int s) const { return s * base + min(s, extra) * unit; }
+  __device__ int count(int s) const { return base + (s < extra ? unit : 0); }
+};
+inline WideSplit wide_split(int slabs, int unit, int splits) {
+  const int units = slabs / unit;
+  return WideSplit{splits, units / splits * unit, units % splits, unit};
+}
+
 struct DenseRows {
   int M;
   struct Tile {
@@ -216,7 +229,7 @@ template <class E, int TM, int WM, int SPG, class BP, class EP, class RM = Dense
 __global__ __launch_bounds__(256, (MINB ? MINB : WideShape<TM, BP::kTN, WM>::kMinBlocks)) void
 tiled_wide_gemm(
     const void* __restrict__ x, BP bp, EP ep, typename E::Part* __restrict__ ws, int M, int N,
-    int K, int splits, int slabs_per_split, RM rm) {
+    int K, WideSplit sp, RM rm) {
   constexpr int TN = BP::kTN;
   constexpr int SK = E::kSlabK;
   constexpr int EB = WSLAB_BYTES / SK;  // bytes per element
@@ -231,16 +244,17 @@ tiled_wide_gemm(
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
   const int wm = wave / WN, wn = wave % WN;
-  const int NB = N / TN;
+  const int splits = sp.splits;
+  const int NB = (N + TN - 1) / TN;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int nb = id % NB;
   const int rest = id / NB;
   const int MB = gridDim.x / (NB * splits);  // row blocks (tile-table entries)
   const int mb = rest % MB;
   const int split = rest / MB;
-  const int n0 = nb * TN;
-  const int kt0 = split * slabs_per_split;
-  const int KT = slabs_per_split;
+  const int n0 = min(nb * TN, N - TN);  // a last tile that N leaves short overlaps its neighbour
+  const int kt0 = sp.begin(split);
+  const int KT = sp.count(split);
   const typename RM::Tile ti = rm.tile(mb, TM);
   if (ti.rows <= 0) return;  // unused tile-table entry (uniform across the workgroup)
   bp = bp.at_expert(ti.expert);
@@ -488,70 +502,98 @@ constexpr size_t kWideMaxSliceBytes = (size_t)64 << 20;
 // Launch geometry: grid = row blocks x column blocks x splits, ids ordered (split, row block,
 // column block) so that consecutive ids, which share an XCD, share a K range.
 struct WidePlan {
-  int tm;               // 128 or 256
-  int splits;           // K ranges
-  int slabs_per_split;  // multiple of the loop unroll
+  int tm;        // tile rows
+  int splits;    // K ranges
+  WideSplit sp;  // their slabs
   int grid;
 };
 
-// Picks the tile height and the split count. Up to small_upto rows (default 128) the tiles are
-// tm_small rows high;
-// above, 256 rows, or (choose_tm) tm_small rows when the cost estimate favours them, i.e. when
-// 256-row tiles would leave CUs idle. `slots` is the number of workgroups the GPU runs at once
-// (256 CUs x workgroups per CU). A split count is valid when it divides the K slabs into ranges
-// of at least 8 slabs that are a multiple of `unroll`; among those, the plan minimises (waves of
-// workgroups) x (slabs per workgroup), preferring fewer splits on a tie.
-inline bool plan_wide(int M, int N, int K, int tn, int slab_k, int unroll, int slots,
-                      WidePlan* p, int tm_small = 128, bool choose_tm = false,
-                      int small_upto = 128) {
-  if (N % tn != 0 || K % (unroll * slab_k) != 0 || M < 1) return false;
-  const int KT = K / slab_k;
-  // Plan for tile height tm; returns the estimated time in units of a third of a 128-row slab
-  // (a 256-row slab measures about 4/3 of a 128-row one, ~1 us at the benchmark shapes), plus
-  // the split-K slices: s slices of M x N 4-byte partial sums are written and read back, about
-  // one unit per 2^18 of them (2 MiB of traffic at ~5 TB/s). Without that term the plan chose
-  // 56 splits at M=384 (336 MiB of slices).
-  auto plan_tm = [&](int tm, WidePlan* q) {
-    q->tm = tm;
-    const int tiles = ((M + tm - 1) / tm) * (N / tn);
-    long best = -1;
-    for (int s = 1; s <= KT / unroll; ++s) {
-      if (KT % s != 0) continue;
-      const int spp = KT / s;
-      if (spp % unroll != 0 || (spp < 8 && s > 1)) continue;
-      if (s > 1 && (size_t)s * M * N * 4u > kWideMaxSliceBytes) continue;
-      const long waves = ((long)tiles * s + slots - 1) / slots;
-      const long slices = s > 1 ? (long)s * M * N >> 18 : 0;
-      const long cost = waves * spp * (tm == 256 ? 4 : 3) + slices;
-      if (best < 0 || cost < best) {
-        best = cost;
-        q->splits = s;
-        q->slabs_per_split = spp;
-      }
+// Estimated time of a wide launch, for comparing plans: R rounds of workgroups over the 256 CUs
+// (x `slots`), each a fixed cost (set-up and epilogue) and one slab cost per slab of the longest K
+// range; a cost per slab and workgroup in the whole launch (the workgroups of a round slow each
+// other down); and the slices of partial sums written and read (per 2^18 of them).
+struct WideCost {
+  float round, slab, load;  // of one tile height
+};
+struct WideCosts {
+  WideCost h64, h128, h256;  // by tile rows
+  float slice, split;        // split: a split at all (the second launch)
+  float uneven;              // factor of splits that are no equal multiples of four slabs
+};
+// fp16/bf16 operands: microseconds, fitted to a sweep of every tile height and split count on
+// MI355X over K x N = 4096 x {4096, 6144, 14336}, 14336 x 4096, 3584 x 18944, 18944 x 3584, 8192 x
+// {28672, 29568} and 28672 x 8192 at M = 64 .. 2048 (W4A16 group 128; FP8 weights fit the same
+// within 0.1%): the plan it picks is 0.7% from the sweep's fastest on average, where rounds times
+// slabs with the same slices lost 3.4% (4096 x 4096 M=512 42.9 -> 34.1 us, 4096 x 14336 M=320 73.5
+// -> 60.9, 4096 x 6144 M=512 50.5 -> 43.4).
+constexpr WideCosts kHalfCosts{{2.98f, 0.335f, 0.f}, {3.15f, 0.32f, 0.179f}, {4.78f, 0.437f, 0.389f},
+                               0.231f, 0.93f, 1.f};
+// bf16 weights cost the producers about 0.07 us more per slab (K=14336 N=4096 M=128 33.4 against
+// 31.4 us, M=2048 247 / 231).
+constexpr WideCosts kBf16Costs{{2.98f, 0.4f, 0.f}, {3.15f, 0.39f, 0.179f}, {4.78f, 0.5f, 0.389f},
+                               0.231f, 0.93f, 1.f};
+// int8 operands (relative): a 256-row slab measures 4/3 of a 128-row one, 2^18 slice values a third
+// of that (a fit as above gained under 0.5% over the sweep). Uneven splits are taken where they
+// save a tenth (K=18944 N=3584 M=128 94.7 -> 28.3 us), not for a few percent of the estimate
+// (K=3584 N=18944 M=256 measured 41 us with 2 splits and 43 with 3).
+constexpr WideCosts kInt8Costs{{0.f, 3.f, 0.f}, {0.f, 3.f, 0.f}, {0.f, 4.f, 0.f}, 1.f, 0.f, 1.1f};
+
+// The split of K of least estimated cost for `tiles` workgroups per split and M x N outputs
+// (*cost, when not null); 0 if K is no multiple of the unit. The splits are whole units, as even as
+// they come, of at least 8 slabs, and make at most two rounds more than an unsplit K. (Even splits
+// alone left K x N whose units have few divisors short of the 256 CUs or with a second round:
+// W4A16 K=3584 N=18944 M=64 41.2 -> 24.8 us, K=18944 N=3584 M=128 131 -> 33.)
+inline int plan_splits(long tiles, int M, int N, int KT, int unit, int slots, const WideCost& c,
+                       const WideCosts& cs, float* cost = nullptr) {
+  if (KT % unit != 0) return 0;
+  const int units = KT / unit;
+  int best_s = 0;
+  float best = 0.f;
+  for (int s = 1; s <= units; ++s) {
+    if (s > 1 && (units / s * unit < 8 || tiles * (s - 1) >= 2L * slots)) break;
+    if (s > 1 && (size_t)s * M * N * 4u > kWideMaxSliceBytes) break;
+    const float longest = (float)((units + s - 1) / s * unit);
+    const float rounds = (float)((tiles * s + slots - 1) / slots);
+    const float t = (rounds * (c.round + longest * c.slab) + (float)(tiles * KT) / 256.0f * c.load +
+                     (s > 1 ? (float)((long)s * M * N >> 18) * cs.slice + cs.split : 0.f)) *
+                    (KT % (4 * s) == 0 ? 1.f : cs.uneven);
+    if (best_s == 0 || t < best) {
+      best = t;
+      best_s = s;
     }
-    q->grid = tiles * q->splits;
-    return best;
-  };
-  if (M <= small_upto) {
-    plan_tm(tm_small, p);
-    return true;
   }
-  const long c256 = plan_tm(256, p);
-  if (choose_tm && tm_small != 256) {
-    WidePlan q;
-    if (plan_tm(tm_small, &q) < c256) *p = q;
-  }
-  return true;
+  if (cost) *cost = best;
+  return best_s;
 }
 
-// Slabs per K range must be a multiple of this for the warp-specialised kernels: their loop
-// iteration of U slabs (two quantization groups of spg slabs, a multiple of the 4-buffer ring and
-// of the prefetch ring), or U / 2 when K holds an odd number of half iterations (the loop then
-// leaves in the middle of its last iteration).
-inline int wide_k_unroll(int K, int spg, int pd) {
-  const int u = 2 * spg > pd ? 2 * spg : pd;
-  return K % (u * 32) == 0 ? u : u / 2;
+// Picks the tile height and the split count by plan_splits: tm_small rows up to 64 (small 64) or
+// 128 rows, above that the cheaper of 128 (choose) and 256 rows. `slots` is the number of
+// workgroups the GPU runs at once (256 CUs x workgroups per CU); unit_small and unit_256 are the
+// slabs per unit of K that the kernel of that tile height takes.
+// N: columns, at least tn and a multiple of 128; the last tile overlaps its neighbour where N is
+// no multiple of tn (both write the same bits).
+inline bool plan_wide(int M, int N, int K, int tn, int slab_k, int unit_small, int unit_256,
+                      int slots, const WideCosts& cs, WidePlan* p, int tm_small = 128) {
+  if (N < tn || N % 128 != 0 || M < 1 || K % slab_k != 0) return false;
+  const int KT = K / slab_k;
+  const auto tiles = [&](int tm) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+  const auto take = [&](int tm, int splits, int unit) {
+    *p = WidePlan{tm, splits, wide_split(KT, unit, splits), (int)tiles(tm) * splits};
+    return true;
+  };
+  float csmall = 0.f, c256 = 0.f;
+  const int ssmall = plan_splits(tiles(tm_small), M, N, KT, unit_small, slots,
+                                 tm_small == 64 ? cs.h64 : cs.h128, cs, &csmall);
+  if (M <= 128) return ssmall > 0 && take(tm_small, ssmall, unit_small);
+  const int s256 = plan_splits(tiles(256), M, N, KT, unit_256, slots, cs.h256, cs, &c256);
+  if (ssmall > 0 && (s256 == 0 || csmall < c256)) return take(tm_small, ssmall, unit_small);
+  return s256 > 0 && take(256, s256, unit_256);
 }
+
+// Slabs per unit of K of the kernels' loop iteration: U slabs (two quantization groups of spg
+// slabs, a multiple of the 4-buffer ring and of the prefetch ring), or, for the warp-specialised
+// kernels, which may leave their loop in the middle of its last iteration, half of it.
+constexpr int wide_iteration(int spg, int pd) { return 2 * spg > pd ? 2 * spg : pd; }
 
 // Workspace: `splits` slices of M x N 4-byte partial sums (none without split-K).
 inline size_t wide_workspace_bytes(int M, int N, int splits) {

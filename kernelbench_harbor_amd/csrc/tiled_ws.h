@@ -56,7 +56,7 @@ template <class E, int TM, int WM, int SPG, class BP, class EP, class RM = Dense
           int PS = 1, bool XD = false>
 __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
     const void* __restrict__ x, BP bp, EP ep, typename E::Part* __restrict__ ws, int M, int N,
-    int K, int splits, int slabs_per_split, RM rm) {
+    int K, WideSplit sp, RM rm) {
   constexpr int TN = BP::kTN;
   constexpr int SK = E::kSlabK;
   static_assert(!E::kStageX, "fp16/bf16 operands: x fragments straight from global memory");
@@ -79,16 +79,17 @@ __global__ __launch_bounds__(256 * (1 + PS), 1) void tiled_ws_gemm(
 
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
-  const int NB = N / TN;
+  const int splits = sp.splits;
+  const int NB = (N + TN - 1) / TN;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int nb = id % NB;
   const int rest = id / NB;
   const int MB = gridDim.x / (NB * splits);  // row blocks (tile-table entries)
   const int mb = rest % MB;
   const int split = rest / MB;
-  const int n0 = nb * TN;
-  const int kt0 = split * slabs_per_split;
-  const int KT = slabs_per_split;
+  const int n0 = min(nb * TN, N - TN);  // a last tile that N leaves short overlaps its neighbour
+  const int kt0 = sp.begin(split);
+  const int KT = sp.count(split);
   const int last = KT - 1;
   const typename RM::Tile ti = rm.tile(mb, TM);
   if (ti.rows <= 0) return;  // unused tile-table entry (uniform across the workgroup)

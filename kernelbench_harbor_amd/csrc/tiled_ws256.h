@@ -29,7 +29,7 @@ namespace kbh {
 template <class E, int SPG, class BP, class EP, int PD = 4>
 __global__ __launch_bounds__(768, 1) void tiled_ws256_gemm(
     const void* __restrict__ x, BP bp, EP ep, typename E::Part* __restrict__ ws, int M, int N,
-    int K, int splits, int slabs_per_split) {
+    int K, WideSplit sp) {
   constexpr int TM = 256, TN = 256;
   static_assert(BP::kTN == TN, "256-column weight policy");
   constexpr int SK = E::kSlabK;        // K elements per slab (64 bytes of every row)
@@ -49,17 +49,19 @@ __global__ __launch_bounds__(768, 1) void tiled_ws256_gemm(
 
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
-  const int NB = N / TN;
+  const int splits = sp.splits;
+  const int NB = (N + TN - 1) / TN;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int nb = id % NB;
   const int rest = id / NB;
   const int MB = gridDim.x / (NB * splits);
   const int mb = rest % MB;
   const int split = rest / MB;
-  const int n0 = nb * TN, m0 = mb * TM;
+  const int n0 = min(nb * TN, N - TN);  // a last tile that N leaves short overlaps its neighbour
+  const int m0 = mb * TM;
   const int rows = min(TM, M - m0);
-  const int kt0 = split * slabs_per_split;
-  const int KT = slabs_per_split;
+  const int kt0 = sp.begin(split);
+  const int KT = sp.count(split);
   const int last = KT - 1;
   constexpr bool kFast = BP::kHasFast;
   const int fr = lane & 31, fg = lane >> 5;

@@ -338,9 +338,9 @@ void dispatch_decode(const DecodePlan& p, const void* x, const int32_t* qw, cons
 // Large-M kernels
 // ======================================================================================
 // Above kWideMinM rows the wide-tile kernel (tiled_wide.h) takes over from the split-K decode
-// kernel: up to 64 rows, 64 x 256 tiles; up to 256 rows, 128 x 256 tiles with one workgroup per
-// CU (128 x 128 tiles, two per CU, up to 128 rows when N is not a multiple of 256); 256 x 256
-// tiles above unless the planner's estimate prefers 128-row tiles. The 256-column tiles run
+// kernel: up to 64 rows, 64 x 256 tiles; up to 128 rows, 128 x 256 tiles with one workgroup per
+// CU (128 x 128 tiles, two per CU, when N is 128); above, 128 x 256 or 256 x 256 tiles by the
+// planner's estimate (plan_wide). The 256-column tiles run
 // with a 4-slab prefetch ring; those of 64 and 128 rows on the warp-specialised kernel
 // (tiled_ws.h: 4 dequantizing and 4 MFMA waves per workgroup), those of 256 rows on its 12-wave
 // form (tiled_ws256.h: 4 waves stage weights and x, 8 MFMA waves; K=14336 N=4096 M=1024
@@ -357,30 +357,35 @@ struct W4Wide {
 // Prefetch depth of a wide W4 launch with tn-column tiles.
 constexpr int w4_wide_pd(int tn) { return tn == 256 ? 4 : 2; }
 
-bool plan_w4_wide(int M, int N, int K, int group, W4Wide* w) {
+bool plan_w4_wide(int M, int N, int K, int group, bool bf16, W4Wide* w) {
   if (M < kWideMinM) return false;
   w->spg = group / 32;
-  const bool small = M <= 128;
-  w->tn = (N % 256 == 0) ? 256 : 128;
-  if (!small && w->tn != 256) return false;
-  const int pd = w4_wide_pd(w->tn);
-  // The kernel's slabs per iteration; the warp-specialised kernels (256-column tiles, x under
-  // 2 GiB) also end in half an iteration: K = 29568 holds an odd number of 128-row groups (on the
-  // LDS-staged and decode kernels, which took it before, N=8192 M=64 / 256 / 1024 ran 164 / 784 /
-  // 771 us; now 62 / 161 / 518).
+  w->tn = N >= 256 ? 256 : 128;
+  if (M > 128 && w->tn != 256) return false;
+  // Slabs per unit of K: the warp-specialised kernels (256-column tiles, x under 2 GiB) take half
+  // iterations. (K = 29568 holds an odd number of 128-row groups: on the LDS-staged and decode
+  // kernels, which took it before, N=8192 M=64 / 256 / 1024 ran 164 / 784 / 771 us; now 62 / 161 /
+  // 518.)
   const bool ws = w->tn == 256 && (size_t)(M + 256) * K * 2 < ((size_t)1 << 31);
-  const int unroll = ws ? wide_k_unroll(K, w->spg, pd) : (2 * w->spg > pd ? 2 * w->spg : pd);
+  const int unit = wide_iteration(w->spg, w4_wide_pd(w->tn)) / (ws ? 2 : 1);
   // Up to 64 rows with 256-column tiles: 64 x 256 tiles (2 x 2 waves of 32 x 128); a 128-row
-  // tile would spend half its MFMAs and A loads on padding. The split count is planned for one
-  // workgroup per CU: more splits (two per CU) measured slower, their fp32 slices outweighing
-  // the extra parallelism (K=14336 N=4096 M=64: 14 splits 31.2 us, 28 splits 34.4 us).
-  // 128-row tiles (one warp-specialised workgroup per CU) up to 256 rows: fewer K splits, so
-  // fewer fp32 slices to write and sum, than 256-row tiles (K=14336 N=4096, M=256: 50.5 against
-  // 53.7 us); above, 256-row tiles on the 12-wave kernel unless the estimate prefers 128 rows
-  // (M=320 68.9 against 75.2 us, M=384 71.4 / 77.3, M=512 80.5 / 84.7).
+  // tile would spend half its MFMAs and A loads on padding there. Above 128 rows the estimate
+  // chooses between 128-row and 256-row tiles.
   const bool rows64 = M <= 64 && w->tn == 256;
-  return plan_wide(M, N, K, w->tn, 32, unroll, w->tn == 128 ? 512 : 256, &w->plan,
-                   rows64 ? 64 : 128, w->tn == 256, w->tn == 256 ? 256 : 128);
+  return plan_wide(M, N, K, w->tn, 32, unit, unit, w->tn == 128 ? 512 : 256,
+                   bf16 ? kBf16Costs : kHalfCosts, &w->plan, rows64 ? 64 : 128);
+}
+
+// Scratch of the wide kernels, for either dtype (the query does not name it): the larger plan's.
+size_t w4_wide_scratch_bytes(int M, int N, int K, int group) {
+  size_t best = 0;
+  for (bool bf16 : {false, true}) {
+    W4Wide w;
+    if (!plan_w4_wide(M, N, K, group, bf16, &w)) continue;
+    const size_t b = wide_workspace_bytes(M, N, w.plan.splits);
+    best = b > best ? b : best;
+  }
+  return best;
 }
 
 template <bool BF16, int TM, int TN, int SPG>
@@ -409,12 +414,12 @@ void launch_w4_wide(const W4Wide& w, const void* x, const int32_t* qw, const voi
       hipLaunchKernelGGL((tiled_ws_gemm<E, TM, WM, SPG, BP, EP, DenseRows, w4_wide_pd(TN), PS,
                                         TM == 128>),
                          dim3(w.plan.grid), dim3(256 * (1 + PS)), 0, st,
-                         x, bp, ep, scratch, M, N, K, w.plan.splits, w.plan.slabs_per_split,
+                         x, bp, ep, scratch, M, N, K, w.plan.sp,
                          DenseRows{M});
     else
       hipLaunchKernelGGL((tiled_ws_gemm<E, TM, WM, SPG, BP, EP, DenseRows, w4_wide_pd(TN), TM == 64 ? 2 : 1>),
                          dim3(w.plan.grid), dim3(TM == 64 ? 768 : 512), 0, st,
-                         x, bp, ep, scratch, M, N, K, w.plan.splits, w.plan.slabs_per_split,
+                         x, bp, ep, scratch, M, N, K, w.plan.sp,
                          DenseRows{M});
   } else {
     // 256 x 256 tiles: the 12-wave kernel while x is under 2 GiB (its buffer offsets are
@@ -423,15 +428,14 @@ void launch_w4_wide(const W4Wide& w, const void* x, const int32_t* qw, const voi
     if constexpr (TM == 256 && TN == 256) {
       if ((size_t)(M + TM) * K * 2 < ((size_t)1 << 31)) {
         hipLaunchKernelGGL((tiled_ws256_gemm<E, SPG, BP, EP, w4_wide_pd(TN)>), dim3(w.plan.grid),
-                           dim3(768), 0, st, x, bp, ep, scratch, M, N, K, w.plan.splits,
-                           w.plan.slabs_per_split);
+                           dim3(768), 0, st, x, bp, ep, scratch, M, N, K, w.plan.sp);
         done = true;
       }
     }
     if (!done)
       hipLaunchKernelGGL((tiled_wide_gemm<E, TM, WM, SPG, BP, EP, DenseRows, 0, w4_wide_pd(TN)>),
                          dim3(w.plan.grid), dim3(256), 0, st,
-                         x, bp, ep, scratch, M, N, K, w.plan.splits, w.plan.slabs_per_split,
+                         x, bp, ep, scratch, M, N, K, w.plan.sp,
                          DenseRows{M});
   }
   if (w.plan.splits > 1) {
@@ -473,8 +477,9 @@ void dispatch_w4_wide(const W4Wide& w, const void* x, const int32_t* qw, const v
 // kernel's split-K scratch, nothing for the LDS-staged kernel, or the decode kernel's split-K
 // workspace (the dispatch order of kbh_w4a16_gemm).
 size_t w4a16_path_bytes(int M, int N, int K, int group) {
+  const size_t wide = w4_wide_scratch_bytes(M, N, K, group);
   W4Wide w;
-  if (plan_w4_wide(M, N, K, group, &w)) return wide_workspace_bytes(M, N, w.plan.splits);
+  if (plan_w4_wide(M, N, K, group, false, &w)) return wide;
   if (M >= kTiledMinM && K % (TBK * TDEPTH) == 0) return 0;
   DecodePlan p;
   if (!plan_decode(M, N, K, group / 32, &p)) return 0;
@@ -491,9 +496,8 @@ extern "C" size_t kbh_w4a16_workspace_bytes(int M, int N, int K, int group) {
 }
 
 extern "C" size_t kbh_w4a16_scratch_bytes(int M, int N, int K, int group) {
-  kbh::W4Wide w;
-  if (M < 1 || N < 128 || K < 32 || group < 32 || !kbh::plan_w4_wide(M, N, K, group, &w)) return 0;
-  return kbh::wide_workspace_bytes(M, N, w.plan.splits);
+  if (M < 1 || N < 128 || K < 32 || group < 32) return 0;
+  return kbh::w4_wide_scratch_bytes(M, N, K, group);
 }
 
 extern "C" int kbh_w4a16_gemm(const void* x, const int32_t* qweight, const void* scales,
@@ -513,7 +517,7 @@ extern "C" int kbh_w4a16_gemm(const void* x, const int32_t* qweight, const void*
   hipStream_t st = (hipStream_t)stream;
 
   W4Wide wide;
-  if (plan_w4_wide(M, N, K, group, &wide)) {
+  if (plan_w4_wide(M, N, K, group, bf, &wide)) {
     const size_t need = wide_workspace_bytes(M, N, wide.plan.splits);
     if (need > 0 && (!scratch || scratch_bytes < need)) return KBH_ERR_WORKSPACE;
     if (need > 0 && !aligned16(scratch)) return KBH_ERR_ALIGN;

@@ -356,11 +356,16 @@ constexpr int kW8WideMinM = 33;
 // Prefetch depth 4 (four 64-deep slabs in flight) when the K slabs come in multiples of 4.
 int w8_wide_pd(int K) { return (K / 64) % 4 == 0 ? 4 : 2; }
 
+// x within the 12-wave kernel's 32-bit offsets.
+bool w8_x_staged(int M, int K) { return (size_t)(M + 256) * K < ((size_t)1 << 31); }
+
 // 128-row tiles (one workgroup per CU) up to 128 rows; above, 256-row tiles unless they would
 // leave CUs idle (plan_wide's choose_tm).
 bool plan_w8_wide(int M, int N, int K, WidePlan* p) {
-  if (M < kW8WideMinM || N % 256 != 0) return false;
-  return plan_wide(M, N, K, 256, 64, w8_wide_pd(K), 256, p, 128, true);
+  if (M < kW8WideMinM || N < 256) return false;
+  // slabs per unit of K: the 128-row kernel's iteration; half of the 12-wave kernel's
+  const int unit256 = w8_x_staged(M, K) ? 2 : w8_wide_pd(K);
+  return plan_wide(M, N, K, 256, 64, w8_wide_pd(K), unit256, 256, kInt8Costs, p);
 }
 
 template <bool OUT_I32, int TM, int PD>
@@ -371,20 +376,18 @@ void launch_w8_wide(const WidePlan& p, const void* x, const void* w, const void*
   const W8WidePolicy bp{(const int8_t*)w, N};
   const EP ep{out, (const uint16_t*)xs, (const uint16_t*)wsc, N};
   constexpr int MINB = TM == 128 ? 1 : 0;
-  // 256-row tiles with a 4-slab ring: the 12-wave kernel (tiled_ws256.h) while x is under 2 GiB.
+  // 256-row tiles: the 12-wave kernel (tiled_ws256.h) while x is under 2 GiB.
   bool done = false;
-  if constexpr (TM == 256 && PD == 4) {
-    if ((size_t)(M + TM) * K < ((size_t)1 << 31)) {
-      hipLaunchKernelGGL((tiled_ws256_gemm<WideI8, 1, W8WidePolicy, EP, PD>), dim3(p.grid),
-                         dim3(768), 0, st, x, bp, ep, scratch, M, N, K, p.splits,
-                         p.slabs_per_split);
+  if constexpr (TM == 256) {
+    if (w8_x_staged(M, K)) {
+      hipLaunchKernelGGL((tiled_ws256_gemm<WideI8, 1, W8WidePolicy, EP, 4>), dim3(p.grid),
+                         dim3(768), 0, st, x, bp, ep, scratch, M, N, K, p.sp);
       done = true;
     }
   }
   if (!done)
     hipLaunchKernelGGL((tiled_wide_gemm<WideI8, TM, 4, 1, W8WidePolicy, EP, DenseRows, MINB, PD>),
-                       dim3(p.grid), dim3(256), 0, st, x, bp, ep, scratch, M, N, K, p.splits,
-                       p.slabs_per_split, DenseRows{M});
+                       dim3(p.grid), dim3(256), 0, st, x, bp, ep, scratch, M, N, K, p.sp, DenseRows{M});
   if (p.splits > 1) {
     const size_t n4 = (size_t)M * N / 4;
     hipLaunchKernelGGL((wide_reduce_kernel<WideI8, EP>), dim3((unsigned)((n4 + 255) / 256)),

@@ -100,3 +100,34 @@ def test_w4a16_half_iteration_tails(dev, M, K, group, dtype):
     assert err.max() <= 2.0 ** -8, (int(err.argmax()), float(err.max()))
     for _ in range(3):
         assert torch.equal(y, ops.w4a16_gemm(*d))
+
+
+# M, K, N: a last column tile that overlaps its neighbour (N % 256 == 128), K ranges of uneven
+# length (units that no split count near the 256 workgroups divides), K / 64 even but not a
+# multiple of 4 (the 12-wave int8 kernel's half iterations)
+WIDE_EDGES = [(33, 1152, 384), (129, 2176, 384), (200, 18944, 640), (300, 1408, 896), (257, 128, 384),
+              (64, 9472, 1152)]
+
+
+@pytest.mark.parametrize("M,K,N", WIDE_EDGES)
+def test_w8a8_wide_edges_bit_exact(dev, M, K, N):
+    g = torch.Generator().manual_seed(M + K)
+    x = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8)
+    w = torch.randint(-128, 128, (K, N), generator=g, dtype=torch.int8)
+    acc = ops.w8a8_gemm_i32(x.to(dev), w.to(dev)).cpu().numpy()
+    # exact: |sum| <= K * 2^14 < 2^53
+    want = x.double().numpy() @ w.double().numpy()
+    assert np.array_equal(acc.astype(np.float64), want)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M,K,N", WIDE_EDGES)
+def test_wide_edges_match_oracle(dev, M, K, N, dtype):
+    x, q, s, z = inputs.w4a16(M, K, N, 128, dtype, seed=M)
+    y = ops.w4a16_gemm(*[t.to(dev) for t in (x, q, s, z)])
+    cmp = compare(y, ow.forward(x.float().numpy(), q.numpy(), s.float().numpy(), z.float().numpy()))
+    assert cmp.ok, cmp
+    x, w, s = inputs.fp8w(M, K, N, 128, dtype, seed=M)
+    y = ops.fp8w_gemm(x.to(dev), w.to(dev), s.to(dev))
+    cmp = compare(y, of.forward(x.float().numpy(), w.view(torch.uint8).numpy(), s.float().numpy()))
+    assert cmp.ok, cmp
