@@ -315,7 +315,7 @@ struct ByteWidePolicy {
 };
 
 constexpr int kByteTiledMinM = 128;
-constexpr int kByteWideMinM = 33;
+constexpr int kByteWideMinM = 17;
 constexpr int kByteWidePD = 4;
 
 struct BytePlan {
@@ -347,8 +347,9 @@ struct ByteWide {
 // ones up to 128, then 128 or 256 rows by the estimate). They replace
 // tiled_f16_gemm's 256 x 128 tiles, which split no K (K=14336 N=4096: 32 workgroups and ~300 us
 // at every M from 128 to 1024; now 30.7 / 43.0 / 75.2 / 124 us at M=128 / 256 / 512 / 1024, and
-// 342 -> 226 at 2048), and the decode kernel's 64-row blocks (M=48 42.9 -> 21.8, M=96 73.2 ->
-// 28.4). Up to 64 rows the decode kernel stays where its grid is one workgroup per CU: every
+// 342 -> 226 at 2048), and the decode kernel's 32- and 64-row blocks (M=32 26.2 -> 19.4, M=48 42.9
+// -> 21.4, M=96 73.2 -> 28.4; 8192 x 28672 M=32 85.5 -> 66.9). Up to 64 rows the decode kernel
+// stays where its grid is one workgroup per CU: every
 // weight is then in flight at once and it needs fewer split-K slices (K=N=4096 M=64 14.6 against
 // 19.8 us, K=2048 N=8192 15.5 / 19.6; with a second round of workgroups the wide tiles win:
 // K=4096 N=6144 25.6 / 18.6, K=N=3584 16.9 / 15.9).

@@ -264,7 +264,7 @@ __global__ __launch_bounds__(256) void w8a8_tiled_kernel(
 constexpr int kW8TiledMinM = 128;
 
 // ======================================================================================
-// Wide-tile kernel (M > 32)
+// Wide-tile kernel (M > 32, and from 17 rows for large weights)
 // ======================================================================================
 
 // int8 weight-slab producer for tiled_wide_gemm: 64 K rows x 256 columns per slab. Thread t owns
@@ -349,7 +349,7 @@ struct W8Out {
   }
 };
 
-constexpr int kW8WideMinM = 33;
+constexpr int kW8WideMinM = 17;
 
 // 256-row tiles at every M: the int8 slab producer holds 8 rows x 8 columns per thread, which
 // does not fit the register budget of two 128-row workgroups per CU.
@@ -363,6 +363,12 @@ bool w8_x_staged(int M, int K) { return (size_t)(M + 256) * K < ((size_t)1 << 31
 // leave CUs idle (plan_wide's choose_tm).
 bool plan_w8_wide(int M, int N, int K, WidePlan* p) {
   if (M < kW8WideMinM || N < 256) return false;
+  // 17 to 32 rows: the decode kernel streams the weights once per 16-row block and stays where its
+  // grid is at most two workgroups per CU (M=32: 4096 x 6144 14.1 against 17.2 us, 5120 x 5120 14.8 /
+  // 17.4); beyond that the wide tiles (14336 x 4096 28.3 -> 21.4, 3584 x 18944 30.3 -> 23.6, 8192 x
+  // 28672 102 -> 58).
+  W8Plan d;
+  if (M <= 32 && plan_w8_decode(M, N, K, &d) && d.ntiles * d.splits * d.mblocks <= 512) return false;
   // slabs per unit of K: the 128-row kernel's iteration; half of the 12-wave kernel's
   const int unit256 = w8_x_staged(M, K) ? 2 : w8_wide_pd(K);
   return plan_wide(M, N, K, 256, 64, w8_wide_pd(K), unit256, 256, kInt8Costs, p);

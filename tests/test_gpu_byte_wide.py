@@ -106,7 +106,7 @@ def test_w4a16_half_iteration_tails(dev, M, K, group, dtype):
 # length (units that no split count near the 256 workgroups divides), K / 64 even but not a
 # multiple of 4 (the 12-wave int8 kernel's half iterations)
 WIDE_EDGES = [(33, 1152, 384), (129, 2176, 384), (200, 18944, 640), (300, 1408, 896), (257, 128, 384),
-              (64, 9472, 1152)]
+              (64, 9472, 1152), (17, 18944, 2176), (32, 9472, 4224)]  # 17-32 rows: 64/128-row tiles
 
 
 @pytest.mark.parametrize("M,K,N", WIDE_EDGES)
