@@ -81,18 +81,33 @@ __device__ inline kbh_u32x2 byte4_dequant(uint32_t v, uint16_t s) {
   }
 }
 
-template <int SPW, bool BF16, int DEC, int MB>
+// Side work that shares a decode launch: `blocks` further workgroups along grid.x (those of
+// blockIdx.y 0) call run(index). None by default.
+struct NoSide {
+  static constexpr bool kAny = false;
+  int blocks = 0;
+  __device__ void run(int) const {}
+};
+
+template <int SPW, bool BF16, int DEC, int MB, class SIDE>
 __global__ __launch_bounds__(kSplitKMaxWaves * 64) void byte_decode_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
     const uint16_t* __restrict__ scales, uint16_t* __restrict__ y, float* __restrict__ acc,
-    int M, int N, int K, int block, int splits) {
+    int M, int N, int K, int block, int splits, SIDE side) {
   constexpr int NCS = 8;  // lane column c owns output columns n0 + 8c .. +7
   constexpr int NWG = 128;
   __shared__ SplitKSmem<NCS, float> sm;
+  const int nblocks = gridDim.x - side.blocks;  // the GEMM's
+  if constexpr (SIDE::kAny) {
+    if ((int)blockIdx.x >= nblocks) {  // uniform across the workgroup
+      if (blockIdx.y == 0) side.run(blockIdx.x - nblocks);
+      return;
+    }
+  }
   const int waves = blockDim.x >> 6;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int id = xcd_remap(blockIdx.x, nblocks);
   const int tile = id / splits, split = id - tile * splits;
   const int n0 = tile * NWG;
   const int m0 = blockIdx.y * 16 * MB;
@@ -384,12 +399,21 @@ void launch_byte_wide(const ByteWide& w, const void* x, const void* wt, const vo
                        dim3(p.grid), dim3(768), 0, st, x, bp, ep, slices, M, N, K, p.sp, DenseRows{M});
 }
 
+// The decode kernel's plan when byte_gemm_run takes that kernel for this shape.
+bool byte_takes_decode(int M, int N, int K, int block, BytePlan* p) {
+  ByteWide w;
+  if (plan_byte_wide(M, N, K, block, &w)) return false;
+  if (M >= kByteTiledMinM && K % (TBK * TDEPTH) == 0) return false;
+  return plan_byte_decode(M, N, K, p);
+}
+
 // Runs the GEMM; with `defer_sum` and a split K the slices are left in the workspace
 // (acc[splits][M][N] fp32) for the caller to sum, and *splits_out tells how many (1: y written).
-template <bool BF16, int DEC>
+// `side` runs with the decode kernel's launch; where another kernel runs, the caller launches it.
+template <bool BF16, int DEC, class SIDE = NoSide>
 int byte_gemm_run(const void* x, const void* w, const void* scales, void* y, void* workspace,
                   size_t workspace_bytes, int M, int N, int K, int block, hipStream_t st,
-                  bool defer_sum = false, int* splits_out = nullptr) {
+                  bool defer_sum = false, int* splits_out = nullptr, SIDE side = SIDE{}) {
   if (splits_out) *splits_out = 1;
   ByteWide wide;
   if (plan_byte_wide(M, N, K, block, &wide)) {
@@ -425,13 +449,13 @@ int byte_gemm_run(const void* x, const void* w, const void* scales, void* y, voi
   const size_t need = splitk_workspace_bytes(M, N, splits);
   if (need > 0 && (!workspace || workspace_bytes < need)) return KBH_ERR_WORKSPACE;
   if (need > 0 && !aligned16(workspace)) return KBH_ERR_ALIGN;
-  dim3 grid(pl.ntiles * splits, pl.mblocks);
+  dim3 grid(pl.ntiles * splits + side.blocks, pl.mblocks);
   float* acc = (float*)workspace;
 #define KBH_BYTE_DEC(SPW_, MB_)                                                                  \
   if (spw == SPW_ && pl.mb == MB_)                                                               \
-    hipLaunchKernelGGL((byte_decode_kernel<SPW_, BF16, DEC, MB_>), grid, dim3(waves * 64), 0, st, \
-                       (const uint16_t*)x, (const uint8_t*)w, (const uint16_t*)scales,           \
-                       (uint16_t*)y, acc, M, N, K, block, splits);
+    hipLaunchKernelGGL((byte_decode_kernel<SPW_, BF16, DEC, MB_, SIDE>), grid, dim3(waves * 64), \
+                       0, st, (const uint16_t*)x, (const uint8_t*)w, (const uint16_t*)scales,    \
+                       (uint16_t*)y, acc, M, N, K, block, splits, side);
   KBH_BYTE_DEC(4, 1) else KBH_BYTE_DEC(2, 1) else KBH_BYTE_DEC(1, 1)
   else KBH_BYTE_DEC(4, 2) else KBH_BYTE_DEC(2, 2) else KBH_BYTE_DEC(1, 2)
   else KBH_BYTE_DEC(2, 4) else KBH_BYTE_DEC(1, 4)

@@ -7,10 +7,12 @@
 //   base = dtype(x @ W)                                              [T, N]      (:13)
 //   lo   = dtype(x[t] @ A[id_t])                                     [T, r]      (:14-15)
 //   y    = dtype(base + dtype(lo[t] @ B[id_t]))                      [T, N]      (:16-17)
-// Three launches: the base GEMM is the byte-weight GEMM of byte_weight_gemm.h with the int8
-// decoder (its split-K slices left in the workspace, or base written into y when K is not
-// split); lora_shrink_kernel computes fp32 partial sums of x[t] @ A[id] over DS ranges of D
-// (T x DS workgroups, so that a few tokens still fill the chip); lora_expand_add_kernel sums
+// Two launches up to 32 rows, three above: the base GEMM is the byte-weight GEMM of
+// byte_weight_gemm.h with the int8 decoder (its split-K slices left in the workspace, or base
+// written into y when K is not split); LoraShrink computes fp32 partial sums of x[t] @ A[id] over
+// DS ranges of D (T x DS workgroups, so that a few tokens still fill the chip), as further
+// workgroups of the decode kernel's launch (its reads of A run beside the weight stream, and a
+// launch and its gap go) or as a kernel of its own; lora_expand_add_kernel sums
 // the DS partials in order and rounds lo to dtype, sums the GEMM's slices in split order (or
 // reads base from y) and rounds base, and writes dtype(base + dtype(lo @ B)) (four columns per
 // thread). Adapter ids index as torch does (reference.py:14-16, A[lora_ids]): an id in [-L, 0)
@@ -40,54 +42,72 @@ __device__ inline int lora_id(const int64_t* ids, int t, int L) {
 // rows per step, the four waves interleave their rows; partial sums meet by lane shuffles, then
 // across waves in LDS.
 template <bool BF16>
-__global__ __launch_bounds__(kLoraThreads) void lora_shrink_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ A, const int64_t* __restrict__ ids,
-    float* __restrict__ out, int T, int D, int r, int L, int dchunk) {
-  __shared__ float part[kLoraThreads / 64][kLoraMaxRank];
-  const int t = blockIdx.x;
-  const int d0 = blockIdx.y * dchunk, d1 = min(D, d0 + dchunk);
-  const int l = lora_id(ids, t, L);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int lpr = r >> 2;          // lanes per row of A
-  const int rps = 64 / lpr;        // rows per wave and step
-  const int c4 = lane % lpr, rr = lane / lpr;
-  const uint16_t* xr = x + (size_t)t * D;
-  const uint16_t* Al = A + (size_t)l * D * r + 4 * c4;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  const int step = 4 * rps;
-  int d = d0 + wave * rps + rr;
-  for (; d + 3 * step < d1; d += 4 * step) {  // four rows in flight
-    kbh_u32x2 a[4];
-    float xv[4];
+struct LoraShrink {
+  static constexpr bool kAny = true;
+  int blocks;  // T x ds: token fastest
+  const uint16_t* x;
+  const uint16_t* A;
+  const int64_t* ids;
+  float* out;
+  int T, D, r, L, dchunk;
+  __device__ void run(int block) const {
+    const int ds = block / T;
+    run(block - ds * T, ds, blockDim.x >> 6);
+  }
+  // Token t, range ds, by the workgroup's `waves` waves.
+  __device__ void run(int t, int ds, int waves) const {
+    __shared__ float part[kSplitKMaxWaves][kLoraMaxRank];
+    const int d0 = ds * dchunk, d1 = min(D, d0 + dchunk);
+    const int l = lora_id(ids, t, L);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lpr = r >> 2;          // lanes per row of A
+    const int rps = 64 / lpr;        // rows per wave and step
+    const int c4 = lane % lpr, rr = lane / lpr;
+    const uint16_t* xr = x + (size_t)t * D;
+    const uint16_t* Al = A + (size_t)l * D * r + 4 * c4;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    const int step = waves * rps;
+    int d = d0 + wave * rps + rr;
+    for (; d + 3 * step < d1; d += 4 * step) {  // four rows in flight
+      kbh_u32x2 a[4];
+      float xv[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      a[u] = *reinterpret_cast<const kbh_u32x2*>(Al + (size_t)(d + u * step) * r);
-      xv[u] = half_bits_to_f32<BF16>(xr[d + u * step]);
+      for (int u = 0; u < 4; ++u) {
+        a[u] = *reinterpret_cast<const kbh_u32x2*>(Al + (size_t)(d + u * step) * r);
+        xv[u] = half_bits_to_f32<BF16>(xr[d + u * step]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          acc[c] += xv[u] * half_bits_to_f32<BF16>((uint16_t)(a[u][c >> 1] >> (16 * (c & 1))));
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (; d < d1; d += step) {
+      const kbh_u32x2 a = *reinterpret_cast<const kbh_u32x2*>(Al + (size_t)d * r);
+      const float xv = half_bits_to_f32<BF16>(xr[d]);
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        acc[c] += xv[u] * half_bits_to_f32<BF16>((uint16_t)(a[u][c >> 1] >> (16 * (c & 1))));
-  }
-  for (; d < d1; d += step) {
-    const kbh_u32x2 a = *reinterpret_cast<const kbh_u32x2*>(Al + (size_t)d * r);
-    const float xv = half_bits_to_f32<BF16>(xr[d]);
+        acc[c] += xv * half_bits_to_f32<BF16>((uint16_t)(a[c >> 1] >> (16 * (c & 1))));
+    }
+    for (int o = lpr; o < 64; o <<= 1)
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      acc[c] += xv * half_bits_to_f32<BF16>((uint16_t)(a[c >> 1] >> (16 * (c & 1))));
-  }
-  for (int o = lpr; o < 64; o <<= 1)
+      for (int c = 0; c < 4; ++c) acc[c] += __shfl_xor(acc[c], o, 64);
+    if (rr == 0)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) acc[c] += __shfl_xor(acc[c], o, 64);
-  if (rr == 0)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) part[wave][4 * c4 + c] = acc[c];
-  __syncthreads();
-  if (threadIdx.x < r) {
-    const int j = threadIdx.x;
-    out[((size_t)blockIdx.y * T + t) * r + j] = part[0][j] + part[1][j] + part[2][j] + part[3][j];
+      for (int c = 0; c < 4; ++c) part[wave][4 * c4 + c] = acc[c];
+    __syncthreads();
+    for (int j = threadIdx.x; j < r; j += 64 * waves) {
+      float v = part[0][j];
+      for (int w = 1; w < waves; ++w) v += part[w][j];
+      out[((size_t)ds * T + t) * r + j] = v;
+    }
   }
+};
+
+// The shrink on its own, beside a base GEMM that is not on the decode kernel.
+template <bool BF16>
+__global__ __launch_bounds__(kLoraThreads) void lora_shrink_kernel(LoraShrink<BF16> s) {
+  s.run(blockIdx.x, blockIdx.y, kLoraThreads / 64);
 }
 
 // lo[t][j] = dtype(sum over ds in order of part[ds][t][j]);
@@ -164,7 +184,7 @@ struct LoraLayout {
 // at least four steps of 1024 / r rows (one round of four loads in flight per lane).
 LoraLayout lora_layout(int T, int D, int N, int r, int group) {
   LoraLayout L;
-  const int step = 1024 / r;
+  const int step = 1024 / r;  // rows per step of 4 waves
   const int ds_max = max(1, min(kLoraMaxSplits, D / (4 * step)));
   L.ds = max(1, min((1024 + T - 1) / T, ds_max));
   L.dchunk = (D + L.ds - 1) / L.ds;
@@ -182,11 +202,22 @@ int lora_run(const void* x, const int8_t* qweight, const void* scales, const voi
   float* part = (float*)ws;
   float* slices = (float*)((char*)ws + lay.slices);
   int splits = 1;
-  const int s = byte_gemm_run<BF16, kDecInt8>(x, qweight, scales, y, slices, ws_bytes - lay.slices,
-                                              T, N, D, group, st, true, &splits);
+  LoraShrink<BF16> shrink{T * lay.ds, (const uint16_t*)x, (const uint16_t*)A, ids, part, T, D, r, L, lay.dchunk};
+  BytePlan bp;
+  int s;
+  // Beside the decode kernel's blocks of 16 and 32 rows (T=1 19.5 -> 13.4 us, T=32 r=16 20.0 ->
+  // 17.5, r=64 25.7 -> 22.7; a launch and its gap less, host time included). Its 64-row blocks hold
+  // 218 registers, so the shrink's workgroups would queue one per CU behind them (T=64 22.1 -> 27.1).
+  if (T <= 32 && byte_takes_decode(T, N, D, group, &bp)) {
+    s = byte_gemm_run<BF16, kDecInt8>(x, qweight, scales, y, slices, ws_bytes - lay.slices, T, N, D,
+                                      group, st, true, &splits, shrink);
+  } else {
+    s = byte_gemm_run<BF16, kDecInt8>(x, qweight, scales, y, slices, ws_bytes - lay.slices, T, N, D,
+                                      group, st, true, &splits);
+    if (s == KBH_OK)
+      hipLaunchKernelGGL(lora_shrink_kernel<BF16>, dim3(T, lay.ds), dim3(kLoraThreads), 0, st, shrink);
+  }
   if (s != KBH_OK) return s;
-  hipLaunchKernelGGL(lora_shrink_kernel<BF16>, dim3(T, lay.ds), dim3(kLoraThreads), 0, st,
-                     (const uint16_t*)x, (const uint16_t*)A, ids, part, T, D, r, L, lay.dchunk);
   const dim3 grid((N / 4 + kLoraThreads - 1) / kLoraThreads, T);
   hipLaunchKernelGGL(lora_expand_add_kernel<BF16>, grid, dim3(kLoraThreads), 0, st,
                      (const float*)part, (const uint16_t*)B, ids, (const float*)slices, splits,

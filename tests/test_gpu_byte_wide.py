@@ -131,3 +131,19 @@ def test_wide_edges_match_oracle(dev, M, K, N, dtype):
     y = ops.fp8w_gemm(x.to(dev), w.to(dev), s.to(dev))
     cmp = compare(y, of.forward(x.float().numpy(), w.view(torch.uint8).numpy(), s.float().numpy()))
     assert cmp.ok, cmp
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("T,D,N,r,L", [(1, 128, 128, 4, 1), (5, 4096, 384, 64, 3), (16, 1056, 256, 32, 2),
+                                       (32, 2048, 512, 8, 4), (33, 4096, 4096, 16, 8)])
+def test_lora_shrink_beside_decode(dev, T, D, N, r, L, dtype):
+    """The shrink as further workgroups of the base GEMM's launch (up to 32 rows: one and two row
+    blocks, fewer waves than four, D ranges shorter than a step) and as its own launch (33)."""
+    x, q, s, A, B, ids = inputs.lora_qgemm(T, D, N, r, L, dtype, seed=T + D)
+    if D % 128:
+        s = (torch.randn(D // 32, N, generator=torch.Generator().manual_seed(1)) * 0.01).to(dtype)
+    ins = [x, q, s, A, B, ids]
+    y = ops.lora_qgemm(*[t.to(dev) for t in ins])
+    cmp = compare(y, ol.forward(*[t.float().numpy() if t.is_floating_point() else t.numpy() for t in ins]))
+    assert cmp.ok, cmp
+    assert torch.equal(y, ops.lora_qgemm(*[t.to(dev) for t in ins]))
