@@ -177,20 +177,29 @@ __global__ __launch_bounds__(1024) void moe_route_build_kernel(int T, int E, int
   __shared__ int cnt[kMoeMaxExperts];
   __shared__ int off[kMoeMaxExperts];
   __shared__ int tbase[kMoeMaxExperts + 1];
+  __shared__ int wsum[2][1024 / 64];
   const int S = K * T;
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < S; i += blockDim.x) mb.slot_of[i] = atomicAdd(&cnt[mb.topi[i]], 1);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int o = 0, tb = 0;
-    for (int e = 0; e < E; ++e) {
-      off[e] = o;
-      tbase[e] = tb;
-      o += cnt[e];
-      tb += (cnt[e] + bm - 1) / bm;
-    }
-    tbase[E] = tb;
+  // Exclusive prefix sums of the counts and tile counts, one expert per thread (at most 4 waves):
+  // a serial walk by one thread took ~0.1 us per expert.
+  const int e0 = threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ce = e0 < E ? cnt[e0] : 0, te = (ce + bm - 1) / bm;
+  int so = ce, stl = te;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int a = __shfl_up(so, d, 64), b = __shfl_up(stl, d, 64);
+    if (lane >= d) { so += a; stl += b; }
+  }
+  if (lane == 63) { wsum[0][wave] = so; wsum[1][wave] = stl; }
+  __syncthreads();
+  if (e0 < E) {
+    for (int w = 0; w < wave; ++w) { so += wsum[0][w]; stl += wsum[1][w]; }
+    off[e0] = so - ce;
+    tbase[e0] = stl - te;
+    if (e0 == E - 1) tbase[E] = stl;
   }
   __syncthreads();
   for (int i = threadIdx.x; i < S; i += blockDim.x) mb.perm[off[mb.topi[i]] + mb.slot_of[i]] = i;
@@ -388,6 +397,8 @@ __device__ inline float silu_fast(float v) {
 // GS > 0 (the reference qMoE op): the producer delivers unscaled integer weights and every GS
 // slabs (one quantization group) the group's fp32 sums are scaled by the group's scales
 // (fscales [E][K/(GS*TBK)][N], x.dtype) into fp32 totals, which are written as fp32 to `out`.
+// gridDim.z > 1 (GS > 0 only): K ranges of equal slabs, whole loop iterations; range z writes its
+// sums to slice z of `out` (part_stride apart).
 template <bool BF16, int BM, class BP, bool GATHER, bool GATED, bool OUT_PERM, int GS = 0>
 __global__ __launch_bounds__(256, GS > 0 ? 2 : 1) void moe_gemm_kernel(const uint16_t* __restrict__ A, int lda,
                                                        const int* __restrict__ perm,
@@ -395,7 +406,7 @@ __global__ __launch_bounds__(256, GS > 0 ? 2 : 1) void moe_gemm_kernel(const uin
                                                        BP bp2, uint16_t* __restrict__ out,
                                                        int ldo, int N, int K, int topk,
                                                        const uint16_t* __restrict__ fscales = nullptr,
-                                                       size_t fs_stride = 0) {
+                                                       size_t fs_stride = 0, size_t part_stride = 0) {
   constexpr int BN = 128;
   constexpr int WM = BM / 64, WN = 4 / WM;  // waves along M and N
   constexpr int WNT = BN / WN / 32;         // 32-column MFMA tiles per wave
@@ -412,7 +423,9 @@ __global__ __launch_bounds__(256, GS > 0 ? 2 : 1) void moe_gemm_kernel(const uin
   const int n0 = blockIdx.x * BN;
   const BP bpe = bp.at_expert(e);
   const BP bpe2 = bp2.at_expert(e);
-  const int KT = K / TBK;
+  // Slabs of this K range (gridDim.z of them with GS > 0) and its first slab.
+  const int KT = GS > 0 ? K / TBK / (int)gridDim.z : K / TBK;
+  const int kb = GS > 0 ? (int)blockIdx.z * KT : 0;
 
   const int a_ch = t & 3, a_row = t >> 2;
   const uint16_t* arow[AL];
@@ -428,7 +441,7 @@ __global__ __launch_bounds__(256, GS > 0 ? 2 : 1) void moe_gemm_kernel(const uin
     typename BP::Regs b[NB];
   };
   auto load = [&](Slab& sl, int kt) {
-    const int k0 = kt * TBK;
+    const int k0 = (kb + kt) * TBK;
 #pragma unroll
     for (int i = 0; i < AL; ++i) sl.a[i] = *reinterpret_cast<const kbh_u32x4*>(arow[i] + k0);
     bpe.load(sl.b[0], k0, n0, t);
@@ -494,7 +507,7 @@ __global__ __launch_bounds__(256, GS > 0 ? 2 : 1) void moe_gemm_kernel(const uin
   auto load_scales = [&](int g) {
 #pragma unroll
     for (int j = 0; j < WNT; ++j)
-      sc[j] = half_bits_to_f32<BF16>(fsc[(size_t)g * N + n0 + wn * 32 * WNT + j * 32 + fr]);
+      sc[j] = half_bits_to_f32<BF16>(fsc[(size_t)(kb / (FOLD ? GS : 1) + g) * N + n0 + wn * 32 * WNT + j * 32 + fr]);
   };
   if constexpr (FOLD) {
 #pragma unroll
@@ -555,7 +568,7 @@ __global__ __launch_bounds__(256, GS > 0 ? 2 : 1) void moe_gemm_kernel(const uin
           const int orow = OUT_PERM ? perm[s] : s;
           const int n = n0 + wn * 32 * WNT + j * 32 + fr;
           if constexpr (FOLD) {
-            reinterpret_cast<float*>(out)[(size_t)orow * ldo + n] = tot[i][j][v];
+            reinterpret_cast<float*>(out)[blockIdx.z * part_stride + (size_t)orow * ldo + n] = tot[i][j][v];
             continue;
           }
           float val = accv[0][i][j][v];
@@ -582,17 +595,19 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const uint16_t* __rest
 
 // y[t][n] = dtype(fp32(o[2t][n] w[2t]) + fp32(o[2t+1][n] w[2t+1])) with fp32 expert outputs
 // and fp32 routing weights: the reference's (sel * topv).sum(dim=1) (reference.py:20-21)
-// evaluated as in the grader's fp32 ground truth, rounded once. Four columns per thread.
+// evaluated as in the grader's fp32 ground truth, rounded once; o is the sum, in order, of `splits`
+// slices. Four columns per thread.
 template <bool BF16>
 __global__ __launch_bounds__(256) void moe_combine_f32_kernel(const float* __restrict__ o,
                                                               const float* __restrict__ w,
                                                               uint16_t* __restrict__ y, int T,
-                                                              int N) {
+                                                              int N, int splits) {
   const size_t i4 = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i4 >= (size_t)T * N) return;
   const size_t t = i4 / N, n = i4 - t * N;
-  const kbh_f32x4 a = *reinterpret_cast<const kbh_f32x4*>(o + (2 * t) * N + n);
-  const kbh_f32x4 b = *reinterpret_cast<const kbh_f32x4*>(o + (2 * t + 1) * N + n);
+  const size_t slice4 = (size_t)2 * T * N / 4;
+  const kbh_f32x4 a = sum_slices(reinterpret_cast<const kbh_f32x4*>(o + (2 * t) * N + n), slice4, splits);
+  const kbh_f32x4 b = sum_slices(reinterpret_cast<const kbh_f32x4*>(o + (2 * t + 1) * N + n), slice4, splits);
   const float w0 = w[2 * t], w1 = w[2 * t + 1];
   uint16_t r[4];
 #pragma unroll
@@ -836,7 +851,7 @@ struct MoeLayout {
 // when an expert averages more than 48 rows, else 64). f32_out: expert outputs o in fp32 and
 // fp32 routing weights (the reference qMoE op), else in the activation dtype.
 MoeLayout moe_layout(int T, int E, int hidden, int out_cols, int bm = 0, size_t part_bytes = 0,
-                     int topk = 2, bool f32_out = false) {
+                     int topk = 2, bool f32_out = false, int splits = 1) {
   MoeLayout L;
   const size_t S = (size_t)topk * T;
   L.topk = topk;
@@ -854,7 +869,7 @@ MoeLayout moe_layout(int T, int E, int hidden, int out_cols, int bm = 0, size_t 
   L.perm = take(S * 4);
   L.tiles = take((size_t)L.max_tiles * 3 * 4);
   L.h = take(S * hidden * 2);
-  L.o = take(S * out_cols * (f32_out ? 4 : 2));
+  L.o = take(S * out_cols * (f32_out ? (size_t)4 * splits : 2));
   L.part = take(part_bytes);
   L.topw32 = f32_out ? take(S * 4) : 0;
   L.total = o;
@@ -896,32 +911,56 @@ void launch_route_topk(const void* logits, int logits_dtype, int T, int E, int w
 template <bool BF16, class BP, bool GATHER, bool GATED, bool OUT_PERM, int GS = 0>
 void launch_moe_gemm(const MoeLayout& L, const void* A, int lda, const MoeBuffers& mb, const BP& bp,
                      const BP& bp2, void* out, int ldo, int N, int K, hipStream_t st,
-                     const uint16_t* fscales = nullptr, size_t fs_stride = 0) {
-  const dim3 grid(N / 128, L.max_tiles);
+                     const uint16_t* fscales = nullptr, size_t fs_stride = 0, int splits = 1,
+                     size_t part_stride = 0) {
+  const dim3 grid(N / 128, L.max_tiles, splits);
   if (L.bm == 64)
     hipLaunchKernelGGL((moe_gemm_kernel<BF16, 64, BP, GATHER, GATED, OUT_PERM, GS>), grid, dim3(256),
                        0, st, (const uint16_t*)A, lda, mb.perm, mb.tiles, bp, bp2, (uint16_t*)out,
-                       ldo, N, K, L.topk, fscales, fs_stride);
+                       ldo, N, K, L.topk, fscales, fs_stride, part_stride);
   else
     hipLaunchKernelGGL((moe_gemm_kernel<BF16, 128, BP, GATHER, GATED, OUT_PERM, GS>), grid,
                        dim3(256), 0, st, (const uint16_t*)A, lda, mb.perm, mb.tiles, bp, bp2,
-                       (uint16_t*)out, ldo, N, K, L.topk, fscales, fs_stride);
+                       (uint16_t*)out, ldo, N, K, L.topk, fscales, fs_stride, part_stride);
+}
+
+// Slabs per unit of K of the reference qMoE op: its largest quantization group (the workspace query
+// does not name the group).
+constexpr int kQMoeUnit = 8;
+
+// K splits of the reference qMoE op's grouped GEMM at small batches, where the experts a batch can
+// reach times the column tiles leave CUs idle and a workgroup walks all of K alone at ~0.5 us per
+// slab: the smallest split of K's units that makes 384 workgroups (fp32 slices, at most 16 MiB,
+// summed by the combine). D=2048 N=1408 E=64 T=1 / 8 / 16 32.6 / 34.7 / 39.3 -> 22.4 / 27.4 / 34.8 us,
+// D=4096 N=14336 E=8 T=1 49.4 -> 44.0. The fp16/bf16 MoE, whose combine must round every expert
+// output, did not gain (D=4096 H=14336 T=1 53 -> 74 us).
+int moe_splits(int T, int E, int D, int N) {
+  const int slabs = D / TBK;
+  if (slabs <= 0 || slabs % kQMoeUnit != 0) return 1;
+  const long S = 2L * T;
+  const long wgs = (S < E ? S : E) * (N / 128);
+  int best = 1;
+  for (int s = 1; s <= slabs / kQMoeUnit && wgs * best < 384; ++s)
+    if ((slabs / kQMoeUnit) % s == 0 && (size_t)s * S * N * 4 <= ((size_t)16 << 20)) best = s;
+  return best;
 }
 
 // The reference qMoE op's expert GEMM: exact integer weights, the scales folded per group
 // (GS = group / TBK slabs), fp32 outputs per (token, k) row.
 template <bool BF16>
 void launch_qmoe_gemm(const MoeLayout& L, const void* x, const MoeBuffers& mb, const int8_t* q,
-                      const void* scales, void* o, int D, int N, int group, hipStream_t st) {
+                      const void* scales, void* o, int T, int D, int N, int group, int splits,
+                      hipStream_t st) {
+  const size_t ps = (size_t)2 * T * N;
   const I8QSlabPolicy<BF16> bp{q, N, (size_t)D * N};
   const uint16_t* sc = (const uint16_t*)scales;
   const size_t ss = (size_t)(D / group) * N;
   using BP = I8QSlabPolicy<BF16>;
   switch (group / TBK) {
-    case 1: return launch_moe_gemm<BF16, BP, true, false, true, 1>(L, x, D, mb, bp, bp, o, N, N, D, st, sc, ss);
-    case 2: return launch_moe_gemm<BF16, BP, true, false, true, 2>(L, x, D, mb, bp, bp, o, N, N, D, st, sc, ss);
-    case 4: return launch_moe_gemm<BF16, BP, true, false, true, 4>(L, x, D, mb, bp, bp, o, N, N, D, st, sc, ss);
-    default: return launch_moe_gemm<BF16, BP, true, false, true, 8>(L, x, D, mb, bp, bp, o, N, N, D, st, sc, ss);
+    case 1: return launch_moe_gemm<BF16, BP, true, false, true, 1>(L, x, D, mb, bp, bp, o, N, N, D, st, sc, ss, splits, ps);
+    case 2: return launch_moe_gemm<BF16, BP, true, false, true, 2>(L, x, D, mb, bp, bp, o, N, N, D, st, sc, ss, splits, ps);
+    case 4: return launch_moe_gemm<BF16, BP, true, false, true, 4>(L, x, D, mb, bp, bp, o, N, N, D, st, sc, ss, splits, ps);
+    default: return launch_moe_gemm<BF16, BP, true, false, true, 8>(L, x, D, mb, bp, bp, o, N, N, D, st, sc, ss, splits, ps);
   }
 }
 
@@ -1083,9 +1122,8 @@ bool moe_shape_ok(int T, int E, int K, int N, int group) {
 }  // namespace kbh
 
 extern "C" size_t kbh_qmoe_workspace_bytes(int T, int D, int N, int E) {
-  (void)D;
   if (T <= 0 || E <= 0) return 0;
-  return kbh::moe_layout(T, E, 0, N, 0, 0, 2, true).total;
+  return kbh::moe_layout(T, E, 0, N, 0, 0, 2, true, kbh::moe_splits(T, E, D, N)).total;
 }
 
 extern "C" int kbh_moe_route_top2(const void* router_logits, int logits_dtype, int32_t* topi,
@@ -1116,7 +1154,8 @@ extern "C" int kbh_qmoe(const void* x, const int8_t* qweight, const void* scales
   if (logits_dtype < 0 || logits_dtype > 2) return KBH_ERR_DTYPE;
   if (!moe_shape_ok(T, E, D, N, group)) return KBH_ERR_SHAPE;
   if (!aligned16(x) || !aligned16(qweight) || !aligned16(scales) || !aligned16(y)) return KBH_ERR_ALIGN;
-  const MoeLayout L = moe_layout(T, E, 0, N, 0, 0, 2, true);
+  const int splits = moe_splits(T, E, D, N);
+  const MoeLayout L = moe_layout(T, E, 0, N, 0, 0, 2, true, splits);
   if (workspace_bytes < L.total) return KBH_ERR_WORKSPACE;
   const MoeBuffers mb = moe_buffers(workspace, L);
   hipStream_t st = (hipStream_t)stream;
@@ -1126,13 +1165,13 @@ extern "C" int kbh_qmoe(const void* x, const int8_t* qweight, const void* scales
   const size_t n = (size_t)T * N;
   const dim3 cgrid((unsigned)((n / 4 + 255) / 256));
   if (bf) {
-    launch_qmoe_gemm<true>(L, x, mb, qweight, scales, o, D, N, group, st);
+    launch_qmoe_gemm<true>(L, x, mb, qweight, scales, o, T, D, N, group, splits, st);
     hipLaunchKernelGGL(moe_combine_f32_kernel<true>, cgrid, dim3(256), 0, st, (const float*)o,
-                       mb.topw32, (uint16_t*)y, T, N);
+                       mb.topw32, (uint16_t*)y, T, N, splits);
   } else {
-    launch_qmoe_gemm<false>(L, x, mb, qweight, scales, o, D, N, group, st);
+    launch_qmoe_gemm<false>(L, x, mb, qweight, scales, o, T, D, N, group, splits, st);
     hipLaunchKernelGGL(moe_combine_f32_kernel<false>, cgrid, dim3(256), 0, st, (const float*)o,
-                       mb.topw32, (uint16_t*)y, T, N);
+                       mb.topw32, (uint16_t*)y, T, N, splits);
   }
   return launch_status();
 }
@@ -1223,8 +1262,8 @@ extern "C" int kbh_qmoe_ffn(const void* x, const void* router_logits, int logits
 }
 
 extern "C" size_t kbh_moe_workspace_bytes(int T, int D, int H, int E, int topk) {
-  (void)D;
   if (T <= 0 || E <= 0 || topk < 1 || topk > kbh::kMoeMaxTopk) return 0;
+  (void)D;
   return kbh::moe_layout(T, E, 0, H, 0, 0, topk).total;
 }
 

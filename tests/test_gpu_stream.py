@@ -90,3 +90,17 @@ def test_w4a16_stream(dev, K, N, group, splits, M, dtype):
     assert _lib.load().kbh_w4a16_gemm_noalloc(*[t.data_ptr() for t in d], y2.data_ptr(), M, N, K,
                                               group, code, st) == 0
     assert torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("T,D,N,E,group", [(1, 2048, 128, 60, 128), (3, 768, 256, 200, 256), (9, 1280, 128, 65, 64),
+                                           (2, 256, 128, 4, 32), (5, 4096, 384, 129, 128)])
+def test_qmoe_split_k(dev, T, D, N, E, group, dtype):
+    """The reference qMoE op at small batches (K split over workgroups, slices summed by the
+    combine) and route tables of one to four waves of experts."""
+    ins = inputs.qmoe(T, D, E, N, dtype, seed=T + E, group=group)
+    y = ops.qmoe(*[t.to(dev) for t in ins])
+    cmp = compare(y, oq.qmoe_forward(*_np(ins)))
+    assert cmp.ok, cmp
+    ops.scratches.get(0, dev).fill_(255)
+    assert torch.equal(y, ops.qmoe(*[t.to(dev) for t in ins]))
