@@ -8,12 +8,14 @@
 // the product with the scale is rounded once (v_pk_mul_f16, or an exact fp32 product rounded to
 // bf16).
 //
-// Both kernels transpose 4x4 byte blocks in registers so that each lane holds consecutive k of
-// one column, as the MFMA B operand needs.
+// The decode and LDS-staged kernels transpose 4x4 byte blocks in registers so that each lane holds
+// consecutive k of one column, as the MFMA B operand needs; the others pair rows by v_perm_b32.
 //  * byte_decode_kernel (small M): a wave owns 128 columns (8 per lane, dwordx2 loads) and SPW
 //    steps of 32 k for MB blocks of 16 rows (each dequantised weight fragment feeds MB MFMAs, so
 //    the weights are streamed once per 16 MB rows); all loads up front; 16x16x32 fp16/bf16
 //    MFMAs; split-K epilogue of splitk.h, once per row block.
+//  * byte_stream_kernel (e4m3, up to 16 rows, layers whose decode grid is over two workgroups per CU):
+//    the same tile, K walked in a continuous stream.
 //  * larger M: the warp-specialised wide tiles (tiled_ws.h, tiled_ws256.h) with ByteWidePolicy, or
 //    tiled_f16_gemm (tiled_f16.h) with ByteSlabPolicy for shapes they do not cover.
 #pragma once
@@ -245,6 +247,106 @@ __device__ inline uint32_t byte_pair_dequant(uint32_t a, uint32_t b, uint16_t s)
   }
 }
 
+// Streaming form for up to 16 rows (e4m3 weights), where the decode kernel's grid does not fit the
+// GPU at once: its workgroups fill the memory pipeline, drain it, and leave a last round that is
+// mostly empty. Here a wave walks its K range in 64-row chunks with two chunk buffers in registers
+// (chunk i + 1's loads go out before chunk i's MFMAs, 8 to 16 KB per wave in flight), 4 waves and
+// 33 KB of LDS per workgroup, so that all the workgroups of the plan are resident together and
+// stream until their K range ends, with fewer slices. Two-row pairs come from v_perm_b32 as in
+// ByteWidePolicy. HBM bound; e4m3 x fp16, back to back on rotating weights: 3584 x 18944 M=1 / 16 18.3 /
+// 21.2 -> 16.9 / 20.3 us, 18944 x 3584 19.9 / 24.6 -> 17.9 / 19.7, 28672 x 8192 M=16 59.0 -> 48.0
+// (235 MB at 4.9 TB/s).
+constexpr int kByteStreamWaves = 4;
+constexpr int kByteStreamChunk = 64;  // K rows (two MFMA steps)
+
+template <bool BF16>
+__global__ __launch_bounds__(64 * kByteStreamWaves, 3) void byte_stream_kernel(
+    const uint16_t* __restrict__ x, const uint8_t* __restrict__ w,
+    const uint16_t* __restrict__ scales, uint16_t* __restrict__ y, float* __restrict__ acc,
+    int M, int N, int K, int block, int splits) {
+  constexpr int NCS = 8;  // lane column c owns output columns n0 + 8c .. +7
+  __shared__ SplitKSmem<NCS, float, kByteStreamWaves> sm;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int c = lane & 15, g = lane >> 4;
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = id / splits, split = id - tile * splits;
+  const int n0 = tile * 128;
+  // This wave's chunks: consecutive parts of the split's, uneven where they must be.
+  const int chunks = K / kByteStreamChunk;
+  const int sb = (int)((long)chunks * split / splits), se = (int)((long)chunks * (split + 1) / splits);
+  const int cb = sb + (se - sb) * wave / kByteStreamWaves;
+  const int ce = sb + (se - sb) * (wave + 1) / kByteStreamWaves;
+
+  const __amdgpu_buffer_rsrc_t wres = make_rsrc(w, (size_t)K * N);
+  const uint32_t wlane = (uint32_t)(8 * g * N + n0 + 8 * c);
+  // Rows past M re-read row 0: an output row depends on its own x row alone, and theirs are
+  // never stored.
+  const uint16_t* xp = x + (size_t)(c < M ? c : 0) * K + 8 * g;
+  const uint16_t* sp = scales + n0 + 8 * c;
+  struct Chunk {
+    kbh_u32x2 w[2][8];
+    kbh_u32x4 x[2], s[2];
+  };
+  auto load = [&](Chunk& ch, int i) {  // past the range: its last chunk again (never used)
+    const int k0 = min(i, ce - 1) * kByteStreamChunk;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        ch.w[u][r] = __builtin_bit_cast(
+            kbh_u32x2, __builtin_amdgcn_raw_buffer_load_b64(wres, wlane, (k0 + 32 * u + r) * N, kBufNT));
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      ch.x[u] = *reinterpret_cast<const kbh_u32x4*>(xp + k0 + 32 * u);
+      ch.s[u] = *reinterpret_cast<const kbh_u32x4*>(sp + (size_t)((k0 + 32 * u) / block) * N);
+    }
+  };
+  kbh_f32x4 part[NCS];
+#pragma unroll
+  for (int cs = 0; cs < NCS; ++cs) part[cs] = kbh_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](const Chunk& ch) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {  // dword h: columns 4h .. 4h+3
+        kbh_u32x4 b[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {  // rows 2p, 2p + 1
+          const uint32_t a0 = ch.w[u][2 * p][h], a1 = ch.w[u][2 * p + 1][h];
+          b[0][p] = byte_pair_dequant<BF16, kDecE4M3, 0>(a0, a1, half_of(ch.s[u], 4 * h + 0));
+          b[1][p] = byte_pair_dequant<BF16, kDecE4M3, 1>(a0, a1, half_of(ch.s[u], 4 * h + 1));
+          b[2][p] = byte_pair_dequant<BF16, kDecE4M3, 2>(a0, a1, half_of(ch.s[u], 4 * h + 2));
+          b[3][p] = byte_pair_dequant<BF16, kDecE4M3, 3>(a0, a1, half_of(ch.s[u], 4 * h + 3));
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[4 * h + j] = mfma16x16x32<BF16>(ch.x[u], b[j], part[4 * h + j]);
+      }
+  };
+  if (cb < ce) {
+    Chunk buf[2];
+    load(buf[0], cb);
+    int i = cb;
+    for (; i + 2 <= ce; i += 2) {
+      load(buf[1], i + 1);
+      __builtin_amdgcn_sched_barrier(0);  // the next chunk's loads go out before this one's math
+      compute(buf[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      load(buf[0], i + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(buf[1]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (i < ce) compute(buf[0]);
+  }
+  splitk_wave_sum<NCS, float, kbh_f32x4>(part, sm, min(M, 16), [&](int r, int n, float v) {
+    if (splits == 1)
+      y[(size_t)r * N + n0 + n] = f32_to_half_bits<BF16>(v);
+    else
+      acc[((size_t)split * M + r) * N + n0 + n] = v;
+  });
+}
+
 // Weight producer of the warp-specialised kernels (32 rows x 256 columns per slab). Thread t owns
 // rows 4rb .. 4rb+3 of columns 8cb .. 8cb+7 (the F16WidePolicy / W8WidePolicy thread map, whose
 // LDS writes are bank-conflict free): four 8-byte loads, and per column its 4 consecutive K values
@@ -353,6 +455,35 @@ bool plan_byte_decode(int M, int N, int K, BytePlan* p) {
   return p->waves > 0;
 }
 
+// K splits of the streaming kernel, or 0 where the decode kernel stays: it does while its grid is
+// resident at once (two workgroups per CU), and where its estimated time is lower. Both estimates
+// (us) are the weights at the rate of a full stream plus the fp32 slices written and read. The
+// decode kernel loses ~5 us to a nearly empty last round while it has few rounds (3584 x 18944:
+// 592 workgroups, 512 at once). The streaming kernel takes as long as its busiest CU, counted as 2.5
+// workgroups where a second one per CU is not there for all (the dispatcher puts three on some:
+// 4096 x 14336 448 / 672 workgroups 21.8 / 18.9 us). The 5% covers the estimates' own error: 8192 x 28672,
+// where 224 column tiles leave CUs idle, stays (M=1 43.4 us, streaming 47.3 at best; M=16 54.3 /
+// 52.1-55.6).
+inline int plan_byte_stream(int M, int N, int K, const BytePlan& d) {
+  const long grid = (long)d.ntiles * d.splits;
+  if (M > 16 || grid <= 512 || K % kByteStreamChunk != 0 || (size_t)K * N >= ((size_t)1 << 31)) return 0;
+  const float slice = (float)M * N * 8.0f / 2.9e6f;
+  float best = 0.95f * ((float)K * N / 5.4e6f + (d.splits > 1 ? d.splits * slice : 0.f) + (grid <= 1280 ? 5.f : 0.f));
+  int best_s = 0;
+  // at most the three workgroups a CU holds, at least two chunks per wave of a split K
+  for (int s = 1; (long)d.ntiles * s <= 768; ++s) {
+    if (s > 1 && K / kByteStreamChunk < 2 * kByteStreamWaves * s) break;
+    const long wgs = (long)d.ntiles * s;
+    const float per_cu = wgs <= 256 ? 1.f : (wgs < 512 ? 2.5f : (float)((wgs + 255) / 256));
+    const float t = per_cu * ((float)K / s) * (128 * 256 / 5.1e6f) + (s > 1 ? s * slice : 0.f);
+    if (t < best) {
+      best = t;
+      best_s = s;
+    }
+  }
+  return best_s;
+}
+
 struct ByteWide {
   WidePlan plan;
   int spg;
@@ -445,6 +576,21 @@ int byte_gemm_run(const void* x, const void* w, const void* scales, void* y, voi
   }
   BytePlan pl;
   if (!plan_byte_decode(M, N, K, &pl)) return KBH_ERR_SHAPE;
+  if constexpr (DEC == kDecE4M3 && !SIDE::kAny) {
+    if (const int s = plan_byte_stream(M, N, K, pl)) {
+      const size_t need = splitk_workspace_bytes(M, N, s);
+      if (need > 0 && (!workspace || workspace_bytes < need)) return KBH_ERR_WORKSPACE;
+      if (need > 0 && !aligned16(workspace)) return KBH_ERR_ALIGN;
+      hipLaunchKernelGGL((byte_stream_kernel<BF16>), dim3(pl.ntiles * s), dim3(64 * kByteStreamWaves),
+                         0, st, (const uint16_t*)x, (const uint8_t*)w, (const uint16_t*)scales,
+                         (uint16_t*)y, (float*)workspace, M, N, K, block, s);
+      if (splits_out) *splits_out = s;
+      if (s > 1 && !defer_sum)
+        launch_splitk_sum(reinterpret_cast<const kbh_f32x4*>(workspace), HalfOut<BF16>{(uint16_t*)y, N},
+                          M, N, pl.ntiles, 128, s, st);
+      return launch_status();
+    }
+  }
   const int spw = pl.spw, waves = pl.waves, splits = pl.splits;
   const size_t need = splitk_workspace_bytes(M, N, splits);
   if (need > 0 && (!workspace || workspace_bytes < need)) return KBH_ERR_WORKSPACE;
@@ -475,7 +621,9 @@ size_t byte_gemm_workspace_bytes(int M, int N, int K, int block) {
   if (M >= kByteTiledMinM && K % (TBK * TDEPTH) == 0) return 0;  // tiled path: no split
   BytePlan p;
   if (!plan_byte_decode(M, N, K, &p)) return 0;
-  return splitk_workspace_bytes(M, N, p.splits);
+  const int s = plan_byte_stream(M, N, K, p);  // FP8 weights; the int8 base takes the decode plan
+  const size_t dec = splitk_workspace_bytes(M, N, p.splits), str = splitk_workspace_bytes(M, N, s);
+  return dec > str ? dec : str;
 }
 
 }  // namespace

@@ -1,5 +1,5 @@
-"""The streaming W4A16 kernel (up to 16 rows per tile): the SiLU FFN at decode batches, against the
-float64 oracle. Edges: one token, an expert of exactly 16 and of 17 rows (a second tile), experts
+"""The streaming kernels (up to 16 rows per tile): W4A16 (the SiLU FFN at decode batches, dense rows)
+and FP8 weights, against the float64 oracle. Edges: one token, an expert of exactly 16 and of 17 rows (a second tile), experts
 without rows, K ranges with fewer units than waves and uneven over waves and splits, every group
 size."""
 import numpy as np
@@ -8,6 +8,7 @@ import torch
 
 from kernelbench_harbor_amd import _lib, inputs, ops
 from kernelbench_harbor_amd.harness import compare
+from oracle import fp8w as of
 from oracle import qmoe as oq
 from oracle import w4a16 as ow
 
@@ -104,3 +105,40 @@ def test_qmoe_split_k(dev, T, D, N, E, group, dtype):
     assert cmp.ok, cmp
     ops.scratches.get(0, dev).fill_(255)
     assert torch.equal(y, ops.qmoe(*[t.to(dev) for t in ins]))
+
+
+# K, N, block: layers whose decode grid is over 512 workgroups. Uneven chunks over splits and waves,
+# unsplit K, an odd chunk count, fewer chunks than waves.
+FP8W = [(3584, 18944, 128), (9472, 7168, 32), (320, 65664, 64), (192, 65664, 32), (2304, 31872, 256)]
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M", [1, 7, 16])
+@pytest.mark.parametrize("K,N,block", FP8W)
+def test_fp8w_stream(dev, K, N, block, M, dtype):
+    print(f"[fp8w stream] M={M} K={K} N={N} B={block} {dtype}", flush=True)
+    x, w, s = inputs.fp8w(M, K, N, block, dtype, seed=M + K)
+    d = [t.to(dev) for t in (x, w, s)]
+    y = ops.fp8w_gemm(*d)
+    codes = w.view(torch.uint8).numpy()
+    for c in (slice(0, 128), slice(N - 128, N)):
+        cmp = compare(y[:, c], of.forward(x.float().numpy(), codes[:, c], s[:, c].float().numpy()))
+        assert cmp.ok, cmp
+    ops.workspaces.get(0, dev).fill_(255)   # no content requirement on the workspace
+    assert torch.equal(y, ops.fp8w_gemm(*d))
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_fp8w_stream_dequant_bit_exact(dev, dtype):
+    """One-hot x: each output row is a dequantized weight row, rounded once, bit for bit."""
+    K, N, block = 2304, 31872, 128
+    g = torch.Generator().manual_seed(3)
+    codes = torch.randint(0, 256, (K, N), generator=g, dtype=torch.uint8)
+    codes[(codes & 0x7F) == 0x7F] = 0x38        # drop the two NaN codes
+    s = (torch.rand(K // block, N, generator=g) * 4 + 0.01).to(torch.float16)
+    ks = torch.randperm(K, generator=g)[:16]
+    x = torch.zeros(16, K, dtype=dtype)
+    x[torch.arange(16), ks] = 1.0
+    y = ops.fp8w_gemm(x.to(dev), codes.view(torch.float8_e4m3fn).to(dev), s.to(dev))
+    W = of.dequant(codes[ks].numpy(), s[ks // block].float().numpy(), "f16" if dtype == F16 else "bf16")
+    assert np.array_equal(y.float().cpu().numpy(), W)
