@@ -99,7 +99,7 @@ __global__ __launch_bounds__(kSplitKMaxWaves * 64) void byte_decode_kernel(
   constexpr int NCS = 8;  // lane column c owns output columns n0 + 8c .. +7
   constexpr int NWG = 128;
   __shared__ SplitKSmem<NCS, float> sm;
-  const int nblocks = gridDim.x - side.blocks;  // the GEMM's
+  const int nblocks = SIDE::kAny ? gridDim.x - side.blocks : gridDim.x;  // the GEMM's
   if constexpr (SIDE::kAny) {
     if ((int)blockIdx.x >= nblocks) {  // uniform across the workgroup
       if (blockIdx.y == 0) side.run(blockIdx.x - nblocks);
