@@ -349,7 +349,8 @@ def moe_route_top2(router_logits: torch.Tensor, dtype: torch.dtype = torch.float
     st = _stream_ptr(idx)
     lib = _lib.load()
     ws, ws_n = scratches.take(_bytes(lib, "kbh_qmoe_workspace_bytes", T, 0, 0, E), dev, idx, st)
-    st = lib.kbh_moe_route_top2(router_logits.contiguous().data_ptr(), _LOGIT_CODE[router_logits.dtype],
+    lg = router_logits.contiguous()
+    st = lib.kbh_moe_route_top2(lg.data_ptr(), _LOGIT_CODE[lg.dtype],
                                 topi.data_ptr(), topw.data_ptr(), ws, ws_n, T, E,
                                 _W_CODE[dtype], st)
     _lib.check(st, "kbh_moe_route_top2")
@@ -382,9 +383,11 @@ def qmoe(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     st = _stream_ptr(idx)
     lib = _lib.load()
     ws, ws_n = scratches.take(_bytes(lib, "kbh_qmoe_workspace_bytes", T, D, N, E), dev, idx, st)
-    st = lib.kbh_qmoe(x.contiguous().data_ptr(), qweight.contiguous().data_ptr(),
-                      scales.contiguous().data_ptr(), router_logits.contiguous().data_ptr(),
-                      _LOGIT_CODE[router_logits.dtype], y.data_ptr(), ws, ws_n,
+    # the copies stay alive until the call: a freed one's memory could go to the next copy, or to
+    # another thread of this stream, before the kernels are queued
+    ts = [t_.contiguous() for t_ in (x, qweight, scales, router_logits)]
+    st = lib.kbh_qmoe(*[t_.data_ptr() for t_ in ts], _LOGIT_CODE[router_logits.dtype],
+                      y.data_ptr(), ws, ws_n,
                       T, D, N, E, group, _DT_CODE[x.dtype], st)
     _lib.check(st, "kbh_qmoe")
     return y
@@ -427,8 +430,9 @@ def qmoe_ffn(x, router_logits, gate_qweight, gate_scales, gate_zeros, up_qweight
     lib = _lib.load()
     ws, ws_n = scratches.take(_bytes(lib, "kbh_qmoe_ffn_workspace_bytes", T, D, F, E), dev, idx, st)
     ts = [t_.contiguous() for t_ in ts]
-    st = lib.kbh_qmoe_ffn(ts[0].data_ptr(), router_logits.contiguous().data_ptr(),
-                          _LOGIT_CODE[router_logits.dtype], *[t_.data_ptr() for t_ in ts[1:]],
+    lg = router_logits.contiguous()
+    st = lib.kbh_qmoe_ffn(ts[0].data_ptr(), lg.data_ptr(), _LOGIT_CODE[lg.dtype],
+                          *[t_.data_ptr() for t_ in ts[1:]],
                           y.data_ptr(), ws, ws_n, T, D, F, E, group,
                           _DT_CODE[x.dtype], st)
     _lib.check(st, "kbh_qmoe_ffn")
@@ -496,8 +500,8 @@ def moe_route_topk(router_logits: torch.Tensor, topk: int, dtype: torch.dtype = 
     st = _stream_ptr(idx)
     lib = _lib.load()
     ws, ws_n = scratches.take(_bytes(lib, "kbh_moe_workspace_bytes", T, 0, 0, E, topk), dev, idx, st)
-    st = lib.kbh_moe_route_topk(router_logits.contiguous().data_ptr(),
-                                _LOGIT_CODE[router_logits.dtype], topi.data_ptr(), topw.data_ptr(),
+    lg = router_logits.contiguous()
+    st = lib.kbh_moe_route_topk(lg.data_ptr(), _LOGIT_CODE[lg.dtype], topi.data_ptr(), topw.data_ptr(),
                                 ws, ws_n, T, E, topk, _W_CODE[dtype],
                                 st)
     _lib.check(st, "kbh_moe_route_topk")
@@ -530,9 +534,9 @@ def moe(x: torch.Tensor, w: torch.Tensor, router_logits: torch.Tensor, topk: int
     st = _stream_ptr(idx)
     lib = _lib.load()
     ws, ws_n = scratches.take(_bytes(lib, "kbh_moe_workspace_bytes", T, D, H, E, topk), dev, idx, st)
-    xc, wc = x.contiguous(), w.contiguous()
-    st = lib.kbh_moe(xc.data_ptr(), wc.data_ptr(), router_logits.contiguous().data_ptr(),
-                     _LOGIT_CODE[router_logits.dtype], y.data_ptr(), ws, ws_n,
+    xc, wc, lg = x.contiguous(), w.contiguous(), router_logits.contiguous()
+    st = lib.kbh_moe(xc.data_ptr(), wc.data_ptr(), lg.data_ptr(), _LOGIT_CODE[lg.dtype],
+                     y.data_ptr(), ws, ws_n,
                      T, D, H, E, topk, _DT_CODE[x.dtype], st)
     _lib.check(st, "kbh_moe")
     return y
