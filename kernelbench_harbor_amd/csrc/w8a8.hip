@@ -374,6 +374,10 @@ bool plan_w8_wide(int M, int N, int K, WidePlan* p) {
   return plan_wide(M, N, K, 256, 64, w8_wide_pd(K), unit256, 256, kInt8Costs, p);
 }
 
+// Calls that a workspace alone has always been enough for (the decode kernel's, which ran them all
+// once): they still take that kernel where no scratch is given.
+bool w8_decode_is_enough(int M, int N) { return M <= 32 || (M < kW8TiledMinM && N % 256 != 0); }
+
 template <bool OUT_I32, int TM, int PD>
 void launch_w8_wide(const WidePlan& p, const void* x, const void* w, const void* xs,
                     const void* wsc, void* out, int* scratch, int M, int N, int K,
@@ -406,7 +410,14 @@ int w8a8_run(const void* x, const void* w, const void* xs, const void* wsc, void
              void* workspace, size_t workspace_bytes, void* scratch, size_t scratch_bytes, int M,
              int N, int K, hipStream_t st) {
   WidePlan wp;
-  if (plan_w8_wide(M, N, K, &wp)) {
+  W8Plan p;
+  bool wide = plan_w8_wide(M, N, K, &wp);
+  if (wide && w8_decode_is_enough(M, N) && plan_w8_decode(M, N, K, &p)) {
+    const size_t sc = wide_workspace_bytes(M, N, wp.splits), need = splitk_workspace_bytes(M, N, p.splits);
+    const bool scratch_ok = sc == 0 || (scratch && scratch_bytes >= sc);
+    if (!scratch_ok && (need == 0 || (workspace && workspace_bytes >= need))) wide = false;
+  }
+  if (wide) {
     const size_t need = wide_workspace_bytes(M, N, wp.splits);
     if (need > 0 && (!scratch || scratch_bytes < need)) return KBH_ERR_WORKSPACE;
     if (need > 0 && !aligned16(scratch)) return KBH_ERR_ALIGN;
@@ -427,7 +438,6 @@ int w8a8_run(const void* x, const void* w, const void* xs, const void* wsc, void
                        (const uint16_t*)wsc, out, M, N, K);
     return launch_status();
   }
-  W8Plan p;
   if (!plan_w8_decode(M, N, K, &p)) return KBH_ERR_SHAPE;
   const size_t need = splitk_workspace_bytes(M, N, p.splits);
   if (need > 0 && (!workspace || workspace_bytes < need)) return KBH_ERR_WORKSPACE;
