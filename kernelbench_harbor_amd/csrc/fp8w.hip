@@ -11,7 +11,16 @@
 #include "byte_weight_gemm.h"
 
 extern "C" size_t kbh_fp8w_workspace_bytes(int M, int N, int K, int block) {
-  return kbh::byte_gemm_workspace_bytes(M, N, K, block);
+  using kbh::byte_gemm_workspace_bytes;
+  if (block >= 32 && block <= 256 && (block & (block - 1)) == 0 && K % block == 0)
+    return byte_gemm_workspace_bytes(M, N, K, block);
+  // Any other block, for which the query has never failed: room for every accepted one.
+  size_t best = 0;
+  for (int b : {32, 64, 128, 256}) {
+    const size_t n = byte_gemm_workspace_bytes(M, N, K, b);
+    best = n > best ? n : best;
+  }
+  return best;
 }
 
 extern "C" int kbh_fp8w_gemm(const void* x, const uint8_t* w_fp8, const void* scales, void* y,
