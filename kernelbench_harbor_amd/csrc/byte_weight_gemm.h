@@ -489,22 +489,36 @@ struct ByteWide {
   int spg;
 };
 
+// Whether the decode kernel keeps a call of 17 to 127 rows from the wide tiles. It does while its
+// grid is resident at once, so that every weight is in flight and few split-K slices are written:
+// its blocks of 32 and 64 rows hold 116 to 228 registers, which leaves 8 waves to a CU. Workgroups of
+// under three waves have too little in flight each (K=N=1024 M=65 17.0 against 12.0 us), and above
+// one workgroup per CU up to 64 rows it also takes whole multiples of 8 workgroups (xcd_remap and the
+// slice sum placed by it: 3072 x 3712 M=64 19.6 against 16.1, 3072 x 3072 15.4 / 15.7). From 65 rows
+// the second row block of a little over one round is mostly padding that costs no MFMAs
+// (2560 x 4096 M=72 13.9 against 18.4). Measured over 169 layers of K and N from 1024 to 14336 and 208
+// with N of 128 mod 256: the choice is 0.3% from the faster kernel on average and never more than 11%
+// slower than decode, where "up to 64 rows and one workgroup per CU" lost up to 46% (M=127: 4096 x 2048
+// 13.8 against 20.0, 2048 x 4096 14.0 / 19.9; M=17: 4096 x 6144 13.1 / 14.1).
+inline bool byte_decode_stays(int M, const BytePlan& d) {
+  const int grid = d.ntiles * d.splits * d.mblocks;
+  const bool resident = grid <= 256 * (d.waves < 8 ? 8 / d.waves : 1);
+  if (M <= 64) return grid <= 256 || (resident && d.waves >= 4 && grid % 8 == 0);
+  return (resident && d.waves >= 3) || (M <= 96 && d.waves >= 5 && grid <= 320);
+}
+
 // Wide tiles from kByteWideMinM rows: the W4A16 geometry (64-row tiles up to 64 rows, 128-row
 // ones up to 128, then 128 or 256 rows by the estimate). They replace
 // tiled_f16_gemm's 256 x 128 tiles, which split no K (K=14336 N=4096: 32 workgroups and ~300 us
 // at every M from 128 to 1024; now 30.7 / 43.0 / 75.2 / 124 us at M=128 / 256 / 512 / 1024, and
-// 342 -> 226 at 2048), and the decode kernel's 32- and 64-row blocks (M=32 26.2 -> 19.4, M=48 42.9
-// -> 21.4, M=96 73.2 -> 28.4; 8192 x 28672 M=32 85.5 -> 66.9). Up to 64 rows the decode kernel
-// stays where its grid is one workgroup per CU: every
-// weight is then in flight at once and it needs fewer split-K slices (K=N=4096 M=64 14.6 against
-// 19.8 us, K=2048 N=8192 15.5 / 19.6; with a second round of workgroups the wide tiles win:
-// K=4096 N=6144 25.6 / 18.6, K=N=3584 16.9 / 15.9).
+// 342 -> 226 at 2048), and the decode kernel's 32- and 64-row blocks where those take several rounds
+// (M=32 26.2 -> 19.4, M=48 42.9 -> 21.4, M=96 73.2 -> 28.4; 8192 x 28672 M=32 85.5 -> 66.9).
 bool plan_byte_wide(int M, int N, int K, int block, ByteWide* w) {
   if (M < kByteWideMinM || N < 256) return false;
   // the kernels stage x with 32-bit offsets
   if ((size_t)(M + 256) * K * 2 >= ((size_t)1 << 31)) return false;
   BytePlan d;
-  if (M <= 64 && plan_byte_decode(M, N, K, &d) && d.ntiles * d.splits * d.mblocks <= 256) return false;
+  if (M < kByteTiledMinM && plan_byte_decode(M, N, K, &d) && byte_decode_stays(M, d)) return false;
   w->spg = block / 32;
   const int unit = wide_iteration(w->spg, kByteWidePD) / 2;
   return plan_wide(M, N, K, 256, 32, unit, unit, 256, kHalfCosts, &w->plan, M <= 64 ? 64 : 128);

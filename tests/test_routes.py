@@ -17,3 +17,10 @@ def test_fp8w_workspace_of_any_block(lib, M):
         assert most > 0
         for b in (0, 1, 96, 512):
             assert lib.kbh_fp8w_workspace_bytes(M, N, K, b) == most
+
+
+# M, K, N, K splits of the decode kernel's plan (the wide tiles' differs): its grid is resident at
+# once, or its second row block is mostly padding
+@pytest.mark.parametrize("M,K,N,splits", [(127, 4096, 2048, 8), (127, 2048, 4096, 4), (72, 2560, 4096, 5), (96, 3072, 3072, 6)])
+def test_fp8w_decode_kernel_stays(lib, M, K, N, splits):
+    assert lib.kbh_fp8w_workspace_bytes(M, N, K, 128) == splits * M * N * 4
