@@ -506,6 +506,7 @@ struct WidePlan {
   int splits;    // K ranges
   WideSplit sp;  // their slabs
   int grid;
+  float cost;    // estimated (plan_splits)
 };
 
 // Estimated time of a wide launch, for comparing plans: R rounds of workgroups over the 256 CUs
@@ -567,7 +568,7 @@ inline int plan_splits(long tiles, int M, int N, int KT, int unit, int slots, co
 }
 
 // Picks the tile height and the split count by plan_splits: tm_small rows up to 64 (small 64) or
-// 128 rows, above that the cheaper of 128 (choose) and 256 rows. `slots` is the number of
+// 128 rows, above that the cheaper of 128 and 256 rows. `slots` is the number of
 // workgroups the GPU runs at once (256 CUs x workgroups per CU); unit_small and unit_256 are the
 // slabs per unit of K that the kernel of that tile height takes.
 // N: columns, at least tn and a multiple of 128; the last tile overlaps its neighbour where N is
@@ -577,17 +578,17 @@ inline bool plan_wide(int M, int N, int K, int tn, int slab_k, int unit_small, i
   if (N < tn || N % 128 != 0 || M < 1 || K % slab_k != 0) return false;
   const int KT = K / slab_k;
   const auto tiles = [&](int tm) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
-  const auto take = [&](int tm, int splits, int unit) {
-    *p = WidePlan{tm, splits, wide_split(KT, unit, splits), (int)tiles(tm) * splits};
+  const auto take = [&](int tm, int splits, int unit, float cost) {
+    *p = WidePlan{tm, splits, wide_split(KT, unit, splits), (int)tiles(tm) * splits, cost};
     return true;
   };
   float csmall = 0.f, c256 = 0.f;
   const int ssmall = plan_splits(tiles(tm_small), M, N, KT, unit_small, slots,
                                  tm_small == 64 ? cs.h64 : cs.h128, cs, &csmall);
-  if (M <= 128) return ssmall > 0 && take(tm_small, ssmall, unit_small);
+  if (M <= 128) return ssmall > 0 && take(tm_small, ssmall, unit_small, csmall);
   const int s256 = plan_splits(tiles(256), M, N, KT, unit_256, slots, cs.h256, cs, &c256);
-  if (ssmall > 0 && (s256 == 0 || csmall < c256)) return take(tm_small, ssmall, unit_small);
-  return s256 > 0 && take(256, s256, unit_256);
+  if (ssmall > 0 && (s256 == 0 || csmall < c256)) return take(tm_small, ssmall, unit_small, csmall);
+  return s256 > 0 && take(256, s256, unit_256, c256);
 }
 
 // Slabs per unit of K of the kernels' loop iteration: U slabs (two quantization groups of spg

@@ -264,7 +264,7 @@ __global__ __launch_bounds__(256) void w8a8_tiled_kernel(
 constexpr int kW8TiledMinM = 128;
 
 // ======================================================================================
-// Wide-tile kernel (M > 32, and from 17 rows for large weights)
+// Wide-tile kernel (from 17 rows; smaller layers from 33, or 128 where N is no multiple of 256)
 // ======================================================================================
 
 // int8 weight-slab producer for tiled_wide_gemm: 64 K rows x 256 columns per slab. Thread t owns
@@ -351,32 +351,47 @@ struct W8Out {
 
 constexpr int kW8WideMinM = 17;
 
-// 256-row tiles at every M: the int8 slab producer holds 8 rows x 8 columns per thread, which
-// does not fit the register budget of two 128-row workgroups per CU.
+// One workgroup per CU at either tile height: the int8 slab producer holds 8 rows x 8 columns per
+// thread, which does not fit the register budget of two 128-row workgroups per CU.
 // Prefetch depth 4 (four 64-deep slabs in flight) when the K slabs come in multiples of 4.
 int w8_wide_pd(int K) { return (K / 64) % 4 == 0 ? 4 : 2; }
 
 // x within the 12-wave kernel's 32-bit offsets.
 bool w8_x_staged(int M, int K) { return (size_t)(M + 256) * K < ((size_t)1 << 31); }
 
-// 128-row tiles (one workgroup per CU) up to 128 rows; above, 256-row tiles unless they would
-// leave CUs idle (plan_wide's choose_tm).
-bool plan_w8_wide(int M, int N, int K, WidePlan* p) {
-  if (M < kW8WideMinM || N < 256) return false;
-  // 17 to 32 rows: the decode kernel streams the weights once per 16-row block and stays where its
-  // grid is at most two workgroups per CU (M=32: 4096 x 6144 14.1 against 17.2 us, 5120 x 5120 14.8 /
-  // 17.4); beyond that the wide tiles (14336 x 4096 28.3 -> 21.4, 3584 x 18944 30.3 -> 23.6, 8192 x
-  // 28672 102 -> 58).
-  W8Plan d;
-  if (M <= 32 && plan_w8_decode(M, N, K, &d) && d.ntiles * d.splits * d.mblocks <= 512) return false;
-  // slabs per unit of K: the 128-row kernel's iteration; half of the 12-wave kernel's
-  const int unit256 = w8_x_staged(M, K) ? 2 : w8_wide_pd(K);
-  return plan_wide(M, N, K, 256, 64, w8_wide_pd(K), unit256, 256, kInt8Costs, p);
+// Calls that the decode kernel may keep from the wide tiles: up to 32 rows, and up to 127 where N is
+// no multiple of 256. It has run them all once, and a workspace alone is still enough for them: they
+// take it where no scratch is given.
+bool w8_decode_range(int M, int N) { return M <= 32 || (M < kW8TiledMinM && N % 256 != 0); }
+
+// Whether the decode kernel keeps a call of that range. It streams the weights once per 16-row block:
+// always while its grid is resident at once (two workgroups per CU: 1024 x 1024 .. 8192 x 1152 at 33 to
+// 127 rows 8-16 us against 14-20), and beyond where its estimated time is at most 3% over the wide
+// plan's, 25% in the second round of full workgroups whose splits are a power of two (the fit has those
+// too slow: 8192 x 1408 M=127 16.2 us against 20.3). Both estimates (us) are least-squares fits to 2000
+// calls of 17 to 127 rows over K from 1024 to 14336 and N from 384 to 14464 (decode 7.6%, wide 5.1%
+// rms): the choice is 0.7% from the faster kernel on average past 512 workgroups; 7 of those calls are
+// 4% or more slower than on decode, where "at most 512 workgroups, and N a multiple of 256" left 769 (by
+// up to 79%: K=2048 N=1408 M=48 9.0 -> 15.0 us).
+bool w8_decode_stays(int M, int N, const W8Plan& d, const WidePlan& w) {
+  const int grid = d.ntiles * d.splits * d.mblocks;
+  if (grid <= 512) return true;
+  float dec = 5.3f + 4.37f * (float)grid * (float)(d.waves * d.spw) / 4096.0f + 1.27f * (float)((grid + 511) / 512);
+  if (d.splits > 1) dec += 0.16f + 0.064f * d.splits + 0.164f * ((float)d.splits * M * N * 8.0f / (float)(1 << 20));
+  const bool full = grid <= 768 && d.waves == 8 && d.splits >= 4 && (d.splits & (d.splits - 1)) == 0;
+  return dec <= (full ? 1.25f : 1.03f) * ((w.splits > 1 ? 8.4f : 4.2f) + 0.288f * w.cost);
 }
 
-// Calls that a workspace alone has always been enough for (the decode kernel's, which ran them all
-// once): they still take that kernel where no scratch is given.
-bool w8_decode_is_enough(int M, int N) { return M <= 32 || (M < kW8TiledMinM && N % 256 != 0); }
+// 128-row tiles (one workgroup per CU) up to 128 rows; above, 128-row or 256-row tiles by the
+// estimate.
+bool plan_w8_wide(int M, int N, int K, WidePlan* p) {
+  if (M < kW8WideMinM || N < 256) return false;
+  // slabs per unit of K: the 128-row kernel's iteration; half of the 12-wave kernel's
+  const int unit256 = w8_x_staged(M, K) ? 2 : w8_wide_pd(K);
+  if (!plan_wide(M, N, K, 256, 64, w8_wide_pd(K), unit256, 256, kInt8Costs, p)) return false;
+  W8Plan d;
+  return !(w8_decode_range(M, N) && plan_w8_decode(M, N, K, &d) && w8_decode_stays(M, N, d, *p));
+}
 
 template <bool OUT_I32, int TM, int PD>
 void launch_w8_wide(const WidePlan& p, const void* x, const void* w, const void* xs,
@@ -412,7 +427,7 @@ int w8a8_run(const void* x, const void* w, const void* xs, const void* wsc, void
   WidePlan wp;
   W8Plan p;
   bool wide = plan_w8_wide(M, N, K, &wp);
-  if (wide && w8_decode_is_enough(M, N) && plan_w8_decode(M, N, K, &p)) {
+  if (wide && w8_decode_range(M, N) && plan_w8_decode(M, N, K, &p)) {
     const size_t sc = wide_workspace_bytes(M, N, wp.splits), need = splitk_workspace_bytes(M, N, p.splits);
     const bool scratch_ok = sc == 0 || (scratch && scratch_bytes >= sc);
     if (!scratch_ok && (need == 0 || (workspace && workspace_bytes >= need))) wide = false;

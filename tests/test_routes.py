@@ -24,3 +24,11 @@ def test_fp8w_workspace_of_any_block(lib, M):
 @pytest.mark.parametrize("M,K,N,splits", [(127, 4096, 2048, 8), (127, 2048, 4096, 4), (72, 2560, 4096, 5), (96, 3072, 3072, 6)])
 def test_fp8w_decode_kernel_stays(lib, M, K, N, splits):
     assert lib.kbh_fp8w_workspace_bytes(M, N, K, 128) == splits * M * N * 4
+
+
+# M, K, N: calls that the decode kernel runs faster than the wide tiles (which take scratch here), and
+# calls past the line
+@pytest.mark.parametrize("M,K,N,wide", [(48, 2048, 1408, False), (127, 4096, 1664, False), (33, 8192, 2432, False), (17, 3584, 14336, False),
+                                        (17, 11008, 1024, False), (127, 2048, 8576, True), (64, 18944, 2176, True), (32, 14336, 4096, True)])
+def test_w8a8_decode_kernel_stays(lib, M, K, N, wide):
+    assert (lib.kbh_w8a8_scratch_bytes(M, N, K) > 0) == wide
