@@ -515,6 +515,7 @@ struct WidePlan {
 // other down); and the slices of partial sums written and read (per 2^18 of them).
 struct WideCost {
   float round, slab, load;  // of one tile height
+  float many;               // added to the factor of uneven splits for each split past 10
 };
 struct WideCosts {
   WideCost h64, h128, h256;  // by tile rows
@@ -527,17 +528,19 @@ struct WideCosts {
 // within 0.1%): the plan it picks is 0.7% from the sweep's fastest on average, where rounds times
 // slabs with the same slices lost 3.4% (4096 x 4096 M=512 42.9 -> 34.1 us, 4096 x 14336 M=320 73.5
 // -> 60.9, 4096 x 6144 M=512 50.5 -> 43.4).
-constexpr WideCosts kHalfCosts{{2.98f, 0.335f, 0.f}, {3.15f, 0.32f, 0.179f}, {4.78f, 0.437f, 0.389f},
+constexpr WideCosts kHalfCosts{{2.98f, 0.335f, 0.f, 0.f}, {3.15f, 0.32f, 0.179f, 0.f}, {4.78f, 0.437f, 0.389f, 0.f},
                                0.231f, 0.93f, 1.f};
 // bf16 weights cost the producers about 0.07 us more per slab (K=14336 N=4096 M=128 33.4 against
 // 31.4 us, M=2048 247 / 231).
-constexpr WideCosts kBf16Costs{{2.98f, 0.4f, 0.f}, {3.15f, 0.39f, 0.179f}, {4.78f, 0.5f, 0.389f},
+constexpr WideCosts kBf16Costs{{2.98f, 0.4f, 0.f, 0.f}, {3.15f, 0.39f, 0.179f, 0.f}, {4.78f, 0.5f, 0.389f, 0.f},
                                0.231f, 0.93f, 1.f};
 // int8 operands (relative): a 256-row slab measures 4/3 of a 128-row one, 2^18 slice values a third
 // of that (a fit as above gained under 0.5% over the sweep). Uneven splits are taken where they
 // save a tenth (K=18944 N=3584 M=128 94.7 -> 28.3 us), not for a few percent of the estimate
-// (K=3584 N=18944 M=256 measured 41 us with 2 splits and 43 with 3).
-constexpr WideCosts kInt8Costs{{0.f, 3.f, 0.f}, {0.f, 3.f, 0.f}, {0.f, 4.f, 0.f}, 1.f, 0.f, 1.1f};
+// (K=3584 N=18944 M=256 measured 41 us with 2 splits and 43 with 3), and many of them less still for
+// 256-row tiles, whose slices cost more than the estimate has it where they are a large part (M=160:
+// 7168 x 5120 29.4 us with 7 splits against 32.5 with 12, 14336 x 2560 29.2 with 14 / 32.5 with 23).
+constexpr WideCosts kInt8Costs{{0.f, 3.f, 0.f, 0.f}, {0.f, 3.f, 0.f, 0.f}, {0.f, 4.f, 0.f, 0.015f}, 1.f, 0.f, 1.1f};
 
 // The split of K of least estimated cost for `tiles` workgroups per split and M x N outputs
 // (*cost, when not null); 0 if K is no multiple of the unit. The splits are whole units, as even as
@@ -557,7 +560,7 @@ inline int plan_splits(long tiles, int M, int N, int KT, int unit, int slots, co
     const float rounds = (float)((tiles * s + slots - 1) / slots);
     const float t = (rounds * (c.round + longest * c.slab) + (float)(tiles * KT) / 256.0f * c.load +
                      (s > 1 ? (float)((long)s * M * N >> 18) * cs.slice + cs.split : 0.f)) *
-                    (KT % (4 * s) == 0 ? 1.f : cs.uneven);
+                    (KT % (4 * s) == 0 ? 1.f : cs.uneven + (s > 10 ? c.many * (float)(s - 10) : 0.f));
     if (best_s == 0 || t < best) {
       best = t;
       best_s = s;

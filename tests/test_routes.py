@@ -32,3 +32,9 @@ def test_fp8w_decode_kernel_stays(lib, M, K, N, splits):
                                         (17, 11008, 1024, False), (127, 2048, 8576, True), (64, 18944, 2176, True), (32, 14336, 4096, True)])
 def test_w8a8_decode_kernel_stays(lib, M, K, N, wide):
     assert (lib.kbh_w8a8_scratch_bytes(M, N, K) > 0) == wide
+
+
+@pytest.mark.parametrize("M,K,N,splits", [(160, 7168, 5120, 7), (160, 14336, 2560, 14), (129, 14336, 2560, 14)])
+def test_w8a8_many_uneven_splits(lib, M, K, N, splits):
+    """256-row tiles that are mostly padding: even splits, not more and shorter ones."""
+    assert lib.kbh_w8a8_scratch_bytes(M, N, K) == splits * M * N * 4
