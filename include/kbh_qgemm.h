@@ -37,6 +37,17 @@ enum kbh_status {
   KBH_ERR_SCRATCH_LIMIT = 7  /* the call needs more than the fixed scratch of a no-alloc entry */
 };
 
+/* The kernel a dense GEMM call takes (kbh_*_kernel): a wide tile's code is its rows. */
+enum kbh_kernel {
+  KBH_KERNEL_NONE = 0,     /* shape not supported */
+  KBH_KERNEL_DECODE = 1,   /* split-K decode kernel */
+  KBH_KERNEL_STREAM = 2,   /* streaming kernel */
+  KBH_KERNEL_STAGED = 3,   /* LDS-staged 256 x 128 tiles */
+  KBH_KERNEL_WIDE64 = 64,
+  KBH_KERNEL_WIDE128 = 128,
+  KBH_KERNEL_WIDE256 = 256
+};
+
 /* Library version of this ABI (KBH_ABI_VERSION). */
 int kbh_abi_version(void);
 
@@ -76,6 +87,10 @@ int kbh_w4a16_gemm(const void* x, const int32_t* qweight, const void* scales, co
                    void* y, void* workspace, size_t workspace_bytes, void* scratch,
                    size_t scratch_bytes, int M, int N, int K, int group, int dtype, void* stream);
 
+/* The kernel (enum kbh_kernel) that kbh_w4a16_gemm takes for these sizes when given the buffers its
+ * queries ask for, and its K splits (splits may be NULL). Host code only; for tests and tuning. */
+int kbh_w4a16_kernel(int M, int N, int K, int group, int dtype, int* splits);
+
 /* The same W4A16 GEMM without any caller buffer or allocation. No counterpart in the reference:
  * it is for callers that cannot allocate device memory or pass a workspace (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). The split-K partial sums live
@@ -109,6 +124,7 @@ int kbh_w4a16_gemm_noalloc(const void* x, const int32_t* qweight, const void* sc
  */
 size_t kbh_w8a8_workspace_bytes(int M, int N, int K);
 size_t kbh_w8a8_scratch_bytes(int M, int N, int K);
+int kbh_w8a8_kernel(int M, int N, int K, int* splits); /* as kbh_w4a16_kernel */
 int kbh_w8a8_gemm(const int8_t* x_int8, const int8_t* w_int8, const void* x_scale,
                   const void* w_scale, void* y, void* workspace, size_t workspace_bytes,
                   void* scratch, size_t scratch_bytes, int M, int N, int K, void* stream);
@@ -132,6 +148,7 @@ int kbh_w8a8_gemm_i32(const int8_t* x_int8, const int8_t* w_int8, int32_t* acc_o
  * workspace: as for kbh_w4a16_gemm, with kbh_fp8w_workspace_bytes().
  */
 size_t kbh_fp8w_workspace_bytes(int M, int N, int K, int block);
+int kbh_fp8w_kernel(int M, int N, int K, int block, int* splits); /* as kbh_w4a16_kernel */
 int kbh_fp8w_gemm(const void* x, const uint8_t* w_fp8, const void* scales, void* y,
                   void* workspace, size_t workspace_bytes, int M, int N, int K, int block,
                   int dtype, void* stream);

@@ -25,6 +25,12 @@ KBH_ERR_ALIGN = 5
 KBH_ERR_LAUNCH = 6
 KBH_ERR_SCRATCH_LIMIT = 7
 
+# Kernel codes of include/kbh_qgemm.h (enum kbh_kernel); a wide tile's code is its rows.
+KBH_KERNEL_NONE = 0
+KBH_KERNEL_DECODE = 1
+KBH_KERNEL_STREAM = 2
+KBH_KERNEL_STAGED = 3
+
 # KBH_W4A16_NOALLOC_SCRATCH_BYTES of include/kbh_qgemm.h: the fixed per-GPU scratch of
 # kbh_w4a16_gemm_noalloc.
 W4A16_NOALLOC_SCRATCH_BYTES = 64 << 20
@@ -45,12 +51,15 @@ SIGNATURES = {
     "kbh_w4a16_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "kbh_w4a16_scratch_bytes": (_sz, [_i, _i, _i, _i]),
     "kbh_w4a16_gemm": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
+    "kbh_w4a16_kernel": (_i, [_i] * 5 + [_vp]),
     "kbh_w4a16_gemm_noalloc": (_i, [_vp] * 5 + [_i] * 5 + [_vp]),
     "kbh_w8a8_workspace_bytes": (_sz, [_i, _i, _i]),
     "kbh_w8a8_scratch_bytes": (_sz, [_i, _i, _i]),
+    "kbh_w8a8_kernel": (_i, [_i] * 3 + [_vp]),
     "kbh_w8a8_gemm": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _sz, _i, _i, _i, _vp]),
     "kbh_w8a8_gemm_i32": (_i, [_vp, _vp, _vp, _vp, _sz, _vp, _sz, _i, _i, _i, _vp]),
     "kbh_fp8w_workspace_bytes": (_sz, [_i, _i, _i, _i]),
+    "kbh_fp8w_kernel": (_i, [_i] * 4 + [_vp]),
     "kbh_fp8w_gemm": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
     "kbh_mxfp8_workspace_bytes": (_sz, [_i, _i, _i]),
     "kbh_mxfp8_gemm": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _vp]),

@@ -23,6 +23,23 @@ extern "C" size_t kbh_fp8w_workspace_bytes(int M, int N, int K, int block) {
   return best;
 }
 
+extern "C" int kbh_fp8w_kernel(int M, int N, int K, int block, int* splits) {
+  using namespace kbh;
+  if (splits) *splits = 1;
+  if (M < 1 || N < 128 || K < 32 || N % 128 != 0 || !quant_group_ok(K, block)) return KBH_KERNEL_NONE;
+  ByteWide w;
+  if (plan_byte_wide(M, N, K, block, &w)) {
+    if (splits) *splits = w.plan.splits;
+    return w.plan.tm;
+  }
+  if (M >= kByteTiledMinM && K % (TBK * TDEPTH) == 0) return KBH_KERNEL_STAGED;
+  BytePlan p;
+  if (!plan_byte_decode(M, N, K, &p)) return KBH_KERNEL_NONE;
+  const int s = plan_byte_stream(M, N, K, p);
+  if (splits) *splits = s > 0 ? s : p.splits;
+  return s > 0 ? KBH_KERNEL_STREAM : KBH_KERNEL_DECODE;
+}
+
 extern "C" int kbh_fp8w_gemm(const void* x, const uint8_t* w_fp8, const void* scales, void* y,
                              void* workspace, size_t workspace_bytes, int M, int N, int K,
                              int block, int dtype, void* stream) {

@@ -26,6 +26,11 @@ int launch_status();
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Quantization groups (scale blocks) the GEMMs take.
+inline bool quant_group_ok(int K, int group) {
+  return (group == 32 || group == 64 || group == 128 || group == 256) && K % group == 0;
+}
+
 inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // ---- device helpers -------------------------------------------------------------------

@@ -500,6 +500,23 @@ extern "C" size_t kbh_w4a16_scratch_bytes(int M, int N, int K, int group) {
   return kbh::w4_wide_scratch_bytes(M, N, K, group);
 }
 
+extern "C" int kbh_w4a16_kernel(int M, int N, int K, int group, int dtype, int* splits) {
+  using namespace kbh;
+  if (splits) *splits = 1;
+  if (M < 1 || N < 128 || K < 32 || N % 128 != 0 || !quant_group_ok(K, group)) return KBH_KERNEL_NONE;
+  W4Wide w;
+  if (plan_w4_wide(M, N, K, group, dtype == KBH_BF16, &w)) {
+    if (splits) *splits = w.plan.splits;
+    return w.plan.tm;
+  }
+  if (M >= kTiledMinM && K % (TBK * TDEPTH) == 0) return KBH_KERNEL_STAGED;
+  DecodePlan p;
+  if (!plan_decode(M, N, K, group / 32, &p)) return KBH_KERNEL_NONE;
+  const int s = plan_stream(p, M, N, K, group);
+  if (splits) *splits = s > 0 ? s : p.splits;
+  return s > 0 ? KBH_KERNEL_STREAM : KBH_KERNEL_DECODE;
+}
+
 extern "C" int kbh_w4a16_gemm(const void* x, const int32_t* qweight, const void* scales,
                               const void* zeros, void* y, void* workspace, size_t workspace_bytes,
                               void* scratch, size_t scratch_bytes, int M, int N, int K, int group,

@@ -497,6 +497,22 @@ extern "C" size_t kbh_w8a8_scratch_bytes(int M, int N, int K) {
   return kbh::wide_workspace_bytes(M, N, p.splits);
 }
 
+extern "C" int kbh_w8a8_kernel(int M, int N, int K, int* splits) {
+  using namespace kbh;
+  if (splits) *splits = 1;
+  if (M < 1 || N < 128 || K < 64 || N % 128 != 0 || K % 64 != 0) return KBH_KERNEL_NONE;
+  WidePlan w;
+  if (plan_w8_wide(M, N, K, &w)) {
+    if (splits) *splits = w.splits;
+    return w.tm;
+  }
+  if (M >= kW8TiledMinM && K % (WBK * WDEPTH) == 0) return KBH_KERNEL_STAGED;
+  W8Plan p;
+  if (!plan_w8_decode(M, N, K, &p)) return KBH_KERNEL_NONE;
+  if (splits) *splits = p.splits;
+  return KBH_KERNEL_DECODE;
+}
+
 extern "C" int kbh_w8a8_gemm(const int8_t* x_int8, const int8_t* w_int8, const void* x_scale,
                              const void* w_scale, void* y, void* workspace, size_t workspace_bytes,
                              void* scratch, size_t scratch_bytes, int M, int N, int K,

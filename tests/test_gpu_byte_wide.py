@@ -1,7 +1,7 @@
 """The byte-weight GEMM (FP8 weights, and the multi-LoRA base) on the warp-specialised wide tiles,
 and K ranges that end in the middle of the kernels' loop iteration.
 
-Edges: the first row count of each tile height (33, 65, 257 rows), full and one-row-over tiles, one
+Edges: row counts about the tile heights of 64 and 128 rows, full and one-row-over tiles, one
 column tile, K of an odd number of quantization groups (half an iteration), every block size, and
 shapes where the decode kernel's grid exceeds one workgroup per CU (64-row tiles)."""
 import numpy as np
@@ -56,7 +56,8 @@ def test_fp8w_wide_dequant_bit_exact(dev, M, block, dtype):
 @pytest.mark.parametrize("T", [65, 129, 257])
 def test_lora_wide_base_matches_native_rounding(dev, T, dtype):
     """One-hot activations and dyadic adapters (every sum exact in fp32), any int8 value in the
-    base weight: bit-exact against the oracle's native path on 128- and 256-row tiles."""
+    base weight: bit-exact against the oracle's native path on 128-row tiles (N = 256 is one column tile,
+    so the estimate never picks 256 rows)."""
     D, N, r, L = 640, 256, 16, 3
     g = torch.Generator().manual_seed(T)
     q = torch.randint(-128, 128, (D, N), generator=g, dtype=torch.int8)
@@ -103,8 +104,8 @@ def test_w4a16_half_iteration_tails(dev, M, K, group, dtype):
 
 
 # M, K, N: a last column tile that overlaps its neighbour (N % 256 == 128), K ranges of uneven
-# length (units that no split count near the 256 workgroups divides), K / 64 even but not a
-# multiple of 4 (the 12-wave int8 kernel's half iterations)
+# length (units that no split count near the 256 workgroups divides). The plans are 64- and 128-row
+# tiles and, where that is faster, the decode kernel; the 256-row tiles' edges are in test_gpu_routes.py.
 WIDE_EDGES = [(33, 1152, 384), (129, 2176, 384), (200, 18944, 640), (300, 1408, 896), (257, 128, 384),
               (64, 9472, 1152), (17, 18944, 2176), (32, 9472, 4224)]  # 17-32 rows: 64/128-row tiles
 

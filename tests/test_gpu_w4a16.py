@@ -51,7 +51,7 @@ CASES = [
     (64, 1024, 768, 256, torch.bfloat16, "reference"),
     (56, 2048, 512, 128, torch.float16, "baseline"),
     (40, 4096, 256, 128, torch.bfloat16, "reference"),
-    # N % 256 != 0 above 128 rows: the 256 x 128 LDS-staged kernel
+    # N % 256 != 0: a last column tile that overlaps its neighbour
     (160, 2048, 384, 128, torch.float16, "baseline"),
     # warp-specialised 128-row tiles (64 < M <= 256, N % 256 == 0) and 256-row tiles above, with
     # 256- and 32-row groups
@@ -96,7 +96,7 @@ def test_w4a16_dequant_bit_exact(dev, dtype, M, N, zeros):
     k_m rounded once to the output dtype: it must equal the reference's own dequantization
     (unpack, subtract zero with one rounding, multiply by scale with one rounding) bit for bit.
     M=16 exercises the split-K decode kernel, M=64 and M=200 the wide-tile kernel (64- and
-    128-row tiles), N=384 at M=160 the 256 x 128 LDS-staged kernel. Zero points with a
+    128-row tiles), N=384 at M=160 a last column tile that overlaps its neighbour. Zero points with a
     fractional part make the subtraction round, which the wide kernel reproduces exactly.
     The 64- and 128-row fp16 tiles take a shorter dequantisation when every zero point of a
     workgroup's K range and columns is an integer below 960 in magnitude: "uint4" and "wide"

@@ -1,7 +1,7 @@
 """The W4A16 entry point that allocates nothing (kbh_w4a16_gemm_noalloc), called through the C
 ABI: bit-identical to kbh_w4a16_gemm (same kernels, same split-K sum order) on consecutive
 calls that use the library's fixed scratch array, each call smaller than the one before it,
-across the wide-tile (split-K scratch), LDS-staged and decode (split-K workspace) paths."""
+across the wide-tile (split-K scratch) and decode (split-K workspace) paths."""
 import ctypes
 
 import pytest
@@ -12,8 +12,8 @@ from kernelbench_harbor_amd import _lib, inputs, ops
 pytestmark = pytest.mark.gpu
 
 # (M, K, N): M=2048 fills the 64 MiB array exactly (two K splits of 2048 x 4096 fp32), M=64 takes
-# 14 K splits on 64 x 256 tiles, M=160 with N=384 the LDS-staged kernel (no scratch), M=16 and
-# M=1 the split-K decode kernel.
+# 14 K splits on 64 x 256 tiles, M=160 with N=384 128-row tiles of which the last overlaps its
+# neighbour, M=16 and M=1 the split-K decode kernel.
 CASES = [(2048, 14336, 4096), (64, 14336, 4096), (160, 2048, 384), (16, 4096, 512), (1, 1024, 256)]
 
 
