@@ -357,6 +357,21 @@ struct W4Wide {
 // Prefetch depth of a wide W4 launch with tn-column tiles.
 constexpr int w4_wide_pd(int tn) { return tn == 256 ? 4 : 2; }
 
+// Whether the decode kernel keeps a call of 33 to 127 rows whose K ends in half an iteration of the wide
+// tiles (it ran all of these before the tiles took them): by the two estimates in us, least-squares
+// fits over 892 such calls (K of an odd number of 128-row groups from 384 to 11136, N from 1024 to 14336,
+// both dtypes; decode 8%, wide 4% rms). The choice is 0.2% from the faster kernel on average and 7
+// calls are 4% or more slower than on decode, where the wide tiles alone left 441, by up to 131%
+// (K=640 N=8192 M=64 7.9 -> 12.7 us).
+bool w4_decode_stays(int M, int N, int K, int group, bool bf16, const WidePlan& w) {
+  DecodePlan d;
+  if (!plan_decode(M, N, K, group / 32, &d)) return false;
+  if (splitk_workspace_bytes(M, N, d.splits) > KBH_W4A16_NOALLOC_SCRATCH_BYTES) return false;  // the no-alloc entry point takes the call
+  const float dec = (d.splits > 1 ? 4.75f : 2.75f) +
+                    0.84f * decode_cost(M, N, d.nw, d.spw, d.waves, d.splits, d.ntiles * d.splits * d.mblocks);
+  return dec <= 1.68f * w.cost + (w.tm == 64 ? -2.5f : -0.7f) + (w.splits > 1 ? 0.8f : 0.f) + (bf16 ? 0.4f : 0.f);
+}
+
 bool plan_w4_wide(int M, int N, int K, int group, bool bf16, W4Wide* w) {
   if (M < kWideMinM) return false;
   w->spg = group / 32;
@@ -372,8 +387,10 @@ bool plan_w4_wide(int M, int N, int K, int group, bool bf16, W4Wide* w) {
   // tile would spend half its MFMAs and A loads on padding there. Above 128 rows the estimate
   // chooses between 128-row and 256-row tiles.
   const bool rows64 = M <= 64 && w->tn == 256;
-  return plan_wide(M, N, K, w->tn, 32, unit, unit, w->tn == 128 ? 512 : 256,
-                   bf16 ? kBf16Costs : kHalfCosts, &w->plan, rows64 ? 64 : 128);
+  if (!plan_wide(M, N, K, w->tn, 32, unit, unit, w->tn == 128 ? 512 : 256, bf16 ? kBf16Costs : kHalfCosts,
+                 &w->plan, rows64 ? 64 : 128))
+    return false;
+  return !(ws && M < kTiledMinM && K % (64 * unit) != 0 && w4_decode_stays(M, N, K, group, bf16, w->plan));
 }
 
 // Scratch of the wide kernels, for either dtype (the query does not name it): the larger plan's.
@@ -476,10 +493,9 @@ void dispatch_w4_wide(const W4Wide& w, const void* x, const int32_t* qw, const v
 // Bytes of device memory the path a call takes needs beyond its inputs and outputs: the wide
 // kernel's split-K scratch, nothing for the LDS-staged kernel, or the decode kernel's split-K
 // workspace (the dispatch order of kbh_w4a16_gemm).
-size_t w4a16_path_bytes(int M, int N, int K, int group) {
-  const size_t wide = w4_wide_scratch_bytes(M, N, K, group);
+size_t w4a16_path_bytes(int M, int N, int K, int group, int dtype) {
   W4Wide w;
-  if (plan_w4_wide(M, N, K, group, false, &w)) return wide;
+  if (plan_w4_wide(M, N, K, group, dtype == KBH_BF16, &w)) return wide_workspace_bytes(M, N, w.plan.splits);
   if (M >= kTiledMinM && K % (TBK * TDEPTH) == 0) return 0;
   DecodePlan p;
   if (!plan_decode(M, N, K, group / 32, &p)) return 0;

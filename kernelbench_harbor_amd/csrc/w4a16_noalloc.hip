@@ -14,7 +14,7 @@
 
 namespace kbh {
 // The scratch need of the path a W4A16 call takes (defined with the kernels in w4a16.hip).
-size_t w4a16_path_bytes(int M, int N, int K, int group);
+size_t w4a16_path_bytes(int M, int N, int K, int group, int dtype);
 
 namespace {
 
@@ -66,7 +66,7 @@ extern "C" int kbh_w4a16_gemm_noalloc(const void* x, const int32_t* qweight, con
   if (M < 1 || N < 128 || K < 32 || (N % 128) != 0 || (K % 32) != 0) return KBH_ERR_SHAPE;
   if (group != 32 && group != 64 && group != 128 && group != 256) return KBH_ERR_SHAPE;
   if (K % group != 0) return KBH_ERR_SHAPE;
-  const size_t need = w4a16_path_bytes(M, N, K, group);
+  const size_t need = w4a16_path_bytes(M, N, K, group, dtype);
   if (need > KBH_W4A16_NOALLOC_SCRATCH_BYTES) return KBH_ERR_SCRATCH_LIMIT;
   void* p = nullptr;
   const int st = noalloc_scratch(&p);

@@ -1,4 +1,6 @@
 """Which kernel a call takes, as far as the size queries tell (CPU: the queries are host code)."""
+import ctypes
+
 import pytest
 
 from kernelbench_harbor_amd import _lib
@@ -7,6 +9,12 @@ from kernelbench_harbor_amd import _lib
 @pytest.fixture(scope="module")
 def lib():
     return _lib.load()
+
+
+def _kernel(query, *sizes):
+    """(kernel code, K splits) of a kbh_*_kernel query."""
+    n = ctypes.c_int()
+    return query(*sizes, ctypes.byref(n)), n.value
 
 
 @pytest.mark.parametrize("M", [1, 16, 32, 100, 300])
@@ -38,3 +46,14 @@ def test_w8a8_decode_kernel_stays(lib, M, K, N, wide):
 def test_w8a8_many_uneven_splits(lib, M, K, N, splits):
     """256-row tiles that are mostly padding: even splits, not more and shorter ones."""
     assert lib.kbh_w8a8_scratch_bytes(M, N, K) == splits * M * N * 4
+
+
+# M, K, N, group, dtype, kernel: K that ends in half an iteration of the wide tiles (the decode kernel ran
+# all of these), where the decode kernel's estimate is lower and where it is not
+@pytest.mark.parametrize("M,K,N,group,dtype,kernel", [
+    (64, 896, 4096, 128, _lib.KBH_F16, _lib.KBH_KERNEL_DECODE), (127, 640, 8192, 128, _lib.KBH_BF16, _lib.KBH_KERNEL_DECODE),
+    (33, 1408, 2048, 128, _lib.KBH_F16, _lib.KBH_KERNEL_DECODE), (48, 1152, 4096, 128, _lib.KBH_BF16, _lib.KBH_KERNEL_DECODE),
+    (127, 1152, 14336, 128, _lib.KBH_F16, 128), (64, 29568, 8192, 128, _lib.KBH_F16, 64), (128, 640, 8192, 128, _lib.KBH_F16, 128),
+    (64, 1024, 4096, 128, _lib.KBH_F16, 64)])
+def test_w4a16_decode_kernel_stays(lib, M, K, N, group, dtype, kernel):
+    assert lib.kbh_w4a16_kernel(M, N, K, group, dtype, None) == kernel
