@@ -45,6 +45,7 @@ enum kbh_kernel {
   KBH_KERNEL_STAGED = 3,   /* LDS-staged 256 x 128 tiles */
   KBH_KERNEL_WIDE64 = 64,
   KBH_KERNEL_WIDE128 = 128,
+  KBH_KERNEL_NARROW128 = 129, /* 128 x 128 tiles */
   KBH_KERNEL_WIDE256 = 256
 };
 

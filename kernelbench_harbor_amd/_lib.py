@@ -30,6 +30,7 @@ KBH_KERNEL_NONE = 0
 KBH_KERNEL_DECODE = 1
 KBH_KERNEL_STREAM = 2
 KBH_KERNEL_STAGED = 3
+KBH_KERNEL_NARROW128 = 129
 
 # KBH_W4A16_NOALLOC_SCRATCH_BYTES of include/kbh_qgemm.h: the fixed per-GPU scratch of
 # kbh_w4a16_gemm_noalloc.

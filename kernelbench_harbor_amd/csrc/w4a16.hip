@@ -376,6 +376,12 @@ bool plan_w4_wide(int M, int N, int K, int group, bool bf16, W4Wide* w) {
   if (M < kWideMinM) return false;
   w->spg = group / 32;
   w->tn = N >= 256 ? 256 : 128;
+  // 65 to 128 rows and N of 128 mod 256: 128-column tiles while their finest split (8 slabs) is at most one
+  // workgroup per CU. The half column tile that the 256-column ones compute twice costs them more there
+  // (bf16 M=96 2048 x 1408 13.4 against 15.2 us, 4096 x 384 13.0 / 14.7; fp16 M=96 4% and M=128 even),
+  // and beyond they win at once (K x N of 8.8 M 7 to 20%, 35 M 40%).
+  if (M > 64 && M <= 128 && N % 256 != 0 && K % (32 * wide_iteration(w->spg, w4_wide_pd(128))) == 0 && (long)N * K <= 256L * 128 * 256)
+    w->tn = 128;
   if (M > 128 && w->tn != 256) return false;
   // Slabs per unit of K: the warp-specialised kernels (256-column tiles, x under 2 GiB) take half
   // iterations. (K = 29568 holds an odd number of 128-row groups: on the LDS-staged and decode
@@ -523,7 +529,7 @@ extern "C" int kbh_w4a16_kernel(int M, int N, int K, int group, int dtype, int* 
   W4Wide w;
   if (plan_w4_wide(M, N, K, group, dtype == KBH_BF16, &w)) {
     if (splits) *splits = w.plan.splits;
-    return w.plan.tm;
+    return w.tn == 128 ? KBH_KERNEL_NARROW128 : w.plan.tm;
   }
   if (M >= kTiledMinM && K % (TBK * TDEPTH) == 0) return KBH_KERNEL_STAGED;
   DecodePlan p;

@@ -153,3 +153,11 @@ def test_lds_staged_dequant_bit_exact(dev, dtype):
     y = ops.fp8w_gemm(x.to(dev), codes.view(torch.float8_e4m3fn).to(dev), s8.to(dev))
     W = of.dequant(codes.numpy(), s8.float().numpy(), dt)
     assert np.array_equal(y.float().cpu().numpy(), W[ks.numpy()])
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M,K,N,group", [(65, 512, 640, 32), (96, 2048, 1408, 128), (128, 1024, 8064, 64), (127, 1024, 384, 256),
+                                         (100, 2048, 128, 128)])
+def test_128_column_tiles(dev, M, K, N, group, dtype):
+    cols = (slice(0, min(N, 256)), slice(N - min(N, 384), N))
+    _w4a16(dev, M, K, N, group, dtype, _lib.KBH_KERNEL_NARROW128, cols)

@@ -57,3 +57,12 @@ def test_w8a8_many_uneven_splits(lib, M, K, N, splits):
     (64, 1024, 4096, 128, _lib.KBH_F16, 64)])
 def test_w4a16_decode_kernel_stays(lib, M, K, N, group, dtype, kernel):
     assert lib.kbh_w4a16_kernel(M, N, K, group, dtype, None) == kernel
+
+
+@pytest.mark.parametrize("M,K,N,group,kernel", [
+    (96, 2048, 1408, 128, 129), (128, 4096, 384, 64, 129), (65, 1024, 8064, 128, 129), (100, 1024, 128, 32, 129),
+    (96, 2048, 4224, 128, 128), (64, 2048, 1408, 128, 64), (96, 2048, 1280, 128, 128), (129, 2048, 1408, 128, 128)])
+def test_w4a16_128_column_tiles(lib, M, K, N, group, kernel):
+    """65 to 128 rows of a small layer with N of 128 mod 256."""
+    for dtype in (_lib.KBH_F16, _lib.KBH_BF16):
+        assert lib.kbh_w4a16_kernel(M, N, K, group, dtype, None) == kernel
