@@ -456,26 +456,28 @@ bool plan_byte_decode(int M, int N, int K, BytePlan* p) {
 }
 
 // K splits of the streaming kernel, or 0 where the decode kernel stays: it does while its grid is
-// resident at once (two workgroups per CU), and where its estimated time is lower. Both estimates
-// (us) are the weights at the rate of a full stream plus the fp32 slices written and read. The
-// decode kernel loses ~5 us to a nearly empty last round while it has few rounds (3584 x 18944:
-// 592 workgroups, 512 at once). The streaming kernel takes as long as its busiest CU, counted as 2.5
-// workgroups where a second one per CU is not there for all (the dispatcher puts three on some:
-// 4096 x 14336 448 / 672 workgroups 21.8 / 18.9 us). The 5% covers the estimates' own error: 8192 x 28672,
-// where 224 column tiles leave CUs idle, stays (M=1 43.4 us, streaming 47.3 at best; M=16 54.3 /
-// 52.1-55.6).
+// resident at once (two workgroups per CU), and where its estimated time is lower. Both estimates (us)
+// are least-squares fits: the decode kernel's to 434 calls of 1 to 16 rows past 512 workgroups (4.6% rms),
+// the streaming kernel's to 790 split counts of 54 layers (K from 2048 to 29568, N from 2560 to 65536; 7.6%
+// rms; its rounds are of one workgroup per CU, and rows of a multiple of 1 KB cost it more: N=10240 is
+// slower at every split). The 2.7% is about the smallest margin with which none of the 74 calls of M=1 and
+// 16 among those came out more than 4% slower than on the decode kernel. (One rate and a constant for each
+// kernel had chosen 22 of them 5 to 34% slower: 8192 x 10240 M=1 21.9 -> 26.7 us, 14336 x 10240 31.4 -> 42.0.)
 inline int plan_byte_stream(int M, int N, int K, const BytePlan& d) {
   const long grid = (long)d.ntiles * d.splits;
   if (M > 16 || grid <= 512 || K % kByteStreamChunk != 0 || (size_t)K * N >= ((size_t)1 << 31)) return 0;
-  const float slice = (float)M * N * 8.0f / 2.9e6f;
-  float best = 0.95f * ((float)K * N / 5.4e6f + (d.splits > 1 ? d.splits * slice : 0.f) + (grid <= 1280 ? 5.f : 0.f));
+  const float mb = (float)K * N * 1e-6f, slice = (float)M * N * 8e-6f;  // MB of weights; of one split's slices
+  float best = 0.973f * (6.89f + 0.149f * mb + (d.splits > 1 ? 0.28f * d.splits * slice : 0.f) +
+                         1.02f * (float)((grid + 511) / 512) + (d.waves < 8 ? 0.33f : 0.f) + 0.0158f * M);
+  const float fixed = 6.67f + (N % 1024 == 0 ? 0.0787f : 0.0637f) * mb + 0.0593f * M;
   int best_s = 0;
-  // at most the three workgroups a CU holds, at least two chunks per wave of a split K
+  // about one to at most the three workgroups a CU holds, at least two chunks per wave of a split K
   for (int s = 1; (long)d.ntiles * s <= 768; ++s) {
     if (s > 1 && K / kByteStreamChunk < 2 * kByteStreamWaves * s) break;
     const long wgs = (long)d.ntiles * s;
-    const float per_cu = wgs <= 256 ? 1.f : (wgs < 512 ? 2.5f : (float)((wgs + 255) / 256));
-    const float t = per_cu * ((float)K / s) * (128 * 256 / 5.1e6f) + (s > 1 ? s * slice : 0.f);
+    if (wgs < 190) continue;
+    const float row = wgs <= 256 ? 3.54e-3f : 3.37e-3f;  // of K and round
+    const float t = fixed + row * (float)((wgs + 255) / 256) * ((float)K / s) + (s > 1 ? 0.196f * s * slice : 0.f);
     if (t < best) {
       best = t;
       best_s = s;

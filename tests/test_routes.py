@@ -66,3 +66,13 @@ def test_w4a16_128_column_tiles(lib, M, K, N, group, kernel):
     """65 to 128 rows of a small layer with N of 128 mod 256."""
     for dtype in (_lib.KBH_F16, _lib.KBH_BF16):
         assert lib.kbh_w4a16_kernel(M, N, K, group, dtype, None) == kernel
+
+
+# rows, K, N: layers that the streaming kernel ran slower than the decode kernel, and ones it runs faster
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (1, 8192, 10240, _lib.KBH_KERNEL_DECODE), (16, 8192, 12288, _lib.KBH_KERNEL_DECODE), (1, 14336, 10240, _lib.KBH_KERNEL_DECODE),
+    (16, 6144, 14336, _lib.KBH_KERNEL_DECODE), (1, 5120, 18944, _lib.KBH_KERNEL_DECODE), (16, 7168, 13824, _lib.KBH_KERNEL_DECODE),
+    (16, 3584, 18944, _lib.KBH_KERNEL_STREAM), (1, 18944, 3584, _lib.KBH_KERNEL_STREAM), (16, 29568, 8192, _lib.KBH_KERNEL_STREAM),
+    (16, 11008, 4096, _lib.KBH_KERNEL_STREAM), (17, 3584, 18944, 64), (16, 4096, 14336, _lib.KBH_KERNEL_DECODE)])
+def test_fp8w_streaming_kernel(lib, M, K, N, kernel):
+    assert lib.kbh_fp8w_kernel(M, N, K, 128, None) == kernel
