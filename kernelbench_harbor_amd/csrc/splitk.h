@@ -27,17 +27,24 @@ struct SplitKSmem {
 };
 
 // V is the 4-element vector of T held per column set (kbh_f32x4 / kbh_i32x4).
+struct SplitKNoFix {
+  template <typename T>
+  __device__ void operator()(T*) const {}
+};
+
 // store(r, n, v): row r (< rows) of the tile, column n (< 16*NCS), value v summed over the waves.
-template <int NCS, typename T, typename V, int WAVES, typename Store>
+// fix(slice): may change the wave's own sums in LDS before they are added.
+template <int NCS, typename T, typename V, int WAVES, typename Store, typename Fix = SplitKNoFix>
 __device__ inline void splitk_wave_sum(const V (&tot)[NCS], SplitKSmem<NCS, T, WAVES>& sm, int rows,
-                                       Store store) {
+                                       Store store, Fix fix = Fix{}) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  T* mine = sm.red + wave * NCS * kSplitKCsStride;
   if (4 * (lane >> 4) < rows) {
-    T* slice = sm.red + wave * NCS * kSplitKCsStride;
 #pragma unroll
     for (int cs = 0; cs < NCS; ++cs)
-      *reinterpret_cast<V*>(&slice[cs * kSplitKCsStride + lane * 4]) = tot[cs];
+      *reinterpret_cast<V*>(&mine[cs * kSplitKCsStride + lane * 4]) = tot[cs];
   }
+  fix(mine);
   __syncthreads();
   // Position p = (lane l, column set cs), cs fastest: consecutive threads read consecutive
   // 16-byte chunks (the slice stride is 16 bytes mod 256) and own consecutive output columns.

@@ -15,6 +15,10 @@
 // parts of its K range and meet in LDS; the workgroup stores its fp32 tile into slice `split` of the
 // workspace.
 //
+// An infinity in x, or sums past fp32's range, leave NaN in all columns of that arithmetic (infinity
+// minus infinity). On expert tiles, whose batches of 32 rows and more per expert multiply dequantized
+// weights, w4_redo computes the sums of such rows once more as those kernels do.
+//
 // Rows: dense (tile y is rows 16 y ..) or an expert tile table of 16-row entries with x rows
 // gathered through the slot permutation. Two weight matrices of one shape (gate and up) may be
 // walked as one: column tiles past the first matrix's go to the second.
@@ -50,6 +54,36 @@ struct W4StreamArgs {
   int gather;          // grouped: x row perm[slot] / 2 (else the slot), output row the slot
                        // (else perm[slot])
 };
+
+// A wave's sums in LDS (column set 8 w + nib, rows 4 g + i of lane 16 g + c) again where they are not
+// finite, over K rows [k0, k1): the x row of slot s0 + that row (by way of perm, unless null) times the
+// weights dequantized as the reference and the wide tiles do it (q - z and the product with s each rounded once), so that an infinity meets each
+// weight's sign (and a zero weight gives NaN). One K row at a time and nothing unrolled: it is rare, and
+// costs the kernel no registers.
+template <bool BF16, int NCS>
+__device__ inline void w4_redo(float* slice, int rows, const uint16_t* x, int s0, const int* perm, const uint32_t* qw,
+                               const uint16_t* sp, const uint16_t* zp, int N, int K, int group, int k0, int k1) {
+  const int lane = threadIdx.x & 63, g4 = 4 * (lane >> 4);
+  const auto round = [](float v) { return half_bits_to_f32<BF16>(f32_to_half_bits<BF16>(keep_f32(v))); };
+#pragma unroll 1
+  for (int i = 0; i < 4; ++i) {
+    if (g4 + i >= rows) break;
+    const uint16_t* xr = x + (size_t)(perm ? perm[s0 + g4 + i] >> 1 : s0 + g4 + i) * K;
+#pragma unroll 1
+    for (int cs = 0; cs < NCS; ++cs) {
+      float& t = slice[cs * kSplitKCsStride + lane * 4 + i];
+      if (__builtin_isfinite(t)) continue;
+      float v = 0.f;
+#pragma unroll 1
+      for (int k = k0; k < k1; ++k) {
+        const size_t o = (size_t)(k / group) * N + cs;
+        const float q = (float)((qw[(size_t)k * (N >> 3) + (cs >> 3)] >> (4 * (cs & 7))) & 15u);
+        v = fmaf(half_bits_to_f32<BF16>(xr[k]), round(round(q - half_bits_to_f32<BF16>(zp[o])) * half_bits_to_f32<BF16>(sp[o])), v);
+      }
+      t = v;
+    }
+  }
+}
 
 // SPG: K steps (32 rows) per quantization group: 1, 2, 4 or 8.
 template <int SPG, bool BF16, bool GROUPED>
@@ -209,12 +243,27 @@ __global__ __launch_bounds__(64 * kStreamWaves, 2) void w4_stream_kernel(W4Strea
 #pragma unroll
   for (int cs = 0; cs < NCS; ++cs) asm volatile("" : "+v"(tot[cs]));
   float* slice = a.slices + (size_t)split * a.M * a.ld + (size_t)tile * kStreamCols;
-  splitk_wave_sum<NCS, float, kbh_f32x4>(tot, sm, rows, [&](int r, int n, float v) {
+  const auto store = [&](int r, int n, float v) {
     int row = s0 + r;
     if constexpr (GROUPED)
       if (!a.gather) row = a.perm[row];
     slice[(size_t)row * a.ld + n] = v;
-  });
+  };
+  if constexpr (GROUPED) {
+    bool redo = false;
+#pragma unroll
+    for (int cs = 0; cs < NCS; ++cs)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) redo |= !__builtin_isfinite(tot[cs][i]);
+    const bool any = __any(redo);
+    splitk_wave_sum<NCS, float, kbh_f32x4>(tot, sm, rows, store, [&](float* mine) {
+      if (any)
+        w4_redo<BF16, NCS>(mine, rows, a.x, s0, a.gather ? a.perm : nullptr, qw + (n0 >> 3) + c * NW, sp, zp, N, K, a.group,
+                           cb * kStreamChunk, ce * kStreamChunk);
+    });
+  } else {
+    splitk_wave_sum<NCS, float, kbh_f32x4>(tot, sm, rows, store);
+  }
 }
 
 // Whether the kernel takes K x N matrices of this group size (32-bit buffer offsets, whole units).

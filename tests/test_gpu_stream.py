@@ -54,6 +54,49 @@ def test_ffn_stream(dev, counts, D, F, group, dtype):
     assert torch.equal(y, ops.qmoe_ffn(*[t.to(dev) for t in ins]))
 
 
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("group", [32, 128])
+def test_ffn_stream_non_finite(dev, dtype, group):
+    """Infinities and NaN in x, and a column of h that leaves the type's range: the streamed rows agree
+    with the same tokens in a batch on the wide tiles, sign by sign (an infinity in one column of h meets each
+    down weight's sign), and the other rows are the same bits as without the values in x."""
+    E, D, F, T = 4, 512, 768, 20
+    ins = inputs.qmoe_ffn(64, D, F, E, group=group, dtype=dtype, seed=9)
+    ins[6][:, :, 100] *= 2.0 ** 17           # up scales: h[:, 100] is past 65504 in many rows
+    clean = [t.to(dev) for t in ins]
+    x = ins[0].clone()
+    big = torch.finfo(dtype).max
+    x[1, 17] = float("inf")
+    x[3, 5], x[3, 300] = float("inf"), float("-inf")
+    x[4, 100] = float("nan")
+    x[6, :] = x[6, :] * (1.5 if dtype == F16 else 2e18)      # bf16: past 3.4e38 in that column alone
+    x[9, :] = x[9, :] * (1.5 if dtype == F16 else 2e18)
+    x[7, 200] = -big
+    x[8, 40], x[8, 41] = 0.9 * big, 0.9 * big
+    x[13, D - 1] = float("-inf")
+    dirty = [x.to(dev)] + clean[1:]
+    few = lambda d: [d[0][:T].contiguous(), d[1][:T].contiguous(), *d[2:]]
+    assert 2 * T < 32 * E <= 2 * 64    # streamed, and on the wide tiles
+    got, want = ops.qmoe_ffn(*few(dirty)).float(), ops.qmoe_ffn(*dirty)[:T].float()
+    assert torch.isnan(want).any() and torch.isinf(want).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert torch.equal(torch.isinf(got), inf) and torch.equal(got[inf], want[inf])
+    fin = torch.isfinite(want)
+    # The wide tiles' weights are rounded to the type (2^-11 / 2^-8 of each, so of a column's sum of typical
+    # size, not of a sum that cancels), and h and o once on both sides: 2^-8 / 2^-5 of the largest output
+    # of the rows of natural size, or of the row.
+    eps = 2.0 ** -8 if dtype == F16 else 2.0 ** -5
+    scale = torch.where(fin, want, 0).abs().amax(dim=1, keepdim=True)
+    natural = [r for r in range(T) if r not in (6, 9)]
+    scale = torch.maximum(scale, scale[natural].max())
+    assert ((got - want).abs()[fin] <= (eps * scale.expand_as(want))[fin]).all()
+    touched = torch.tensor([1, 3, 4, 6, 7, 8, 9, 13])
+    same = torch.ones(T, dtype=torch.bool)
+    same[touched] = False
+    assert torch.equal(got.cpu()[same].nan_to_num(), ops.qmoe_ffn(*few(clean)).float().cpu()[same].nan_to_num())
+
+
 def test_ffn_stream_full_width(dev):
     """The benchmark's layer (D=4096, F=14336, E=8) at 9 tokens, the last 256 output columns."""
     ins = inputs.qmoe_ffn(T=9, seed=5)
