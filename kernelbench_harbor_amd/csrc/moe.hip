@@ -744,7 +744,7 @@ struct SiluPairOut {
 template <bool BF16>
 __global__ __launch_bounds__(256) void moe_reduce_combine_kernel(
     const float* __restrict__ part, int splits, const uint16_t* __restrict__ topw,
-    uint16_t* __restrict__ y, int T, int N) {
+    uint16_t* __restrict__ y, int T, int N, int ldy) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   const size_t n4 = (size_t)T * N / 4;
   if (i >= n4) return;
@@ -767,15 +767,15 @@ __global__ __launch_bounds__(256) void moe_reduce_combine_kernel(
   kbh_u32x2 o;
   o[0] = (uint32_t)r[0] | ((uint32_t)r[1] << 16);
   o[1] = (uint32_t)r[2] | ((uint32_t)r[3] << 16);
-  *reinterpret_cast<kbh_u32x2*>(y + e) = o;
+  *reinterpret_cast<kbh_u32x2*>(y + (size_t)t * ldy + n) = o;
 }
 
 // h[s][n] = dtype(silu(g) * u) with g and u the sums, in split order, of columns n and F + n of the
-// slices [splits][S][2F] (the streaming kernel's gate/up partial sums; fp32 math, one rounding).
-// Four columns per thread.
+// slices [splits][S][2F] (the streaming kernel's gate/up partial sums; fp32 math, one rounding); ldh:
+// the row stride of h. Four columns per thread.
 template <bool BF16>
 __global__ __launch_bounds__(256) void moe_silu_sum_kernel(const float* __restrict__ part, int splits,
-                                                           uint16_t* __restrict__ h, int S, int F) {
+                                                           uint16_t* __restrict__ h, int S, int F, int ldh) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= (size_t)S * F / 4) return;
   const size_t s = 4 * i / (size_t)F, n = 4 * i - s * F;
@@ -788,7 +788,7 @@ __global__ __launch_bounds__(256) void moe_silu_sum_kernel(const float* __restri
   kbh_u32x2 o;
   o[0] = (uint32_t)r[0] | ((uint32_t)r[1] << 16);
   o[1] = (uint32_t)r[2] | ((uint32_t)r[3] << 16);
-  *reinterpret_cast<kbh_u32x2*>(h + s * F + n) = o;
+  *reinterpret_cast<kbh_u32x2*>(h + s * ldh + n) = o;
 }
 
 // FFN on the streaming kernel (w4_stream.h), below 32 routed rows per expert on average: 16-row
@@ -799,8 +799,11 @@ __global__ __launch_bounds__(256) void moe_silu_sum_kernel(const float* __restri
 // rate of a large copy). Each 16-row tile past an expert's first costs its conversion again; the
 // line at 32 rows is where the 128-row tiles' measured cost is met within the range tested (1.36x
 // at 127 tokens). Both GEMMs leave fp32 slices, K split for the tiles the batch can reach.
+// The slices of a pass are at most kWideMaxSliceBytes, as those of the wide tiles: larger batches (of many
+// experts: E=64 F=14336 T=1000 makes 230 MB of them) take the columns in several passes over the same rows.
 struct FfnStream {
   int s1, s2;  // K splits of gate/up and of down
+  int c1, c2;  // columns of a pass (of gate and up each; of down)
 };
 bool plan_ffn_stream(int T, int E, int D, int F, int group, FfnStream* p) {
   if ((size_t)2 * T >= (size_t)32 * E) return false;
@@ -808,6 +811,13 @@ bool plan_ffn_stream(int T, int E, int D, int F, int group, FfnStream* p) {
   const int reach = 2 * T < E ? 2 * T : E;  // experts the batch can reach
   p->s1 = w4_stream_splits(2 * T, F, D, group, reach, 2);
   p->s2 = w4_stream_splits(2 * T, D, F, group, reach, 1);
+  // passes of equal whole column tiles
+  const auto columns = [](size_t column_bytes, int N) {
+    const size_t passes = (column_bytes * N + kWideMaxSliceBytes - 1) / kWideMaxSliceBytes, tiles = N / kStreamCols;
+    return (int)((tiles + passes - 1) / passes) * kStreamCols;
+  };
+  p->c1 = columns((size_t)p->s1 * 2 * T * 2 * 4, F);
+  p->c2 = columns((size_t)p->s2 * 2 * T * 4, D);
   return true;
 }
 
@@ -1013,7 +1023,7 @@ void launch_ffn_wide_spg(const FfnPlan& fp, const MoeLayout& L, const MoeBuffers
     if (splits > 1) {
       const size_t n4 = (size_t)T * D / 4;
       hipLaunchKernelGGL((moe_reduce_combine_kernel<BF16>), dim3((unsigned)((n4 + 255) / 256)),
-                         dim3(256), 0, st, part, splits, mb.topw, (uint16_t*)y, T, D);
+                         dim3(256), 0, st, part, splits, mb.topw, (uint16_t*)y, T, D, D);
     } else {
       launch_combine<BF16>(o, mb.topw, y, T, D, st);
     }
@@ -1057,39 +1067,47 @@ void launch_ffn_stream(const FfnStream& fs, const MoeLayout& L, const MoeBuffers
                        void* y, int T, int D, int F, int group, size_t gq, size_t gs, size_t dq,
                        size_t ds, hipStream_t st) {
   const int S = 2 * T;
+  const auto at = [](const W4Mat& m, int n) { return W4Mat{m.qw + n / 8, m.scales + n, m.zeros + n}; };
   W4StreamArgs a;
   a.x = (const uint16_t*)x;
-  a.mat[0] = gate;
-  a.mat[1] = up;
   a.slices = part;
   a.tiles = mb.tiles;
   a.perm = mb.perm;
   a.q_stride = gq;
   a.s_stride = gs;
   a.M = S;
-  a.ld = 2 * F;
   a.N = F;
   a.K = D;
   a.group = group;
   a.splits = fs.s1;
-  a.tiles0 = F / kStreamCols;
   a.gather = 1;
-  launch_w4_stream<BF16, true>(a, 2 * F / kStreamCols, L.max_tiles, st);
-  hipLaunchKernelGGL((moe_silu_sum_kernel<BF16>), dim3((unsigned)(((size_t)S * F / 4 + 255) / 256)),
-                     dim3(256), 0, st, (const float*)part, fs.s1, (uint16_t*)h, S, F);
+  for (int n = 0; n < F; n += fs.c1) {
+    const int cols = min(fs.c1, F - n);
+    a.mat[0] = at(gate, n);
+    a.mat[1] = at(up, n);
+    a.ld = 2 * cols;
+    a.tiles0 = cols / kStreamCols;
+    launch_w4_stream<BF16, true>(a, 2 * cols / kStreamCols, L.max_tiles, st);
+    hipLaunchKernelGGL((moe_silu_sum_kernel<BF16>), dim3((unsigned)(((size_t)S * cols / 4 + 255) / 256)),
+                       dim3(256), 0, st, (const float*)part, fs.s1, (uint16_t*)h + n, S, cols, F);
+  }
   a.x = (const uint16_t*)h;
-  a.mat[0] = a.mat[1] = down;
   a.q_stride = dq;
   a.s_stride = ds;
-  a.ld = a.N = D;
+  a.N = D;
   a.K = F;
   a.splits = fs.s2;
-  a.tiles0 = D / kStreamCols;
   a.gather = 0;
-  launch_w4_stream<BF16, true>(a, D / kStreamCols, L.max_tiles, st);
-  hipLaunchKernelGGL((moe_reduce_combine_kernel<BF16>),
-                     dim3((unsigned)(((size_t)T * D / 4 + 255) / 256)), dim3(256), 0, st,
-                     (const float*)part, fs.s2, mb.topw, (uint16_t*)y, T, D);
+  for (int n = 0; n < D; n += fs.c2) {
+    const int cols = min(fs.c2, D - n);
+    a.mat[0] = a.mat[1] = at(down, n);
+    a.ld = cols;
+    a.tiles0 = cols / kStreamCols;
+    launch_w4_stream<BF16, true>(a, cols / kStreamCols, L.max_tiles, st);
+    hipLaunchKernelGGL((moe_reduce_combine_kernel<BF16>),
+                       dim3((unsigned)(((size_t)T * cols / 4 + 255) / 256)), dim3(256), 0, st,
+                       (const float*)part, fs.s2, mb.topw, (uint16_t*)y + n, T, cols, D);
+  }
 }
 
 // FFN layout: TM-row tiles (the plan's) and room for the down projection's split-K partials when the wide
@@ -1099,7 +1117,7 @@ MoeLayout ffn_layout(int T, int E, int D, int F, int group, bool* wide, FfnPlan*
   *wide = false;
   *stream = plan_ffn_stream(T, E, D, F, group, fs);
   if (*stream) {  // the down projection's slices reuse the gate/up ones' place
-    const size_t gu = (size_t)fs->s1 * 2 * T * 2 * F * 4, dn = (size_t)fs->s2 * 2 * T * D * 4;
+    const size_t gu = (size_t)fs->s1 * 2 * T * 2 * fs->c1 * 4, dn = (size_t)fs->s2 * 2 * T * fs->c2 * 4;
     return moe_layout(T, E, F, 0, 16, gu > dn ? gu : dn);
   }
   // The wide path stages x (T x D) and h (2T x F) through LDS with 32-bit buffer offsets, so it

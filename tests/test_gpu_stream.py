@@ -97,6 +97,23 @@ def test_ffn_stream_non_finite(dev, dtype, group):
     assert torch.equal(got.cpu()[same].nan_to_num(), ops.qmoe_ffn(*few(clean)).float().cpu()[same].nan_to_num())
 
 
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("D,F", [(256, 5376), (8448, 256)])
+def test_ffn_stream_passes(dev, D, F, dtype):
+    """Slices past 64 MiB: two passes over the columns (11 and 10 tiles of gate/up, 17 and 16 of down)."""
+    T, E = 1000, 64
+    ins = inputs.qmoe_ffn(T, D, F, E, group=128, dtype=dtype, seed=2)
+    assert 2 * T * (2 * F if F > D else D) * 4 > 64 << 20
+    d = [t.to(dev) for t in ins]
+    y = ops.qmoe_ffn(*d)
+    a = _np(ins)
+    rows = np.r_[0:24, T - 24:T]
+    cmp = compare(y[torch.from_numpy(rows).to(dev)], oq.ffn_forward(a[0][rows], a[1][rows], *a[2:]))
+    assert cmp.ok, cmp
+    ops.scratches.get(0, dev).fill_(255)   # no content requirement on the workspace
+    assert torch.equal(y, ops.qmoe_ffn(*d))
+
+
 def test_ffn_stream_full_width(dev):
     """The benchmark's layer (D=4096, F=14336, E=8) at 9 tokens, the last 256 output columns."""
     ins = inputs.qmoe_ffn(T=9, seed=5)

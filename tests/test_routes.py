@@ -76,3 +76,9 @@ def test_w4a16_128_column_tiles(lib, M, K, N, group, kernel):
     (16, 11008, 4096, _lib.KBH_KERNEL_STREAM), (17, 3584, 18944, 64), (16, 4096, 14336, _lib.KBH_KERNEL_DECODE)])
 def test_fp8w_streaming_kernel(lib, M, K, N, kernel):
     assert lib.kbh_fp8w_kernel(M, N, K, 128, None) == kernel
+
+
+@pytest.mark.parametrize("T,D,F,E", [(127, 4096, 14336, 8), (500, 4096, 14336, 64), (1000, 4096, 14336, 64), (4000, 7168, 2048, 256)])
+def test_ffn_stream_slices_are_bounded(lib, T, D, F, E):
+    """Streamed batches: h, at most 64 MiB of slices, and tables of a few words per token and expert."""
+    assert lib.kbh_qmoe_ffn_workspace_bytes(T, D, F, E) <= 2 * T * F * 2 + (64 << 20) + 256 * (T + E)
