@@ -852,6 +852,9 @@ bool plan_ffn(int T, int E, int D, int F, int group, FfnPlan* p) {
 }
 
 // ---- host side ------------------------------------------------------------------------------
+// Row tile of the grouped kernels: 128 when an expert averages more than 48 rows, else 64.
+int moe_row_tile(long slots, int E) { return slots / (E > 0 ? E : 1) > 48 ? 128 : 64; }
+
 struct MoeLayout {
   size_t topi, topw, slot_of, perm, tiles, h, o, part, topw32, total;
   int bm, max_tiles, topk;
@@ -865,7 +868,7 @@ MoeLayout moe_layout(int T, int E, int hidden, int out_cols, int bm = 0, size_t 
   MoeLayout L;
   const size_t S = (size_t)topk * T;
   L.topk = topk;
-  L.bm = bm ? bm : ((int)S / (E > 0 ? E : 1) > 48 ? 128 : 64);
+  L.bm = bm ? bm : moe_row_tile((long)S, E);
   L.max_tiles = (int)((S + L.bm - 1) / L.bm) + E;
   size_t o = 0;
   auto take = [&](size_t bytes) {
@@ -939,19 +942,31 @@ void launch_moe_gemm(const MoeLayout& L, const void* A, int lda, const MoeBuffer
 constexpr int kQMoeUnit = 8;
 
 // K splits of the reference qMoE op's grouped GEMM at small batches, where the experts a batch can
-// reach times the column tiles leave CUs idle and a workgroup walks all of K alone at ~0.5 us per
-// slab: the smallest split of K's units that makes 384 workgroups (fp32 slices, at most 16 MiB,
-// summed by the combine). D=2048 N=1408 E=64 T=1 / 8 / 16 32.6 / 34.7 / 39.3 -> 22.4 / 27.4 / 34.8 us,
-// D=4096 N=14336 E=8 T=1 49.4 -> 44.0. The fp16/bf16 MoE, whose combine must round every expert
-// output, did not gain (D=4096 H=14336 T=1 53 -> 74 us).
+// reach times the column tiles leave CUs idle and a workgroup walks all of K alone, at 0.27 us per slab
+// (64-row tiles; 0.35 with 128 rows): the split of K's units, up to the smallest that makes 384 workgroups,
+// that saves most of the walk over what it costs, measured as 2 us (3 with 128-row tiles) and 0.45 us per MB
+// more of fp32 slices written and summed by the combine (they are at most 16 MiB). D=2048 N=1408 E=64 T=1 / 8 / 16 32.1 / 34.7 /
+// 41.8 -> 19.8 / 26.1 / 33.8 us, D=4096 N=1024 E=8 T=64 48.5 -> 27.5; without the cost D=1024 N=2048 E=8 T=192
+// was split, 26.3 -> 29.8, and N=1024 T=1024, 38.2 -> 41.1. The fp16/bf16 MoE, whose combine must round every
+// expert output, did not gain (D=4096 H=14336 T=1 53 -> 74 us).
 int moe_splits(int T, int E, int D, int N) {
   const int slabs = D / TBK;
   if (slabs <= 0 || slabs % kQMoeUnit != 0) return 1;
   const long S = 2L * T;
   const long wgs = (S < E ? S : E) * (N / 128);
-  int best = 1;
-  for (int s = 1; s <= slabs / kQMoeUnit && wgs * best < 384; ++s)
-    if ((slabs / kQMoeUnit) % s == 0 && (size_t)s * S * N * 4 <= ((size_t)16 << 20)) best = s;
+  const bool tall = moe_row_tile(S, E) == 128;
+  const float walk = (float)slabs * (tall ? 0.35f : 0.27f), fixed = tall ? 3.0f : 2.0f;
+  int best = 1, last = 1;
+  float most = 0.f;
+  for (int s = 2; s <= slabs / kQMoeUnit && wgs * last < 384; ++s) {
+    if ((slabs / kQMoeUnit) % s != 0 || (size_t)s * S * N * 4 > ((size_t)16 << 20)) continue;
+    last = s;
+    const float saved = walk * (1.0f - 1.0f / (float)s) - fixed - 0.45f * (float)(s - 1) * (float)S * (float)N * 8e-6f;
+    if (saved > most) {
+      most = saved;
+      best = s;
+    }
+  }
   return best;
 }
 

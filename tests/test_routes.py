@@ -82,3 +82,11 @@ def test_fp8w_streaming_kernel(lib, M, K, N, kernel):
 def test_ffn_stream_slices_are_bounded(lib, T, D, F, E):
     """Streamed batches: h, at most 64 MiB of slices, and tables of a few words per token and expert."""
     assert lib.kbh_qmoe_ffn_workspace_bytes(T, D, F, E) <= 2 * T * F * 2 + (64 << 20) + 256 * (T + E)
+
+
+# T, D, N, E, whether K is split (fp32 slices next to the one [2T, N] of outputs)
+@pytest.mark.parametrize("T,D,N,E,split", [(1024, 1024, 1024, 8, False), (512, 1024, 1024, 8, False), (192, 1024, 2048, 8, False), (384, 1024, 1024, 16, False),
+                                           (1, 2048, 1408, 64, True), (16, 2048, 1408, 60, True), (512, 4096, 1024, 8, True), (256, 4096, 14336, 8, False)])
+def test_qmoe_split_only_where_it_pays(lib, T, D, N, E, split):
+    slices = lib.kbh_qmoe_workspace_bytes(T, D, N, E) // (2 * T * N * 4)
+    assert (slices > 1) == split
