@@ -121,7 +121,8 @@ int kbh_w4a16_gemm_noalloc(const void* x, const int32_t* qweight, const void* sc
  * Requirements: M >= 1, N % 128 == 0, K % 64 == 0, x/w/y 16-byte aligned.
  * workspace / scratch: as for kbh_w4a16_gemm, with kbh_w8a8_workspace_bytes() and
  * kbh_w8a8_scratch_bytes(). From 17 rows a call uses the scratch where the query asks for some; up
- * to 32 rows (127 where N is no multiple of 256) the workspace alone is enough, on a slower kernel.
+ * to 32 rows, and at any number where N is no multiple of 256, the workspace alone is enough, on a
+ * slower kernel.
  */
 size_t kbh_w8a8_workspace_bytes(int M, int N, int K);
 size_t kbh_w8a8_scratch_bytes(int M, int N, int K);

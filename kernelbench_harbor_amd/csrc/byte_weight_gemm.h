@@ -563,11 +563,14 @@ int byte_gemm_run(const void* x, const void* w, const void* scales, void* y, voi
                   bool defer_sum = false, int* splits_out = nullptr, SIDE side = SIDE{}) {
   if (splits_out) *splits_out = 1;
   ByteWide wide;
-  if (plan_byte_wide(M, N, K, block, &wide)) {
+  bool is_wide = plan_byte_wide(M, N, K, block, &wide);
+  if (is_wide) {  // without room for the slices, the kernels that ran the call before the wide tiles
+    const size_t need = wide_workspace_bytes(M, N, wide.plan.splits);
+    is_wide = need == 0 || (workspace && workspace_bytes >= need);
+  }
+  if (is_wide) {
     const int splits = wide.plan.splits;
-    const size_t need = wide_workspace_bytes(M, N, splits);
-    if (need > 0 && (!workspace || workspace_bytes < need)) return KBH_ERR_WORKSPACE;
-    if (need > 0 && !aligned16(workspace)) return KBH_ERR_ALIGN;
+    if (splits > 1 && !aligned16(workspace)) return KBH_ERR_ALIGN;
     float* slices = (float*)workspace;
     switch (wide.spg) {
       case 1: launch_byte_wide<BF16, DEC, 1>(wide, x, w, scales, y, slices, M, N, K, block, st); break;

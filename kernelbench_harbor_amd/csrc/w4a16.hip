@@ -399,6 +399,13 @@ bool plan_w4_wide(int M, int N, int K, int group, bool bf16, W4Wide* w) {
   return !(ws && M < kTiledMinM && K % (64 * unit) != 0 && w4_decode_stays(M, N, K, group, bf16, w->plan));
 }
 
+// Calls of the wide tiles that needed no scratch before those took them (K that ends in half an
+// iteration, more than 128 rows of N of 128 mod 256): without scratch they keep the LDS-staged or, on the
+// workspace, the decode kernel.
+bool w4_scratch_free(int M, int N, int K, int spg) {
+  return (M > 128 && N % 256 != 0) || K % (32 * wide_iteration(spg, w4_wide_pd(N % 256 == 0 ? 256 : 128))) != 0;
+}
+
 // Scratch of the wide kernels, for either dtype (the query does not name it): the larger plan's.
 size_t w4_wide_scratch_bytes(int M, int N, int K, int group) {
   size_t best = 0;
@@ -556,10 +563,17 @@ extern "C" int kbh_w4a16_gemm(const void* x, const int32_t* qweight, const void*
   hipStream_t st = (hipStream_t)stream;
 
   W4Wide wide;
-  if (plan_w4_wide(M, N, K, group, bf, &wide)) {
+  bool is_wide = plan_w4_wide(M, N, K, group, bf, &wide);
+  if (is_wide) {
     const size_t need = wide_workspace_bytes(M, N, wide.plan.splits);
-    if (need > 0 && (!scratch || scratch_bytes < need)) return KBH_ERR_WORKSPACE;
-    if (need > 0 && !aligned16(scratch)) return KBH_ERR_ALIGN;
+    if (need > 0 && (!scratch || scratch_bytes < need)) {
+      if (!w4_scratch_free(M, N, K, wide.spg)) return KBH_ERR_WORKSPACE;
+      is_wide = false;
+    } else if (need > 0 && !aligned16(scratch)) {
+      return KBH_ERR_ALIGN;
+    }
+  }
+  if (is_wide) {
     if (bf) dispatch_w4_wide<true>(wide, x, qweight, scales, zeros, y, (float*)scratch, M, N, K, group, st);
     else dispatch_w4_wide<false>(wide, x, qweight, scales, zeros, y, (float*)scratch, M, N, K, group, st);
     return launch_status();

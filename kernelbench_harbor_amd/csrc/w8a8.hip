@@ -427,15 +427,23 @@ int w8a8_run(const void* x, const void* w, const void* xs, const void* wsc, void
   WidePlan wp;
   W8Plan p;
   bool wide = plan_w8_wide(M, N, K, &wp);
-  if (wide && w8_decode_range(M, N) && plan_w8_decode(M, N, K, &p)) {
-    const size_t sc = wide_workspace_bytes(M, N, wp.splits), need = splitk_workspace_bytes(M, N, p.splits);
-    const bool scratch_ok = sc == 0 || (scratch && scratch_bytes >= sc);
-    if (!scratch_ok && (need == 0 || (workspace && workspace_bytes >= need))) wide = false;
-  }
   if (wide) {
     const size_t need = wide_workspace_bytes(M, N, wp.splits);
-    if (need > 0 && (!scratch || scratch_bytes < need)) return KBH_ERR_WORKSPACE;
-    if (need > 0 && !aligned16(scratch)) return KBH_ERR_ALIGN;
+    if (need > 0 && (!scratch || scratch_bytes < need)) {
+      // Calls that needed no scratch before the wide tiles took them keep the kernels that ran them.
+      if (w8_decode_range(M, N)) {
+        wide = !plan_w8_decode(M, N, K, &p);
+        const size_t dec = wide ? 0 : splitk_workspace_bytes(M, N, p.splits);
+        wide |= dec > 0 && (!workspace || workspace_bytes < dec);
+      } else {
+        wide = N % 256 == 0 || K % (WBK * WDEPTH) != 0;
+      }
+      if (wide) return KBH_ERR_WORKSPACE;
+    } else if (need > 0 && !aligned16(scratch)) {
+      return KBH_ERR_ALIGN;
+    }
+  }
+  if (wide) {
     const bool pd4 = w8_wide_pd(K) == 4;
     if (wp.tm == 128) {
       if (pd4) launch_w8_wide<OUT_I32, 128, 4>(wp, x, w, xs, wsc, out, (int*)scratch, M, N, K, st);

@@ -43,6 +43,37 @@ def test_w8a8_without_scratch(dev, M, K, N):
                                  M, N, K, st) == _lib.KBH_ERR_WORKSPACE
 
 
+# rows, K, N whose W8A8, W4A16 and FP8 calls take slices on the wide tiles and ran without before them
+@pytest.mark.parametrize("M,K,N", [(300, 2048, 384), (129, 4096, 640)])
+def test_calls_without_scratch(dev, M, K, N):
+    """More than 128 rows of N of 128 mod 256 are accepted without scratch (and FP8 calls without a workspace),
+    on the LDS-staged kernels; N a multiple of 256 is refused as before (W4A16, W8A8)."""
+    lib = _lib.load()
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib.kbh_w8a8_scratch_bytes(M, N, K) > 0 and lib.kbh_w4a16_scratch_bytes(M, N, K, 128) > 0
+    x, w = _int8(M, K, N, seed=M)
+    xd, wd = x.to(dev), w.to(dev)
+    acc = torch.empty(M, N, dtype=torch.int32, device=dev)
+    call = lambda n: lib.kbh_w8a8_gemm_i32(xd.data_ptr(), wd.data_ptr(), acc.data_ptr(), None, 0, None, 0, M, n, K, st)
+    assert call(N) == 0
+    assert np.array_equal(acc.cpu().numpy().astype(np.float64), x.double().numpy() @ w.double().numpy())
+    assert call(256) == _lib.KBH_ERR_WORKSPACE
+    x, q, s, z = inputs.w4a16(M, K, N, 128, F16, seed=M)
+    d = [t.to(dev) for t in (x, q, s, z)]
+    y = torch.empty(M, N, dtype=F16, device=dev)
+    call = lambda n: lib.kbh_w4a16_gemm(*[t.data_ptr() for t in d], y.data_ptr(), None, 0, None, 0, M, n, K, 128, 0, st)
+    assert call(N) == 0
+    cmp = compare(y, ow.forward(x.float().numpy(), q.numpy(), s.float().numpy(), z.float().numpy()))
+    assert cmp.ok, cmp
+    assert call(256) == _lib.KBH_ERR_WORKSPACE
+    x, w, s = inputs.fp8w(M, K, N, 128, F16, seed=M)
+    d = [t.to(dev) for t in (x, w, s)]
+    assert lib.kbh_fp8w_workspace_bytes(M, N, K, 128) > 0
+    assert lib.kbh_fp8w_gemm(*[t.data_ptr() for t in d], y.data_ptr(), None, 0, M, N, K, 128, 0, st) == 0
+    cmp = compare(y, of.forward(x.float().numpy(), w.view(torch.uint8).numpy(), s.float().numpy()))
+    assert cmp.ok, cmp
+
+
 def _w4a16(dev, M, K, N, group, dtype, kernel, cols):
     assert _lib.load().kbh_w4a16_kernel(M, N, K, group, DT[dtype], None) == kernel
     x, q, s, z = inputs.w4a16(M, K, N, group, dtype, seed=M + K)
