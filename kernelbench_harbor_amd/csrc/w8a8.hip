@@ -364,10 +364,10 @@ bool w8_x_staged(int M, int K) { return (size_t)(M + 256) * K < ((size_t)1 << 31
 // take it where no scratch is given.
 bool w8_decode_range(int M, int N) { return M <= 32 || (M < kW8TiledMinM && N % 256 != 0); }
 
-// Whether the decode kernel keeps a call of that range. It streams the weights once per 16-row block:
-// always while its grid is resident at once (two workgroups per CU: 1024 x 1024 .. 8192 x 1152 at 33 to
-// 127 rows 8-16 us against 14-20), and beyond where its estimated time is at most 3% over the wide
-// plan's, 25% in the second round of full workgroups whose splits are a power of two (the fit has those
+// Whether the decode kernel keeps a call of that range past one round of workgroups. It streams the weights
+// once per 16-row block, and plan_w8_wide keeps it always while its grid is resident at once (two workgroups
+// per CU: 1024 x 1024 .. 8192 x 1152 at 33 to 127 rows 8-16 us against 14-20); beyond that where its estimated
+// time is at most 3% over the wide plan's, 25% in the second round of full workgroups whose splits are a power of two (the fit has those
 // too slow: 8192 x 1408 M=127 16.2 us against 20.3). Both estimates (us) are least-squares fits to 2000
 // calls of 17 to 127 rows over K from 1024 to 14336 and N from 384 to 14464 (decode 7.6%, wide 5.1%
 // rms): the choice is 0.7% from the faster kernel on average past 512 workgroups; 7 of those calls are
@@ -375,7 +375,6 @@ bool w8_decode_range(int M, int N) { return M <= 32 || (M < kW8TiledMinM && N % 
 // up to 79%: K=2048 N=1408 M=48 9.0 -> 15.0 us).
 bool w8_decode_stays(int M, int N, const W8Plan& d, const WidePlan& w) {
   const int grid = d.ntiles * d.splits * d.mblocks;
-  if (grid <= 512) return true;
   float dec = 5.3f + 4.37f * (float)grid * (float)(d.waves * d.spw) / 4096.0f + 1.27f * (float)((grid + 511) / 512);
   if (d.splits > 1) dec += 0.16f + 0.064f * d.splits + 0.164f * ((float)d.splits * M * N * 8.0f / (float)(1 << 20));
   const bool full = grid <= 768 && d.waves == 8 && d.splits >= 4 && (d.splits & (d.splits - 1)) == 0;
@@ -386,11 +385,13 @@ bool w8_decode_stays(int M, int N, const W8Plan& d, const WidePlan& w) {
 // estimate.
 bool plan_w8_wide(int M, int N, int K, WidePlan* p) {
   if (M < kW8WideMinM || N < 256) return false;
+  W8Plan d;
+  const bool decode = w8_decode_range(M, N) && plan_w8_decode(M, N, K, &d);
+  if (decode && d.ntiles * d.splits * d.mblocks <= 512) return false;
   // slabs per unit of K: the 128-row kernel's iteration; half of the 12-wave kernel's
   const int unit256 = w8_x_staged(M, K) ? 2 : w8_wide_pd(K);
   if (!plan_wide(M, N, K, 256, 64, w8_wide_pd(K), unit256, 256, kInt8Costs, p)) return false;
-  W8Plan d;
-  return !(w8_decode_range(M, N) && plan_w8_decode(M, N, K, &d) && w8_decode_stays(M, N, d, *p));
+  return !(decode && w8_decode_stays(M, N, d, *p));
 }
 
 template <bool OUT_I32, int TM, int PD>
