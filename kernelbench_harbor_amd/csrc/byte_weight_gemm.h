@@ -253,9 +253,9 @@ __device__ inline uint32_t byte_pair_dequant(uint32_t a, uint32_t b, uint16_t s)
 // (chunk i + 1's loads go out before chunk i's MFMAs, 8 to 16 KB per wave in flight), 4 waves and
 // 33 KB of LDS per workgroup, so that all the workgroups of the plan are resident together and
 // stream until their K range ends, with fewer slices. Two-row pairs come from v_perm_b32 as in
-// ByteWidePolicy. HBM bound; e4m3 x fp16, back to back on rotating weights: 3584 x 18944 M=1 / 16 18.3 /
-// 21.2 -> 16.9 / 20.3 us, 18944 x 3584 19.9 / 24.6 -> 17.9 / 19.7, 28672 x 8192 M=16 59.0 -> 48.0
-// (235 MB at 4.9 TB/s).
+// ByteWidePolicy. HBM bound; e4m3 x fp16, back to back on rotating weights, against the decode kernel: 3584 x
+// 18944 M=1 / 16 19.4 / 22.1 -> 17.7 / 20.8 us, 18944 x 3584 20.4 / 25.3 -> 19.2 / 20.7, 28672 x 8192 M=16
+// 58.0 -> 48.3 (235 MB at 4.9 TB/s), 11008 x 4096 17.9 / 24.4 -> 14.0 / 15.6.
 constexpr int kByteStreamWaves = 4;
 constexpr int kByteStreamChunk = 64;  // K rows (two MFMA steps)
 
@@ -349,7 +349,8 @@ __global__ __launch_bounds__(64 * kByteStreamWaves, 3) void byte_stream_kernel(
 
 // Weight producer of the warp-specialised kernels (32 rows x 256 columns per slab). Thread t owns
 // rows 4rb .. 4rb+3 of columns 8cb .. 8cb+7 (the F16WidePolicy / W8WidePolicy thread map, whose
-// LDS writes are bank-conflict free): four 8-byte loads, and per column its 4 consecutive K values
+// 8-byte LDS writes are bank-conflict free; the 4-byte ones of two producer sets are not, 12 k cycles per
+// workgroup at bf16 M=300 K=14336 N=4096, and still gain by the second set): four 8-byte loads, and per column its 4 consecutive K values
 // as one 8-byte piece of the K-contiguous operand layout (wide_b_offset). The two-row pairs come
 // straight from v_perm_b32 on two rows (no 4x4 byte transpose): the e4m3 conversions take either
 // 16-bit half of a dword.

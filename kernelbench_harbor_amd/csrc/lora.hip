@@ -7,8 +7,8 @@
 //   base = dtype(x @ W)                                              [T, N]      (:13)
 //   lo   = dtype(x[t] @ A[id_t])                                     [T, r]      (:14-15)
 //   y    = dtype(base + dtype(lo[t] @ B[id_t]))                      [T, N]      (:16-17)
-// Two launches up to 32 rows, three above: the base GEMM is the byte-weight GEMM of
-// byte_weight_gemm.h with the int8 decoder (its split-K slices left in the workspace, or base
+// Two launches up to 32 rows where the base GEMM takes the decode kernel, else three: the base GEMM is
+// the byte-weight GEMM of byte_weight_gemm.h with the int8 decoder (its split-K slices left in the workspace, or base
 // written into y when K is not split); LoraShrink computes fp32 partial sums of x[t] @ A[id] over
 // DS ranges of D (T x DS workgroups, so that a few tokens still fill the chip), as further
 // workgroups of the decode kernel's launch (its reads of A run beside the weight stream, and a

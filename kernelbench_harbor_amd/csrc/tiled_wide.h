@@ -526,8 +526,8 @@ struct WideCosts {
 // MI355X over K x N = 4096 x {4096, 6144, 14336}, 14336 x 4096, 3584 x 18944, 18944 x 3584, 8192 x
 // {28672, 29568} and 28672 x 8192 at M = 64 .. 2048 (W4A16 group 128; FP8 weights fit the same
 // within 0.1%): the plan it picks is 0.7% from the sweep's fastest on average, where rounds times
-// slabs with the same slices lost 3.4% (4096 x 4096 M=512 42.9 -> 34.1 us, 4096 x 14336 M=320 73.5
-// -> 60.9, 4096 x 6144 M=512 50.5 -> 43.4).
+// slabs with the same slices lost 3.4% (4096 x 4096 M=512 43 -> 34.3 us, 4096 x 14336 M=300 72.3 ->
+// 61.4, 4096 x 6144 M=512 46.5 -> 43.6).
 constexpr WideCosts kHalfCosts{{2.98f, 0.335f, 0.f, 0.f}, {3.15f, 0.32f, 0.179f, 0.f}, {4.78f, 0.437f, 0.389f, 0.f},
                                0.231f, 0.93f, 1.f};
 // bf16 weights cost the producers about 0.07 us more per slab (K=14336 N=4096 M=128 33.4 against
@@ -546,7 +546,7 @@ constexpr WideCosts kInt8Costs{{0.f, 3.f, 0.f, 0.f}, {0.f, 3.f, 0.f, 0.f}, {0.f,
 // (*cost, when not null); 0 if K is no multiple of the unit. The splits are whole units, as even as
 // they come, of at least 8 slabs, and make at most two rounds more than an unsplit K. (Even splits
 // alone left K x N whose units have few divisors short of the 256 CUs or with a second round:
-// W4A16 K=3584 N=18944 M=64 41.2 -> 24.8 us, K=18944 N=3584 M=128 131 -> 33.)
+// W4A16 K=3584 N=18944 M=64 42.8 -> 27.9 us, K=18944 N=3584 M=128 133 -> 34.7.)
 inline int plan_splits(long tiles, int M, int N, int KT, int unit, int slots, const WideCost& c,
                        const WideCosts& cs, float* cost = nullptr) {
   if (KT % unit != 0) return 0;

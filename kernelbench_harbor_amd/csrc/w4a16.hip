@@ -25,8 +25,8 @@
 //    converts to the output dtype (splitk.h). Workgroup ids are remapped so that all K splits
 //    of a column tile run on one XCD.
 //
-// Larger M (M > 32): tiled_wide_gemm (tiled_wide.h) with W4WidePolicy, which dequantizes each
-// packed 32 x TN weight slab once per workgroup into LDS with the exact reference arithmetic
+// Larger M (M > 32, except where the decode kernel stays faster): tiled_wide_gemm (tiled_wide.h) with
+// W4WidePolicy, which dequantizes each packed 32 x TN weight slab once per workgroup into LDS with the exact reference arithmetic
 // ((q - z) rounded to the input dtype, times s rounded), in MFMA fragment order; x goes from
 // global memory straight into MFMA registers. Split-K partial sums use the caller's scratch.
 // Shapes it does not cover fall back to tiled_f16_gemm (256 x 128 LDS-staged tiles) or to the
