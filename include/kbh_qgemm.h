@@ -79,7 +79,7 @@ int kbh_last_hip_error(void);
  * scratch: >= kbh_w4a16_scratch_bytes(M, N, K, group) bytes (may be 0, then NULL is accepted)
  * of device memory with no content requirement (split-K partial sums of the large-M kernel,
  * never more than 64 MiB); calls that share it must be ordered like workspace. A call uses
- * either the workspace (M <= 32, and some layers up to M = 127) or the scratch, never both, so one
+ * either the workspace (M <= 32, and some layers above that) or the scratch, never both, so one
  * buffer of the larger size may be passed as both.
  */
 size_t kbh_w4a16_workspace_bytes(int M, int N, int K, int group);

@@ -357,19 +357,25 @@ struct W4Wide {
 // Prefetch depth of a wide W4 launch with tn-column tiles.
 constexpr int w4_wide_pd(int tn) { return tn == 256 ? 4 : 2; }
 
-// Whether the decode kernel keeps a call of 33 to 127 rows whose K ends in half an iteration of the wide
-// tiles (it ran all of these before the tiles took them): by the two estimates in us, least-squares
-// fits over 892 such calls (K of an odd number of 128-row groups from 384 to 11136, N from 1024 to 14336,
-// both dtypes; decode 8%, wide 4% rms). The choice is 0.2% from the faster kernel on average and 7
-// calls are 4% or more slower than on decode, where the wide tiles alone left 441, by up to 131%
-// (K=640 N=8192 M=64 7.9 -> 12.7 us).
+// Whether the decode kernel keeps a call from 33 rows whose K ends in half an iteration of the wide tiles.
+// It ran all of these up to 127 rows before the tiles took them, and above that where K is no multiple of
+// the LDS-staged kernel's 128 rows. Two estimates in us, compared on 1601 calls timed on both kernels
+// (M 33 to 256, K from 320 to 11136, N from 1024 to 14336; fp16 and bf16 at groups of 128, fp16 alone at 64
+// and 256; decode's misses by 8% rms, the wide one's by 10%). The factor on the wide side leans to decode,
+// where a miss costs more. The choice is 0.2% from the faster kernel on average and 12 calls are more
+// than 4% slower than on decode (14% at most); the wide tiles alone had 489, by up to 131%
+// (K=896 N=8192 M=127 bf16 8.5 -> 19.6 us).
+// From 128 rows on it gives decode only short K (812 such calls of M 128 to 2048, groups of 32 and 64, both
+// dtypes: 0.48 to 0.68 of the wide tiles' time on average; 16 calls 5 to 32% slower, as they were before the tiles:
+// K=448 N=2048 M=768 bf16 15.3 -> 11.6 us, but K=2752 N=256 M=128 13.9 -> 18.3).
 bool w4_decode_stays(int M, int N, int K, int group, bool bf16, const WidePlan& w) {
   DecodePlan d;
   if (!plan_decode(M, N, K, group / 32, &d)) return false;
   if (splitk_workspace_bytes(M, N, d.splits) > KBH_W4A16_NOALLOC_SCRATCH_BYTES) return false;  // the no-alloc entry point takes the call
-  const float dec = (d.splits > 1 ? 4.75f : 2.75f) +
-                    0.84f * decode_cost(M, N, d.nw, d.spw, d.waves, d.splits, d.ntiles * d.splits * d.mblocks);
-  return dec <= 1.68f * w.cost + (w.tm == 64 ? -2.5f : -0.7f) + (w.splits > 1 ? 0.8f : 0.f) + (bf16 ? 0.4f : 0.f);
+  const int grid = d.ntiles * d.splits * d.mblocks;
+  const float dec = (d.splits > 1 ? 5.94f : 4.1f) + 0.673f * decode_cost(M, N, d.nw, d.spw, d.waves, d.splits, grid) +
+                    0.93f * (float)((grid + 255) / 256) - 0.26f * (float)d.waves;
+  return dec <= 1.05f * (1.68f * w.cost + (w.tm == 64 ? -2.5f : -0.7f) + (w.splits > 1 ? 0.8f : 0.f) + (bf16 ? 0.4f : 0.f));
 }
 
 bool plan_w4_wide(int M, int N, int K, int group, bool bf16, W4Wide* w) {
@@ -396,7 +402,8 @@ bool plan_w4_wide(int M, int N, int K, int group, bool bf16, W4Wide* w) {
   if (!plan_wide(M, N, K, w->tn, 32, unit, unit, w->tn == 128 ? 512 : 256, bf16 ? kBf16Costs : kHalfCosts,
                  &w->plan, rows64 ? 64 : 128))
     return false;
-  return !(ws && M < kTiledMinM && K % (64 * unit) != 0 && w4_decode_stays(M, N, K, group, bf16, w->plan));
+  return !(ws && (M < kTiledMinM || K % (TBK * TDEPTH) != 0) && K % (64 * unit) != 0 &&
+           w4_decode_stays(M, N, K, group, bf16, w->plan));
 }
 
 // Calls of the wide tiles that needed no scratch before those took them (K that ends in half an

@@ -53,7 +53,9 @@ def test_w8a8_many_uneven_splits(lib, M, K, N, splits):
 @pytest.mark.parametrize("M,K,N,group,dtype,kernel", [
     (64, 896, 4096, 128, _lib.KBH_F16, _lib.KBH_KERNEL_DECODE), (127, 640, 8192, 128, _lib.KBH_BF16, _lib.KBH_KERNEL_DECODE),
     (33, 1408, 2048, 128, _lib.KBH_F16, _lib.KBH_KERNEL_DECODE), (48, 1152, 4096, 128, _lib.KBH_BF16, _lib.KBH_KERNEL_DECODE),
-    (127, 1152, 14336, 128, _lib.KBH_F16, 128), (64, 29568, 8192, 128, _lib.KBH_F16, 64), (128, 640, 8192, 128, _lib.KBH_F16, 128),
+    (48, 1792, 6144, 256, _lib.KBH_F16, _lib.KBH_KERNEL_DECODE), (96, 2304, 4096, 256, _lib.KBH_F16, _lib.KBH_KERNEL_DECODE),
+    (256, 320, 2048, 64, _lib.KBH_F16, _lib.KBH_KERNEL_DECODE), (128, 960, 2048, 64, _lib.KBH_BF16, _lib.KBH_KERNEL_DECODE),
+    (256, 2752, 8192, 64, _lib.KBH_F16, 128), (127, 1152, 14336, 128, _lib.KBH_F16, 128), (64, 29568, 8192, 128, _lib.KBH_F16, 64), (128, 640, 8192, 128, _lib.KBH_F16, 128),
     (64, 1024, 4096, 128, _lib.KBH_F16, 64)])
 def test_w4a16_decode_kernel_stays(lib, M, K, N, group, dtype, kernel):
     assert lib.kbh_w4a16_kernel(M, N, K, group, dtype, None) == kernel
