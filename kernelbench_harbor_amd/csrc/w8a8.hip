@@ -366,15 +366,18 @@ bool w8_decode_range(int M, int N) { return M <= 32 || (M < kW8TiledMinM && N % 
 
 // Whether the decode kernel keeps a call of that range past one round of workgroups. It streams the weights
 // once per 16-row block, and plan_w8_wide keeps it always while its grid is resident at once (two workgroups
-// per CU: 1024 x 1024 .. 8192 x 1152 at 33 to 127 rows 8-16 us against 14-20); beyond that where its estimated
-// time is at most 3% over the wide plan's, 25% in the second round of full workgroups whose splits are a power of two (the fit has those
-// too slow: 8192 x 1408 M=127 16.2 us against 20.3). Both estimates (us) are least-squares fits to 2000
-// calls of 17 to 127 rows over K from 1024 to 14336 and N from 384 to 14464 (decode 7.6%, wide 5.1%
-// rms): the choice is 0.7% from the faster kernel on average past 512 workgroups; 7 of those calls are
-// 4% or more slower than on decode, where "at most 512 workgroups, and N a multiple of 256" left 769 (by
-// up to 79%: K=2048 N=1408 M=48 9.0 -> 15.0 us).
+// per CU: 1024 x 1024 .. 8192 x 1152 at 33 to 127 rows 8-16 us against 14-20). In a second round it stays where its
+// estimated time is at most 3% over the wide plan's, 25% for full workgroups up to one and a half rounds whose
+// splits are a power of two (the fit has those too slow: 8192 x 1408 M=127 16.2 us against 20.3). From the third
+// round on the wide tiles take the call: their estimate is 9% too high there and decode lost 12% on average
+// (17 to 31 rows of 3584 x 18944 24.1-25.4 us against 28.3-30.6, 6144 x 11008 M=32 26.5 / 35.8). Both
+// estimates (us) are least-squares fits to 2000 calls of 17 to 127 rows over K from 1024 to 14336 and N from
+// 384 to 14464 (decode 7.6%, wide 5.1% rms): of the 820 calls past 512 workgroups the choice is 0.3% from the
+// faster kernel on average and 9 are more than 4% slower than on decode (9% at most), where "at most 512
+// workgroups, and N a multiple of 256" left 769 of all (by up to 79%: K=2048 N=1408 M=48 9.0 -> 15.0 us).
 bool w8_decode_stays(int M, int N, const W8Plan& d, const WidePlan& w) {
   const int grid = d.ntiles * d.splits * d.mblocks;
+  if (grid > 1024) return false;
   float dec = 5.3f + 4.37f * (float)grid * (float)(d.waves * d.spw) / 4096.0f + 1.27f * (float)((grid + 511) / 512);
   if (d.splits > 1) dec += 0.16f + 0.064f * d.splits + 0.164f * ((float)d.splits * M * N * 8.0f / (float)(1 << 20));
   const bool full = grid <= 768 && d.waves == 8 && d.splits >= 4 && (d.splits & (d.splits - 1)) == 0;

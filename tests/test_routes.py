@@ -37,9 +37,15 @@ def test_fp8w_decode_kernel_stays(lib, M, K, N, splits):
 # M, K, N: calls that the decode kernel runs faster than the wide tiles (which take scratch here), and
 # calls past the line
 @pytest.mark.parametrize("M,K,N,wide", [(48, 2048, 1408, False), (127, 4096, 1664, False), (33, 8192, 2432, False), (17, 3584, 14336, False),
-                                        (17, 11008, 1024, False), (127, 2048, 8576, True), (64, 18944, 2176, True), (32, 14336, 4096, True)])
+                                        (17, 11008, 1024, False), (127, 2048, 8576, True), (64, 18944, 2176, True), (32, 14336, 4096, True),
+                                        (32, 6144, 11008, True), (24, 7168, 11008, True)])
 def test_w8a8_decode_kernel_stays(lib, M, K, N, wide):
     assert (lib.kbh_w8a8_scratch_bytes(M, N, K) > 0) == wide
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 3584, 18944), (31, 3584, 18944), (32, 14336, 5504)])
+def test_w8a8_wide_from_the_third_round(lib, M, K, N):
+    assert lib.kbh_w8a8_kernel(M, N, K, None) == 128
 
 
 @pytest.mark.parametrize("M,K,N,splits", [(160, 7168, 5120, 7), (160, 14336, 2560, 14), (129, 14336, 2560, 14)])
