@@ -261,6 +261,7 @@ int kbh_moe(const void* x, const void* w, const void* router_logits, int logits_
  * workspace >= kbh_lora_qgemm_workspace_bytes(T, D, N, r), no content requirement.
  */
 size_t kbh_lora_qgemm_workspace_bytes(int T, int D, int N, int r);
+int kbh_lora_qgemm_kernel(int T, int D, int N, int group, int* splits); /* of the base; as kbh_w4a16_kernel */
 int kbh_lora_qgemm(const void* x, const int8_t* qweight, const void* scales, const void* A,
                    const void* B, const int64_t* lora_ids, void* y, void* workspace,
                    size_t workspace_bytes, int T, int D, int N, int r, int L, int group, int dtype,

@@ -503,8 +503,14 @@ struct ByteWide {
 // with N of 128 mod 256: the choice is 0.3% from the faster kernel on average and never more than 11%
 // slower than decode, where "up to 64 rows and one workgroup per CU" lost up to 46% (M=127: 4096 x 2048
 // 13.8 against 20.0, 2048 x 4096 14.0 / 19.9; M=17: 4096 x 6144 13.1 / 14.1).
-inline bool byte_decode_stays(int M, const BytePlan& d) {
+// The int8 base of the multi-LoRA linear from 33 rows (`int8`): only one workgroup per CU, or full ones whose second
+// row block is mostly padding. The GEMM alone is the slower one beyond that (3584 x 3584 T=64 16.4 us against the
+// wide tiles' 12.1); FP8 weights earn it back in the slice sum placed by XCD, which this linear's last kernel replaces.
+// Of 364 calls (28 layers, 17 to 127 rows, fp16) 25 were more than 4% slower than on the wide tiles under the
+// line of the FP8 weights (3584 x 3584 r=8 T=57 19.9 against 23.3 us, 2560 x 2560 T=96 22.7 / 25.3) and none is now.
+inline bool byte_decode_stays(int M, const BytePlan& d, bool int8) {
   const int grid = d.ntiles * d.splits * d.mblocks;
+  if (int8 && M > 32 && grid > 256 && !(M > 64 && d.waves == 8)) return false;
   const bool resident = grid <= 256 * (d.waves < 8 ? 8 / d.waves : 1);
   if (M <= 64) return grid <= 256 || (resident && d.waves >= 4 && grid % 8 == 0);
   return (resident && d.waves >= 3) || (M <= 96 && d.waves >= 5 && grid <= 320);
@@ -516,12 +522,12 @@ inline bool byte_decode_stays(int M, const BytePlan& d) {
 // at every M from 128 to 1024; now 30.7 / 43.0 / 75.2 / 124 us at M=128 / 256 / 512 / 1024, and
 // 342 -> 226 at 2048), and the decode kernel's 32- and 64-row blocks where those take several rounds
 // (M=32 26.2 -> 19.4, M=48 42.9 -> 21.4, M=96 73.2 -> 28.4; 8192 x 28672 M=32 85.5 -> 66.9).
-bool plan_byte_wide(int M, int N, int K, int block, ByteWide* w) {
+bool plan_byte_wide(int M, int N, int K, int block, bool int8, ByteWide* w) {
   if (M < kByteWideMinM || N < 256) return false;
   // the kernels stage x with 32-bit offsets
   if ((size_t)(M + 256) * K * 2 >= ((size_t)1 << 31)) return false;
   BytePlan d;
-  if (M < kByteTiledMinM && plan_byte_decode(M, N, K, &d) && byte_decode_stays(M, d)) return false;
+  if (M < kByteTiledMinM && plan_byte_decode(M, N, K, &d) && byte_decode_stays(M, d, int8)) return false;
   w->spg = block / 32;
   const int unit = wide_iteration(w->spg, kByteWidePD) / 2;
   return plan_wide(M, N, K, 256, 32, unit, unit, 256, kHalfCosts, &w->plan, M <= 64 ? 64 : 128);
@@ -548,9 +554,9 @@ void launch_byte_wide(const ByteWide& w, const void* x, const void* wt, const vo
 }
 
 // The decode kernel's plan when byte_gemm_run takes that kernel for this shape.
-bool byte_takes_decode(int M, int N, int K, int block, BytePlan* p) {
+bool byte_takes_decode(int M, int N, int K, int block, bool int8, BytePlan* p) {
   ByteWide w;
-  if (plan_byte_wide(M, N, K, block, &w)) return false;
+  if (plan_byte_wide(M, N, K, block, int8, &w)) return false;
   if (M >= kByteTiledMinM && K % (TBK * TDEPTH) == 0) return false;
   return plan_byte_decode(M, N, K, p);
 }
@@ -564,7 +570,7 @@ int byte_gemm_run(const void* x, const void* w, const void* scales, void* y, voi
                   bool defer_sum = false, int* splits_out = nullptr, SIDE side = SIDE{}) {
   if (splits_out) *splits_out = 1;
   ByteWide wide;
-  bool is_wide = plan_byte_wide(M, N, K, block, &wide);
+  bool is_wide = plan_byte_wide(M, N, K, block, DEC == kDecInt8, &wide);
   if (is_wide) {  // without room for the slices, the kernels that ran the call before the wide tiles
     const size_t need = wide_workspace_bytes(M, N, wide.plan.splits);
     is_wide = need == 0 || (workspace && workspace_bytes >= need);
@@ -634,10 +640,10 @@ int byte_gemm_run(const void* x, const void* w, const void* scales, void* y, voi
 }
 
 // Workspace bytes of byte_gemm_run for this shape (0 when K is not split).
-size_t byte_gemm_workspace_bytes(int M, int N, int K, int block) {
+size_t byte_gemm_workspace_bytes(int M, int N, int K, int block, bool int8) {
   if (M < 1 || N < 128 || K < 32 || block < 32 || K % block != 0) return 0;
   ByteWide w;
-  if (plan_byte_wide(M, N, K, block, &w)) return wide_workspace_bytes(M, N, w.plan.splits);
+  if (plan_byte_wide(M, N, K, block, int8, &w)) return wide_workspace_bytes(M, N, w.plan.splits);
   if (M >= kByteTiledMinM && K % (TBK * TDEPTH) == 0) return 0;  // tiled path: no split
   BytePlan p;
   if (!plan_byte_decode(M, N, K, &p)) return 0;

@@ -13,11 +13,11 @@
 extern "C" size_t kbh_fp8w_workspace_bytes(int M, int N, int K, int block) {
   using kbh::byte_gemm_workspace_bytes;
   if (block >= 32 && block <= 256 && (block & (block - 1)) == 0 && K % block == 0)
-    return byte_gemm_workspace_bytes(M, N, K, block);
+    return byte_gemm_workspace_bytes(M, N, K, block, false);
   // Any other block, for which the query has never failed: room for every accepted one.
   size_t best = 0;
   for (int b : {32, 64, 128, 256}) {
-    const size_t n = byte_gemm_workspace_bytes(M, N, K, b);
+    const size_t n = byte_gemm_workspace_bytes(M, N, K, b, false);
     best = n > best ? n : best;
   }
   return best;
@@ -28,7 +28,7 @@ extern "C" int kbh_fp8w_kernel(int M, int N, int K, int block, int* splits) {
   if (splits) *splits = 1;
   if (M < 1 || N < 128 || K < 32 || N % 128 != 0 || !quant_group_ok(K, block)) return KBH_KERNEL_NONE;
   ByteWide w;
-  if (plan_byte_wide(M, N, K, block, &w)) {
+  if (plan_byte_wide(M, N, K, block, false, &w)) {
     if (splits) *splits = w.plan.splits;
     return w.plan.tm;
   }

@@ -189,7 +189,7 @@ LoraLayout lora_layout(int T, int D, int N, int r, int group) {
   L.ds = max(1, min((1024 + T - 1) / T, ds_max));
   L.dchunk = (D + L.ds - 1) / L.ds;
   L.slices = round_up((size_t)L.ds * T * r * 4, 256);
-  L.total = L.slices + round_up(byte_gemm_workspace_bytes(T, N, D, group), 256);
+  L.total = L.slices + round_up(byte_gemm_workspace_bytes(T, N, D, group, true), 256);
   return L;
 }
 
@@ -208,7 +208,7 @@ int lora_run(const void* x, const int8_t* qweight, const void* scales, const voi
   // Beside the decode kernel's blocks of 16 and 32 rows (T=1 19.5 -> 13.4 us, T=32 r=16 20.0 ->
   // 17.5, r=64 25.7 -> 22.7; a launch and its gap less, host time included). Its 64-row blocks hold
   // 218 registers, so the shrink's workgroups would queue one per CU behind them (T=64 22.1 -> 27.1).
-  if (T <= 32 && byte_takes_decode(T, N, D, group, &bp)) {
+  if (T <= 32 && byte_takes_decode(T, N, D, group, true, &bp)) {
     s = byte_gemm_run<BF16, kDecInt8>(x, qweight, scales, y, slices, ws_bytes - lay.slices, T, N, D,
                                       group, st, true, &splits, shrink);
   } else {
@@ -239,6 +239,22 @@ extern "C" size_t kbh_lora_qgemm_workspace_bytes(int T, int D, int N, int r) {
     best = b > best ? b : best;
   }
   return best;
+}
+
+extern "C" int kbh_lora_qgemm_kernel(int T, int D, int N, int group, int* splits) {
+  using namespace kbh;
+  if (splits) *splits = 1;
+  if (T < 1 || N < 128 || D < 32 || N % 128 != 0 || !quant_group_ok(D, group)) return KBH_KERNEL_NONE;
+  ByteWide w;
+  if (plan_byte_wide(T, N, D, group, true, &w)) {
+    if (splits) *splits = w.plan.splits;
+    return w.plan.tm;
+  }
+  if (T >= kByteTiledMinM && D % (TBK * TDEPTH) == 0) return KBH_KERNEL_STAGED;
+  BytePlan p;
+  if (!plan_byte_decode(T, N, D, &p)) return KBH_KERNEL_NONE;
+  if (splits) *splits = p.splits;
+  return KBH_KERNEL_DECODE;
 }
 
 extern "C" int kbh_lora_qgemm(const void* x, const int8_t* qweight, const void* scales,

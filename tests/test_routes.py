@@ -34,6 +34,14 @@ def test_fp8w_decode_kernel_stays(lib, M, K, N, splits):
     assert lib.kbh_fp8w_workspace_bytes(M, N, K, 128) == splits * M * N * 4
 
 
+# T, D, N: base GEMMs of two workgroups per CU, which the wide tiles run faster, and ones that the decode kernel does
+@pytest.mark.parametrize("T,D,N,kernel", [
+    (57, 3584, 3584, 64), (33, 3072, 3072, 64), (64, 3072, 3584, 64), (96, 2560, 2560, 128), (127, 2048, 3584, 128), (64, 4096, 4096, _lib.KBH_KERNEL_DECODE),
+    (17, 7168, 3584, _lib.KBH_KERNEL_DECODE), (32, 7168, 3584, _lib.KBH_KERNEL_DECODE), (80, 5120, 2048, _lib.KBH_KERNEL_DECODE), (127, 4096, 2048, _lib.KBH_KERNEL_DECODE)])
+def test_lora_base_kernel(lib, T, D, N, kernel):
+    assert lib.kbh_lora_qgemm_kernel(T, D, N, 128, None) == kernel
+
+
 # M, K, N: calls that the decode kernel runs faster than the wide tiles (which take scratch here), and
 # calls past the line
 @pytest.mark.parametrize("M,K,N,wide", [(48, 2048, 1408, False), (127, 4096, 1664, False), (33, 8192, 2432, False), (17, 3584, 14336, False),
