@@ -504,8 +504,9 @@ struct ByteWide {
 // slower than decode, where "up to 64 rows and one workgroup per CU" lost up to 46% (M=127: 4096 x 2048
 // 13.8 against 20.0, 2048 x 4096 14.0 / 19.9; M=17: 4096 x 6144 13.1 / 14.1).
 // The int8 base of the multi-LoRA linear from 33 rows (`int8`): only one workgroup per CU, or full ones whose second
-// row block is mostly padding. The GEMM alone is the slower one beyond that (3584 x 3584 T=64 16.4 us against the
-// wide tiles' 12.1); FP8 weights earn it back in the slice sum placed by XCD, which this linear's last kernel replaces.
+// row block is mostly padding. Beyond that int8 codes cost the decode kernel more and the wide tiles less than FP8
+// codes do (the GEMM alone, 3584 x 3584 and 64 rows: 16.4 against 12.1 us, FP8 15.2 / 13.4), and the slice sum that
+// the decode plan makes faster (FP8 3.9 / 4.3) is replaced by this linear's last kernel.
 // Of 364 calls (28 layers, 17 to 127 rows, fp16) 25 were more than 4% slower than on the wide tiles under the
 // line of the FP8 weights (3584 x 3584 r=8 T=57 19.9 against 23.3 us, 2560 x 2560 T=96 22.7 / 25.3) and none is now.
 inline bool byte_decode_stays(int M, const BytePlan& d, bool int8) {
